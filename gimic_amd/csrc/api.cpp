@@ -272,9 +272,10 @@ struct gimic_ctx {
     double screen_thrs = 1e-6;
     int giao = 1, diamag = 1, paramag = 1;
     int nset = 0;
-    std::vector<double> dens;  // nset*4*n*n column-major, as given
+    DevBuf dens;               // nset*4*n*n doubles on the device, as given
+    bool dens_rows = false;    // blocks given row-major
     int lda = 0, ncol_pad = 0;
-    DevBuf shells, exps, ncc, coords, rf64, rf32;
+    DevBuf shells, exps, ncc, coords, rf64, rf32, fun;  // fun: fun_orig on the device
     // right operands per (spin list, precision)
     struct Mats {
         DevBuf b64;
@@ -457,6 +458,7 @@ void setup_device(gimic_ctx *c) {
     }
     up(c->rf64, rf.data(), rf.size() * sizeof(double));
     up(c->rf32, rf32.data(), rf32.size() * sizeof(float));
+    up(c->fun, c->fun_orig.data(), c->fun_orig.size() * sizeof(int));
     std::vector<double> sph;
     for (int l = 2; l <= kDevMaxL; l++) {
         auto T = sph_transform(l);
@@ -466,118 +468,56 @@ void setup_device(gimic_ctx *c) {
     hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
 }
 
-// FP64 density family of one spin case: 4 n*n column-major blocks.
-std::vector<double> spin_family(const gimic_ctx *c, int spin) {
-    const size_t n = (size_t)c->basis.nbf, blk = 4 * n * n;
-    if (c->nset == 0) throw Error(GIMIC_ESTATE, "no density set");
-    if (c->nset == 1) {
-        if (spin == GIMIC_SPIN_BETA)
-            throw Error(GIMIC_ESTATE, "beta current requested, but not open-shell system!");
-        if (spin == GIMIC_SPIN_SPINDENS)
-            throw Error(GIMIC_ESTATE, "spindens requested, but not open-shell system!");
-        return std::vector<double>(c->dens.begin(), c->dens.begin() + blk);
-    }
-    std::vector<double> out(blk);
-    const double *a = c->dens.data(), *bb = c->dens.data() + blk;
-    for (size_t i = 0; i < blk; i++) {
-        switch (spin) {
-            case GIMIC_SPIN_ALPHA: out[i] = a[i]; break;
-            case GIMIC_SPIN_BETA: out[i] = bb[i]; break;
-            case GIMIC_SPIN_SPINDENS: out[i] = a[i] - bb[i]; break;
-            default: out[i] = a[i] + bb[i]; break;
-        }
-    }
-    return out;
+// Densities as given: uploaded once, the operands are built from them on the
+// device.  The previous densities stay in force if the upload fails.
+void upload_density(gimic_ctx *c, int nset, const double *dens, bool rows) {
+    const size_t n = (size_t)c->basis.nbf, bytes = (size_t)nset * 4 * n * n * sizeof(double);
+    DevBuf fresh;
+    fresh.alloc(bytes, c->stream, false);
+    hip_check(hipMemcpyAsync(fresh.p, dens, bytes, hipMemcpyHostToDevice, c->stream),
+              "hipMemcpyAsync");
+    hip_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    std::swap(c->dens.p, fresh.p);
+    std::swap(c->dens.bytes, fresh.bytes);
+    c->nset = nset;
+    c->dens_rows = rows;
+    c->mats.clear();
 }
 
 gimic_ctx::Mats &get_mats(gimic_ctx *c, const std::vector<int> &spins, int prec) {
     auto key = std::make_pair(spins, prec);
     auto it = c->mats.find(key);
     if (it != c->mats.end()) return *it->second;
-    const size_t n = (size_t)c->basis.nbf, ld = (size_t)c->lda, nc = (size_t)c->ncol_pad;
-    const size_t matsz = nc * ld, setsz = kNMat * matsz;
+    const size_t n = (size_t)c->basis.nbf, ld = (size_t)c->lda;
     auto m = std::make_unique<gimic_ctx::Mats>();
     m->nmatset = (int)spins.size();
-    std::vector<double> B(setsz * spins.size(), 0.0);
-    // atom of each caller-ordered function; the internal order is fun_orig
-    std::vector<int> atom_of(n);
-    for (auto &s : c->basis.shells) {
-        const int nout = c->basis.spherical ? 2 * s.l + 1 : ncart(s.l);
-        for (int f = 0; f < nout; f++) atom_of[s.fout + f] = s.atom;
-    }
-    const std::vector<int> &fo = c->fun_orig;
-    for (size_t si = 0; si < spins.size(); si++) {
-        std::vector<double> fam = spin_family(c, spins[si]);
-        double *Bs = &B[si * setsz];
-        // matrix j column nu (K = mu contiguous), internal order:
-        // D(mu,nu) = fam[blk + fo[mu] + n*fo[nu]].
-        // The GIAO right operands are W_d(mu,nu) = D(mu,nu) (R_nu - R_mu)_d:
-        // phi W_d equals R_d (phi D) - phi diag(R_d) D without the
-        // cancellation between those two terms (and is zero on one-atom blocks).
-        for (size_t nu = 0; nu < n; nu++) {
-            const size_t onu = (size_t)fo[nu];
-            const double *Rn = &c->basis.coords[3 * atom_of[onu]];
-            for (size_t mu = 0; mu < n; mu++) {
-                const size_t omu = (size_t)fo[mu];
-                const double D = fam[omu + n * onu];
-                const double *Rm = &c->basis.coords[3 * atom_of[omu]];
-                Bs[0 * matsz + nu * ld + mu] = D;
-                for (int b = 1; b < 4; b++)
-                    Bs[b * matsz + nu * ld + mu] = fam[(size_t)b * n * n + omu + n * onu];
-                for (int d = 0; d < 3; d++)
-                    Bs[(4 + d) * matsz + nu * ld + mu] = D * (Rn[d] - Rm[d]);
-            }
-        }
-    }
     hipStream_t st = c->stream;
-    if (prec == GIMIC_PREC_FP64) {
-        m->b64.alloc(B.size() * sizeof(double), st, false);
-        hip_check(hipMemcpyAsync(m->b64.p, B.data(), B.size() * sizeof(double),
-                                 hipMemcpyHostToDevice, st),
-                  "hipMemcpyAsync");
-    } else {
-        std::vector<float> b32(B.begin(), B.end());
-        // the FP32 values as their first kBParts BF16 parts (three parts:
-        // x = h + m + l exactly), one pair block per (set, 8-function K-group
-        // gk, 8-function N-group gn), [part][matrix][n][k]; rows of K-groups
-        // of ngn + 1 blocks (the last zero) and a zero row last: the mixed
-        // kernels gather the 16 blocks of an N-tile's K-step into their LDS
-        // buffers
-        const size_t nkg = ld / 8, ngn = nc / 8, pe = kMx2PairElems;
-        const size_t setel = mx2_set_elems((int)ld, (int)nc);
-        std::vector<uint16_t> bs(spins.size() * setel, 0);
-        auto bf = [](float x) {
-            uint32_t u;
-            std::memcpy(&u, &x, 4);
-            u += 0x7FFFu + ((u >> 16) & 1u);
-            return (uint16_t)(u >> 16);
-        };
-        auto fl = [](uint16_t h) {
-            const uint32_t u = (uint32_t)h << 16;
-            float x;
-            std::memcpy(&x, &u, 4);
-            return x;
-        };
-        for (size_t si = 0; si < spins.size(); si++)
-            for (size_t mat = 0; mat < (size_t)kNMat; mat++)
-                for (size_t nu = 0; nu < nc; nu++) {
-                    const float *src = &b32[si * setsz + mat * matsz + nu * ld];
-                    const size_t gn = nu / 8, nn = nu % 8;
-                    for (size_t mu = 0; mu < ld; mu++) {
-                        const size_t gk = mu / 8, kk = mu % 8;
-                        uint16_t *dst = &bs[si * setel + (gk * (ngn + 1) + gn) * pe];
-                        float x = src[mu];
-                        for (int p = 0; p < kBParts; p++) {
-                            const uint16_t h = bf(x);
-                            dst[((p * kNMat + mat) * 8 + nn) * 8 + kk] = h;
-                            x -= fl(h);
-                        }
-                    }
-                }
-        m->bs3.alloc(bs.size() * 2, st, false);
-        hip_check(hipMemcpyAsync(m->bs3.p, bs.data(), bs.size() * 2, hipMemcpyHostToDevice, st),
-                  "hipMemcpyAsync");
-        hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
+    const bool f64 = prec == GIMIC_PREC_FP64;
+    const size_t setel = f64 ? kNMat * ld * ld : mx2_set_elems(c->lda, c->ncol_pad);
+    (f64 ? m->b64 : m->bs3).alloc(spins.size() * setel * (f64 ? 8 : 2), st, false);
+    for (size_t si = 0; si < spins.size(); si++) {
+        const int spin = spins[si];
+        if (c->nset == 0) throw Error(GIMIC_ESTATE, "no density set");
+        if (c->nset == 1) {
+            if (spin == GIMIC_SPIN_BETA)
+                throw Error(GIMIC_ESTATE, "beta current requested, but not open-shell system!");
+            if (spin == GIMIC_SPIN_SPINDENS)
+                throw Error(GIMIC_ESTATE, "spindens requested, but not open-shell system!");
+        }
+        // alpha, beta, or alpha +- beta of two sets; the one set of a closed shell
+        const double *alpha = c->dens.as<double>(), *beta = alpha + 4 * n * n;
+        OperandArgs oa{};
+        oa.dens = c->nset == 2 && spin == GIMIC_SPIN_BETA ? beta : alpha;
+        oa.second = c->nset == 2 && (spin == GIMIC_SPIN_TOTAL || spin == GIMIC_SPIN_SPINDENS)
+                        ? beta : nullptr;
+        oa.subtract = spin == GIMIC_SPIN_SPINDENS;
+        oa.row_major = c->dens_rows;
+        oa.n = (int)n;
+        oa.ld = c->lda;
+        oa.fun = c->fun.as<int>();
+        oa.rf64 = c->rf64.as<double>();
+        if (f64) hip_check(launch_operand_f64(oa, m->b64.as<double>() + si * setel, st), "operand_f64");
+        else hip_check(launch_operand_split(oa, m->bs3.as<__bf16>() + si * setel, st), "operand_split");
     }
     hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
     auto &ref = *m;
@@ -1333,11 +1273,10 @@ int gimic_ctx_create_files(gimic_ctx **out, const char *molfile, const char *den
         auto c = std::make_unique<gimic_ctx>();
         c->basis = read_mol(molfile);
         c->screen_thrs = screen_thrs;
-        if (densfile) {
-            c->nset = uhf ? 2 : 1;
-            c->dens = read_xdens(densfile, c->basis, c->nset, uhf != 0);
-        }
+        std::vector<double> dens;
+        if (densfile) dens = read_xdens(densfile, c->basis, uhf ? 2 : 1, uhf != 0);
         setup_device(c.get());
+        if (densfile) upload_density(c.get(), uhf ? 2 : 1, dens.data(), false);
         *out = c.release();
     });
 }
@@ -1363,14 +1302,20 @@ int gimic_ctx_create(gimic_ctx **out, int natoms, const double *coords, int nshe
     });
 }
 
-int gimic_ctx_set_density(gimic_ctx *c, int nset, const double *dens) {
+static int set_density(gimic_ctx *c, int nset, const double *dens, bool rows) {
     return guarded([&] {
         if (!c || !dens || (nset != 1 && nset != 2)) throw Error(GIMIC_EINVAL, "bad argument");
-        const size_t n = (size_t)c->basis.nbf;
-        c->nset = nset;
-        c->dens.assign(dens, dens + (size_t)nset * 4 * n * n);
-        c->mats.clear();
+        DeviceGuard device(c->device);
+        upload_density(c, nset, dens, rows);
     });
+}
+
+int gimic_ctx_set_density(gimic_ctx *c, int nset, const double *dens) {
+    return set_density(c, nset, dens, false);
+}
+
+int gimic_ctx_set_density_rows(gimic_ctx *c, int nset, const double *dens) {
+    return set_density(c, nset, dens, true);
 }
 
 int gimic_ctx_set_flags(gimic_ctx *c, int giao, int diamag, int paramag) {

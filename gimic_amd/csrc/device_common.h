@@ -173,6 +173,23 @@ __host__ __device__ constexpr size_t mx2_set_elems(int lda, int ncol_pad) {
 constexpr int kMx2GroupElems = kBParts * kMx2Cols * 8;   // 5376 for three parts
 constexpr int kMx2BlockElems = (4 * kMx2GroupElems * 2 + 1023) / 1024 * 512;
 
+// Right operands from the caller's densities (operands.hip): 4 n x n blocks D,
+// DBx, DBy, DBz of one spin set, plus or minus those of a second one if
+// `second` is set; element (mu, nu) in caller order at mu * n + nu (row_major)
+// or mu + n * nu; fun[i] is the caller's index of internal function i < n,
+// rf64 the centres [3][ld] by internal index.  One set's operand each:
+// launch_operand_f64 [matrix][nu][mu] with rows of ld, launch_operand_split the
+// pair blocks of mx2_set_elems(ld, ld) elements; padding is written as zeros.
+struct OperandArgs {
+    const double *dens, *second;
+    int subtract, row_major;
+    int n, ld;
+    const int *fun;
+    const double *rf64;
+};
+hipError_t launch_operand_f64(const OperandArgs &a, double *out, hipStream_t s);
+hipError_t launch_operand_split(const OperandArgs &a, __bf16 *out, hipStream_t s);
+
 struct FinalizeArgs {
     const double *part;  // [nmatset][nsplit][kNQ][rows], or [nmatset][nsplit][rows][kNQ] if part_rows
     int part_rows;

@@ -18,7 +18,7 @@ EXPORTS = [
     "gimic_init", "gimic_finalize", "gimic_set_uhf", "gimic_set_magnet", "gimic_set_spin",
     "gimic_set_screening", "gimic_calc_jtensor", "gimic_calc_jvector", "gimic_calc_modj",
     "gimic_get_gauss_points", "mkgausspoints", "gimic_last_error", "gimic_ctx_create_files",
-    "gimic_ctx_create", "gimic_ctx_set_density", "gimic_ctx_set_flags", "gimic_ctx_info",
+    "gimic_ctx_create", "gimic_ctx_set_density", "gimic_ctx_set_density_rows", "gimic_ctx_set_flags", "gimic_ctx_info",
     "gimic_ctx_destroy", "gimic_ctx_atoms", "gimic_ctx_atom_symbols", "gimic_ctx_set_timing", "gimic_ctx_get_timing", "gimic_ctx_tuning", "gimic_ctx_tuning_log", "gimic_ctx_set_mixed_kernel", "gimic_ctx_set_tile_stats", "gimic_ctx_tile_stats", "gimic_ctx_set_fp64_radius", "gimic_ctx_fp64_refined", "gimic_ctx_set_chunk_bytes", "gimic_ctx_chunk_bytes", "gimic_ctx_set_graph", "gimic_ctx_graph_stats", "gimic_jtensor_batch", "gimic_jtensor_batch_device", "gimic_jtensor_batch_device_noalloc",
     "gimic_jtensor_multi_device", "gimic_flux_planes", "gimic_flux_plane_grids", "gimic_ctx_properties", "gimic_sph_transform", "gimic_quadrature",
     "gimic_selftest_mfma_layout", "gimic_selftest_mfma32_layout", "gimic_mlp_create", "gimic_mlp_destroy", "gimic_mlp_set_stream", "gimic_mlp_info",
@@ -68,6 +68,7 @@ def load():
         "gimic_ctx_create_files": [P, ctypes.c_char_p, ctypes.c_char_p, I, D],
         "gimic_ctx_create": [P, I, P, I, P, P, P, P, P, P, I, I, D],
         "gimic_ctx_set_density": [P, I, P],
+        "gimic_ctx_set_density_rows": [P, I, P],
         "gimic_ctx_set_flags": [P, I, I, I],
         "gimic_ctx_info": [P, P, P, P, P, P],
         "gimic_ctx_destroy": [P],
@@ -364,9 +365,10 @@ class Context:
         d = np.asarray(dens, dtype=np.float64)
         if d.ndim == 3:
             d = d[None]
-        nset = d.shape[0]
-        flat = np.ascontiguousarray(d.transpose(0, 1, 3, 2)).reshape(-1)
-        check(self._lib.gimic_ctx_set_density(self._h, nset, ptr(flat)))
+        if d.ndim != 4:
+            raise ValueError("densities must be (nset, 4, n, n)")
+        d = np.ascontiguousarray(d)
+        check(self._lib.gimic_ctx_set_density_rows(self._h, d.shape[0], ptr(d)))
 
     def set_flags(self, giao=True, diamag=True, paramag=True):
         check(self._lib.gimic_ctx_set_flags(self._h, int(giao), int(diamag), int(paramag)))

@@ -105,6 +105,8 @@ int gimic_ctx_create(gimic_ctx **ctx, int natoms, const double *coords, int nshe
 /* nset = 1 (closed shell) or 2 (alpha, beta): nset*4 blocks of nbf*nbf
  * column-major doubles D, DBx, DBy, DBz, used exactly as given. */
 int gimic_ctx_set_density(gimic_ctx *ctx, int nset, const double *dens);
+/* the same with row-major blocks: element (mu, nu) at mu * nbf + nu */
+int gimic_ctx_set_density_rows(gimic_ctx *ctx, int nset, const double *dens);
 
 /* GIAO, diamagnetic and paramagnetic terms (jtensor.F90:180-228) */
 int gimic_ctx_set_flags(gimic_ctx *ctx, int giao, int diamag, int paramag);
