@@ -8,9 +8,11 @@
 // element (mu, nu) computes all seven matrices, so D and the centres are
 // loaded once; a wavefront covers 8 x 8 elements, whose stores are whole
 // 64- or 128-byte pieces.  Bound by memory: 32 bytes read and 56 (FP64) or 42
-// (split) bytes written per element.  Built on the host and copied, the 60-atom
-// cage's operands (nbf 1800) took 80 ms in FP64 and 90 ms more split; here
-// the upload of the 104 MB of densities and the kernel take the time.
+// (split) bytes written per element.  Building them on the host and copying them
+// took most of a first evaluation: a whole run on the 60-atom cage (nbf 1800:
+// context, densities, one 140 x 140 plane in FP64) went from 214 to 101 ms, the
+// first mixed evaluation of a 200-atom open shell (nbf 2620, two spin cases)
+// from 1352 to 288 ms, its tuning runs included.
 #include "device_common.h"
 
 namespace gimic {
