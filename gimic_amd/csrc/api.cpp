@@ -129,7 +129,7 @@ struct Workspace {
     DevBuf phi64, grad64, phis, grad32, part;
     // spatial tiles of a chunk: sorted points, their caller indices, sort
     // scratch, and the screening block list of every contraction row tile
-    DevBuf spts, perm, bpart, sortscr, bcount, blist, toff, k8count, k8list, bzero;
+    DevBuf spts, perm, bpart, sortscr, bcount, k8count, toff, kcount, klist;
     // FP64 pass near nuclei: selection index list, their points, selection
     // scratch and count
     DevBuf near_idx, near_pts, near_scr, near_cnt;
@@ -287,10 +287,8 @@ struct gimic_ctx {
     Workspace ws;
     DevBuf pts_tmp, jt_tmp, contrib, planes, pparams, offs, outs;
     // internal function order (see setup_device): fun_orig[i] is the caller's
-    // index of internal function i; per 32-function block the shells with a
-    // function in it (blk_beg ranges into blk_sh)
+    // index of internal function i
     std::vector<int> fun_orig;
-    DevBuf blk_beg, blk_sh;
     // property quadrature (gimic_ctx_properties): points + weights, tensors,
     // partition offsets, nuclei, sums
     DevBuf prop_in, prop_jt, prop_offs, prop_nuc, prop_out;
@@ -412,24 +410,12 @@ void setup_device(gimic_ctx *c) {
     // kernels hand consecutive shells of a point to consecutive lanes, so a
     // wavefront then runs one l branch (one polynomial and transform) at a
     // time instead of all of them with most lanes masked off.
-    std::vector<int> dorder(nsh), dpos(nsh);
+    std::vector<int> dorder(nsh);
     for (int i = 0; i < nsh; i++) dorder[i] = i;
     std::stable_sort(dorder.begin(), dorder.end(), [&](int x, int y) {
         if (b.shells[x].l != b.shells[y].l) return b.shells[x].l < b.shells[y].l;
         return fnew[x] < fnew[y];
     });
-    for (int k = 0; k < nsh; k++) dpos[dorder[k]] = k;
-    const int nblk = c->lda / 32;
-    std::vector<int> blk_beg(nblk + 1, 0), blk_sh;  // entries index the device array
-    for (int k = 0; k < nblk; k++) {
-        blk_beg[k] = (int)blk_sh.size();
-        for (int si : order) {
-            const int f0 = fnew[si], f1 = f0 + nout_of(b.shells[si]);
-            if (f0 < 32 * (k + 1) && f1 > 32 * k) blk_sh.push_back(dpos[si]);
-        }
-    }
-    blk_beg[nblk] = (int)blk_sh.size();
-    if (blk_sh.empty()) blk_sh.push_back(0);
     std::vector<DevShell> sh;
     for (int k = 0; k < nsh; k++) {
         const Shell &s = b.shells[dorder[k]];
@@ -444,8 +430,6 @@ void setup_device(gimic_ctx *c) {
     up(c->exps, b.exps.data(), b.exps.size() * sizeof(double));
     up(c->ncc, b.ncc.data(), b.ncc.size() * sizeof(double));
     up(c->coords, b.coords.data(), b.coords.size() * sizeof(double));
-    up(c->blk_beg, blk_beg.data(), blk_beg.size() * sizeof(int));
-    up(c->blk_sh, blk_sh.data(), blk_sh.size() * sizeof(int));
     std::vector<double> rf(3 * (size_t)c->ncol_pad, 0.0);
     std::vector<float> rf32(3 * (size_t)c->ncol_pad, 0.f);
     for (int i = 0; i < nsh; i++) {
@@ -488,12 +472,12 @@ gimic_ctx::Mats &get_mats(gimic_ctx *c, const std::vector<int> &spins, int prec)
     auto key = std::make_pair(spins, prec);
     auto it = c->mats.find(key);
     if (it != c->mats.end()) return *it->second;
-    const size_t n = (size_t)c->basis.nbf, ld = (size_t)c->lda;
+    const size_t n = (size_t)c->basis.nbf;
     auto m = std::make_unique<gimic_ctx::Mats>();
     m->nmatset = (int)spins.size();
     hipStream_t st = c->stream;
     const bool f64 = prec == GIMIC_PREC_FP64;
-    const size_t setel = f64 ? kNMat * ld * ld : mx2_set_elems(c->lda, c->ncol_pad);
+    const size_t setel = f64 ? f64_set_elems(c->lda) : mx2_set_elems(c->lda, c->ncol_pad);
     (f64 ? m->b64 : m->bs3).alloc(spins.size() * setel * (f64 ? 8 : 2), st, false);
     for (size_t si = 0; si < spins.size(); si++) {
         const int spin = spins[si];
@@ -582,7 +566,7 @@ int mixed_tile_rows(int variant) { return variant == 5 || variant >= 8 ? 256 : 1
 // kSmallF64Points points (the FP64 pass over the points next to nuclei, the
 // nuclei's share of property grids): there neighbouring points are far
 // apart, and the smaller tiles list a fifth fewer group pairs on the
-// 60-atom cage.  The screening lists are sized for the smallest tile.
+// 60-atom cage (3% less time on its whole grid).  The screening lists are sized for the smallest tile.
 constexpr int kMinTileRows = 64;
 constexpr size_t kSmallF64Points = 131072;
 int f64_tile_rows(size_t points) { return points <= kSmallF64Points ? 64 : kWgRows; }
@@ -595,7 +579,7 @@ size_t scratch_eval_bytes(const gimic_ctx *c, int prec, int nmatset, size_t rows
     size_t n = prec == GIMIC_PREC_FP64 ? r(rows * ld * 8) + r(3 * rows * ld * 8)
                                        : r(rows * ld * 2 * kAParts) + r(3 * rows * ld * 4);
     n += r(rows * 24) + r(rows * 4) + r(256 * 6 * 8) + r((size_t)sort_scratch_ints((int)rows) * 4);
-    n += r(t * 4) + r(t * nblk * 4) + r((t + 1) * 4) + r(t * 4) + r(t * nblk * 16) + r(12 * 1024);
+    n += 3 * r(t * 4) + r((t + 1) * 4) + r(t * nblk * 32);
     n += r((size_t)nmatset * split * kNQ * rows * 8);
     return n;
 }
@@ -737,11 +721,10 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
     grow(W.bpart, 256 * 6 * 8, false);
     grow(W.sortscr, (size_t)sort_scratch_ints((int)rows_cap) * 4, false);
     grow(W.bcount, rows_cap / kMinTileRows * 4, false);
-    grow(W.blist, rows_cap / kMinTileRows * nblk * 4, false);
-    grow(W.toff, (rows_cap / kMinTileRows + 1) * 4, false);
     grow(W.k8count, rows_cap / kMinTileRows * 4, false);
-    grow(W.k8list, rows_cap / kMinTileRows * nblk * 4 * 4, false);
-    grow(W.bzero, 12 * 1024, W.bzero.bytes < 12 * 1024);  // zeroed once, never written
+    grow(W.toff, (rows_cap / kMinTileRows + 1) * 4, false);
+    grow(W.kcount, rows_cap / kMinTileRows * 4, false);
+    grow(W.klist, rows_cap / kMinTileRows * nblk * 8 * 4, false);  // granules of 4 at most
     const int nmatset = M.nmatset;
     // chunks in rotated order, the middle one first: the autotuner times the
     // first chunk it sees, and the middle of a grid around a molecule is
@@ -791,25 +774,24 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
         ca.rf64 = c->rf64.as<double>();
         ca.rf32 = c->rf32.as<float>();
         ca.nblk = nblk;
-        ca.k8count = W.k8count.as<int>();
-        ca.k8list = W.k8list.as<int>();
-        ca.bzero = W.bzero.as<__bf16>();
-        // screening block lists for row tiles of tile_rows rows
-        auto lists = [&](int tile_rows) {
+        ca.kcount = W.kcount.as<int>();
+        ca.klist = W.klist.as<int>();
+        // screening lists of `gran`-function groups for row tiles of tile_rows rows
+        auto lists = [&](int tile_rows, int gran) {
             TileArgs ta{};
             ta.spts = spts;
             ta.npts = n_c;
             ta.rows = rows;
             ta.tile_rows = tile_rows;
             ta.nblk = nblk;
-            ta.blk_beg = c->blk_beg.as<int>();
-            ta.blk_sh = c->blk_sh.as<int>();
+            ta.gran = gran;
             ta.shells = c->shells.as<DevShell>();
+            ta.nshell = (int)c->basis.shells.size();
             ta.coords = c->coords.as<double>();
             ta.bcount = W.bcount.as<int>();
-            ta.blist = W.blist.as<int>();
             ta.k8count = W.k8count.as<int>();
-            ta.k8list = W.k8list.as<int>();
+            ta.kcount = W.kcount.as<int>();
+            ta.klist = W.klist.as<int>();
             hip_check(launch_block_lists(ta, st), "block_lists");
             if (c->tile_stats && mode == EvalMode::Eager) {
                 const int nt = rows / tile_rows;
@@ -832,15 +814,21 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
                 c->tile_acc[3] = tile_rows;
             }
         };
-        // work split over N so a launch has at least ~8192 workgroups (32
-        // per CU; small FP64 launches, such as the pass over the points next
-        // to nuclei, ran 4.5% faster than at 2048 and 22% faster than at
-        // 512), or the split count the tuner chose for the pre-split kernel
+        // work split over N: the split count the tuner chose for a mixed
+        // kernel, else so that a launch has 4096 (row tile, split) pairs or
+        // more, 8 or 16 per CU, which even out the tiles' unequal lists (cage60,
+        // 857,375 points: 87.1, 80.5, 79.3 and 79.1 ms at 1024, 2048, 4096 and
+        // 8192).  The FP64 kernel's cost of starting a workgroup (about 4 us)
+        // wants some 32 K-steps in each, though, and a tile of a small basis has
+        // few: then half as many pairs (ring12, 64,000 points: 0.183 ms at
+        // 2048 against 0.227 at 4096 and 0.266 at 8192)
         auto plan = [&](int wg_rows, int tile_cols, int want_split = 0) {
             ca.ntiles = c->ncol_pad / tile_cols;
-            const long long per = (long long)(rows / wg_rows) * nmatset;
-            int nsplit = (int)std::min<long long>(ca.ntiles,
-                                                  std::max<long long>(1, (8192 + per - 1) / per));
+            const long long per = (long long)(rows / wg_rows) * nmatset, nt = ca.ntiles;
+            auto pairs = [&](long long n) { return std::max<long long>(1, (n + per - 1) / per); };
+            int nsplit = (int)std::min(nt, pairs(prec == GIMIC_PREC_FP64 ? 4096 : 8192));
+            if (prec == GIMIC_PREC_FP64)
+                nsplit = (int)std::min<long long>(nsplit, std::max(pairs(2048), nt * nt / 128));
             if (want_split > 0) nsplit = std::min(want_split, ca.ntiles);
             if (scratch) nsplit = std::min(nsplit, kScratchMaxSplit);
             ca.tiles_per_split = (ca.ntiles + nsplit - 1) / nsplit;
@@ -858,9 +846,10 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
         // and offsets built before the basis evaluation)
         auto run = [&](int variant, int split = -1) {
             plan_variant(variant, split);
-            if (variant == 0) lists(f64_tile_rows(n_c));  // the FP64 kernel walks lists over dense rows
+            if (variant == 0) lists(f64_tile_rows(n_c), 4);  // the FP64 kernel walks lists over dense rows
             ca.toff = variant != 0 ? W.toff.as<int>() : nullptr;
-            if (variant == 0) hip_check(launch_contract_f64(ca, f64_tile_rows(n_c), st), "contract_f64");
+            ca.tile_rows = f64_tile_rows(n_c);
+            if (variant == 0) hip_check(launch_contract_f64(ca, st), "contract_f64");
             else if (variant == 3) hip_check(launch_contract_mx2(ca, 2, 2, 4, st), "contract_mx2");
             else if (variant == 4) hip_check(launch_contract_mx2(ca, 3, 2, 4, st), "contract_mx2");
             else if (variant == 5) hip_check(launch_contract_mx2(ca, 2, 4, 4, st), "contract_mx2");
@@ -873,11 +862,11 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
             ea.toff = nullptr;
             if (variant != 0) {
                 const int tr = mixed_tile_rows(variant);
-                lists(tr);
-                hip_check(launch_tile_offsets(W.k8count.as<int>(), rows / tr, W.toff.as<int>(), st),
+                lists(tr, 8);
+                hip_check(launch_tile_offsets(W.kcount.as<int>(), rows / tr, W.toff.as<int>(), st),
                           "tile_offsets");
-                ea.k8count = W.k8count.as<int>();
-                ea.k8list = W.k8list.as<int>();
+                ea.kcount = W.kcount.as<int>();
+                ea.klist = W.klist.as<int>();
                 ea.toff = W.toff.as<int>();
                 ea.nblk = nblk;
                 ea.tile_rows = tr;
@@ -1587,8 +1576,8 @@ void flux_run(gimic_ctx *c, int64_t npts, int nplanes, const int64_t *offs, cons
             (uintptr_t)c->ws.part.p, (uintptr_t)M.b64.p, (uintptr_t)c->ws.phis.p,
             (uintptr_t)M.bs3.p, (uintptr_t)c->mixed_split, (uintptr_t)c->ws.spts.p,
             (uintptr_t)c->ws.perm.p, (uintptr_t)c->ws.bpart.p, (uintptr_t)c->ws.sortscr.p,
-            (uintptr_t)c->ws.bcount.p, (uintptr_t)c->ws.blist.p, (uintptr_t)c->ws.toff.p,
-            (uintptr_t)c->ws.k8count.p, (uintptr_t)c->ws.k8list.p, (uintptr_t)c->ws.bzero.p,
+            (uintptr_t)c->ws.bcount.p, (uintptr_t)c->ws.k8count.p, (uintptr_t)c->ws.toff.p,
+            (uintptr_t)c->ws.kcount.p, (uintptr_t)c->ws.klist.p,
             (uintptr_t)refine,
             (uintptr_t)c->chunk_bytes};
         key.insert(key.end(), source.begin(), source.end());

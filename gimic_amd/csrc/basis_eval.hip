@@ -310,13 +310,13 @@ void basis_eval_staged_kernel(EvalArgs a) {
     size_t grad_plane = (size_t)a.gplane;
     if (!F64 && a.toff) {
         const int t = (int)(row0 / a.tile_rows);
-        const int kg = a.k8count[t];
+        const int kg = a.kcount[t];
         if (kg == 0) return;  // nothing of this tile is read (uniform per workgroup)
         wt = 8 * kg;
         gpos = (short *)(basis_tile + a.lds_image);
         for (int i = tid; i < 4 * a.nblk; i += 256) gpos[i] = -1;
         __syncthreads();
-        for (int i = tid; i < kg; i += 256) gpos[a.k8list[(size_t)t * a.nblk * 4 + i] >> 12] = (short)i;
+        for (int i = tid; i < kg; i += 256) gpos[a.klist[(size_t)t * a.nblk * 4 + i] >> 12] = (short)i;
         const size_t base = (size_t)a.toff[t] * a.tile_rows * 8;
         const size_t rin = row0 - (size_t)t * a.tile_rows;
         phi_dst = a.phis + base * kAParts + rin * kAParts * (size_t)wt;

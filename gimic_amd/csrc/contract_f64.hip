@@ -15,150 +15,247 @@
 // is accumulated as sum Y0 phi (r - R_nu) (gauge origin at each function's
 // centre), again free of cancellation.
 //
-// Tiling: WAVES wavefronts (4, or 2 for small launches); a workgroup owns
-// 32 WAVES point rows (32 per wavefront: two 16-row MFMA blocks) and walks a
-// range of 16-column N-tiles; per N-tile each wavefront keeps 2 x 7
-// v_mfma_f64_16x16x4 blocks.  Row tiles of 64 rather than 128 points list
-// fewer groups where neighbouring points are far apart, as in the FP64 pass
-// over the points next to nuclei, whose 128-row tiles mostly take in two
-// nuclei.
-// Only what screening leaves non-zero over the row tile (tiles.hip) is
-// visited: the live 8-function groups of its listed 32-function blocks,
-// two per 16-column N-tile (split evenly over the workgroups that share
-// the row tile) and two per 16-wide K-step.
-// The K index is remapped inside every K-step so each lane loads 32
-// contiguous bytes of its A row and of each B column (lane group g holds
-// elements 4(g&1)..+3 of group g/2; sub-step s feeds the s-th of them to
-// both operands).
+// Tiling: one wavefront owns 16 points, a workgroup four of them.  Only what
+// screening leaves non-zero over the row tile (tiles.hip; 64 or 128 points, one
+// or two workgroups) is visited, in granules of four functions, the K of one
+// v_mfma_f64_16x16x4: an N-tile is four of the tile's live granules (16
+// functions x 7 matrices), a K-step another four (lane group g owns the g-th).
+// The N-tiles of a row tile are split evenly over nsplit ranges.
+//
+// The matrices are the first MFMA operand and the points the second, so the
+// lane (g, c) of an output block holds Y of the four functions of granule g
+// at point c.  Each of the 22 sums then lives in one register pair per lane
+// over all N-tiles of the workgroup, and lanes are added once at its end (the
+// other way round each N-tile ends in a 16-lane reduction of 22 sums for
+// every row: 5,000 VALU cycles per N-tile and wavefront instead of 450).
+//
+// The right operand comes in pair blocks of 4 x 4 elements x 7 matrices
+// (operands.hip), 16 of which make a K-step: the workgroup copies them
+// through registers into one of three LDS buffers ahead of their use, so a
+// block is read once for 64 points.  Two workgroups share a CU (256 registers,
+// 43 KB of LDS each) and fill each other's barriers, starts and epilogues: one
+// workgroup of 128 points per CU with the same pipeline took 82.0 ms where
+// this takes 77.5, two buffers and a barrier that drains the matrix pipe 86.9.
+//
+// Bound: the matrix pipe.  On the 60-atom cage (857,375 points, 4.5 TFLOP of
+// listed work) 77.5 ms, 58 TF/s, 81% of a large FP64 matrix product on the
+// same card (71.6 TF/s); the kernel it replaced (points first, 8-function
+// groups, operands from global memory into registers) took 136 ms.  With every
+// operand load redirected to one cached block it ran within 1% of that.
+//
+// Workgroup order: the ranges of a row tile run back to back on one XCD
+// (workgroup i goes to XCD i mod 8), so its basis rows come from that L2.
 #include "device_common.h"
 
 namespace gimic {
 
-template <int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void contract_f64_kernel(ContractArgs a) {
-    constexpr int kRows = 32 * WAVES;
-    __shared__ double qs[kRows * kNQ];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int g = lane >> 4, c = lane & 15;
-    const int set = blockIdx.z, split = blockIdx.y;
-    const size_t row0 = (size_t)blockIdx.x * kRows;
-    const int lda = a.lda;
-    const size_t rows = (size_t)a.rows;
-    const size_t matsz = (size_t)a.ncol_pad * lda;
-    const size_t gplane = (size_t)a.gplane;
-    for (int i = tid; i < kRows * kNQ; i += 64 * WAVES) qs[i] = 0.0;
-    __syncthreads();
+namespace {
 
-    const double *A0 = a.a64 + (row0 + wave * 32 + c) * lda;
-    const double *A1 = A0 + 16 * (size_t)lda;
-    const double *Bset = a.b64 + (size_t)set * kNMat * matsz;
-    // the live 8-function groups of the listed blocks (tiles.hip), two per
-    // 16-wide K-step: lane group g takes group 2 kk + g / 2, elements
-    // 4 (g & 1) .. + 3.  A padding entry (-1) reads A from the zero buffer
-    // (B from any valid place: the product is zero).  Two per N-tile too:
-    // lane c owns function c & 7 of group 2 e + c / 8 (a padding entry: a
-    // column whose products the epilogue drops).
-    const int *K8 = a.k8list + (size_t)blockIdx.x * a.nblk * 4;
-    const int nks = (a.k8count[blockIdx.x] + 1) >> 1;
+typedef double v2d __attribute__((ext_vector_type(2)));
+
+constexpr int kUnits = kF64PairElems / 2;  // 16-byte units of a pair block
+constexpr int kStepUnits = 16 * kUnits;    // of a K-step: 16 pair blocks
+// s_waitcnt immediate: lgkmcnt 0, the other counters at their maximum
+constexpr int kWaitLds = 0xC07F;
+
+}  // namespace
+
+// one workgroup: 64 points of a row tile of a.tile_rows (64 or 128), a range
+// of its N-tiles; 4 wavefronts, two workgroups per CU
+__global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
+    constexpr int kRows = 64;
+    // [step mod 3][matrix][k pair][lane][2 k], lanes swizzled (below)
+    __shared__ v2d buf[3 * kStepUnits];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, c = lane & 15;
+    const int parts = a.tile_rows / kRows;  // workgroups that share a list and a range
+    const int xcd = blockIdx.x & 7, slot = (blockIdx.x >> 3) / parts;
+    const int ntile = a.rows / a.tile_rows, per_set = (ntile + 7) / 8 * a.nsplit;
+    const int set = slot / per_set, split = slot % a.nsplit;
+    const int rtile = slot % per_set / a.nsplit * 8 + xcd;
+    if (rtile >= ntile) return;
+    const int *K4 = a.klist + (size_t)rtile * a.nblk * 8;
+    const int nks = (a.kcount[rtile] + 3) >> 2;
     const int e0 = (int)((long long)split * nks / a.nsplit);
     const int e1 = (int)((long long)(split + 1) * nks / a.nsplit);
-    const double *zero = (const double *)a.bzero;
-    auto kent = [&](int kk) { return K8[2 * kk + (g >> 1)]; };
-    auto koff = [&](int v) { return v < 0 ? 0 : (v >> 12) * 8 + (g & 1) * 4; };
 
-    for (int e = e0; e < e1; e++) {
-        const int xn = K8[2 * e + (c >> 3)];
-        const bool live = xn >= 0;
-        const int col = live ? (xn >> 12) * 8 + (c & 7) : 0;
-        const double *Bc = Bset + (size_t)col * lda;
-        v4d acc[2][kNMat];
-#pragma unroll
-        for (int m = 0; m < kNMat; m++) acc[0][m] = acc[1][m] = v4d{0.0, 0.0, 0.0, 0.0};
+    const int ng = a.lda / 4;  // granules per row; index ng: the zero blocks
+    const v2d *B = (const v2d *)(a.b64 + (size_t)set * f64_set_elems(a.lda));
+    const size_t rowst = (size_t)(ng + 1) * kUnits;
+    const size_t row = (size_t)rtile * a.tile_rows + (blockIdx.x >> 3) % parts * kRows + wave * 16 + c;
+    const double *A = a.a64 + row * a.lda;
+    const double *G = a.g64 + row * a.lda;
+    const size_t gplane = (size_t)a.gplane;
+    const bool valid = row < (size_t)a.npts;
+    const double r[3] = {valid ? a.pts[3 * row] : 0.0, valid ? a.pts[3 * row + 1] : 0.0,
+                         valid ? a.pts[3 * row + 2] : 0.0};
+    // a padding entry (-1) reads the row's first granule against zero blocks
+    auto acol = [&](int v) { return v < 0 ? 0 : (v >> 13) * 4; };
 
-        const int v0 = kent(0), k0 = koff(v0);
-        v4d a0 = *(const v4d *)(v0 < 0 ? zero : A0 + k0), a1 = *(const v4d *)(v0 < 0 ? zero : A1 + k0);
-        v4d b[kNMat];
+    // Element pair sp of matrix m for lane l is at (2 m + sp) * 64 +
+    // (l ^ (l >> 3 & 1) ^ 2 sp): eight consecutive lanes of a read (c fixed in
+    // bit 3) and of a write (functions n = c >> 2 and sp of one pair block)
+    // then fall into different 16-byte columns.
+    // Wavefront w copies the pair blocks of K-granule w, one N-granule i a
+    // pass: lane < kUnits takes unit (m, sp, function n), for lane
+    // (w, i + 4 n), whose place is put0 ^ i.
+    const int unit = min(lane, kUnits - 1), un = unit & 3;
+    const int put0 = (unit >> 2) * 64 + ((wave * 16 + 4 * un) ^ un >> 1 ^ (unit >> 1 & 2));
+    const int rd0 = lane ^ (lane >> 3 & 1), rd1 = 64 + (rd0 ^ 2);
+
+    double q[kNQ];
 #pragma unroll
-        for (int m = 0; m < kNMat; m++) b[m] = *(const v4d *)(Bc + m * matsz + k0);
-        // group entry of the next K-step, read one step early
-        int vnext = kent(nks > 1 ? 1 : 0);
-        for (int kk = 0; kk < nks; kk++) {
-            // prefetch the next K-step while this one runs on the matrix cores
-            const int vn = vnext, kn = koff(vn);
-            vnext = kent(kk + 2 < nks ? kk + 2 : nks - 1);
-            const v4d na0 = *(const v4d *)(vn < 0 ? zero : A0 + kn);
-            const v4d na1 = *(const v4d *)(vn < 0 ? zero : A1 + kn);
-            v4d nb[kNMat];
+    for (int i = 0; i < kNQ; i++) q[i] = 0.0;
+
+    if (e0 < e1) {
+        // The K-steps of all N-tiles form one sequence t.  During step t the
+        // workgroup computes on buffer t mod 3, stores step t + 2 (loaded
+        // during step t - 1) and loads step t + 3; one barrier ends a step.
+        // Step t + 1 was complete before step t began, so its first operands
+        // are read before the barrier and the matrix pipe does not drain.
+        int fe = e0, fk = 0;  // N-tile and K-step of the next load
+        // (list entries are read a K-step or an N-tile early and used raw, per
+        // lane: a scalar or converted value would be waited for at once)
+        unsigned noff[4];
+        int4 nxt;
+        auto offsets = [&] {
+            const int x[4] = {nxt.x, nxt.y, nxt.z, nxt.w};
 #pragma unroll
-            for (int m = 0; m < kNMat; m++) nb[m] = *(const v4d *)(Bc + m * matsz + kn);
+            for (int i = 0; i < 4; i++)
+                noff[i] = ((unsigned)(x[i] < 0 ? ng : x[i] >> 13) * kUnits + unit) * 16u;
+        };
+        nxt = *(const int4 *)(K4 + 4 * fe);
+        offsets();
+        nxt = *(const int4 *)(K4 + 4 * min(fe + 1, e1 - 1));
+        v2d st[4];
+        const int wv = tid >> 6;
+        int kent = K4[wv];
+        auto source = [&] {
+            const int x = __builtin_amdgcn_readfirstlane(kent);
+            return (const char *)(B + (size_t)(x < 0 ? ng : x >> 13) * rowst);
+        };
+        auto load = [&](const char *src) {
 #pragma unroll
-            for (int s = 0; s < 4; s++) {
-#pragma unroll
-                for (int m = 0; m < kNMat; m++) {
-                    acc[0][m] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[s], b[m][s], acc[0][m], 0, 0, 0);
-                    acc[1][m] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[s], b[m][s], acc[1][m], 0, 0, 0);
-                }
+            for (int i = 0; i < 4; i++) st[i] = *(const v2d *)(src + noff[i]);
+            if (++fk == nks) {  // on to the next N-tile (past the last: it again)
+                fk = 0;
+                fe = min(fe + 1, e1 - 1);
+                offsets();
+                nxt = *(const int4 *)(K4 + 4 * min(fe + 1, e1 - 1));
             }
-            a0 = na0;
-            a1 = na1;
+            kent = K4[4 * fk + wv];  // for the next step's load
+        };
+        auto put = [&](v2d *b) {
+            if (lane < kUnits)
 #pragma unroll
-            for (int m = 0; m < kNMat; m++) b[m] = nb[m];
-        }
+                for (int i = 0; i < 4; i++) b[put0 ^ i] = st[i];
+        };
+        int cur = 0, nx1 = kStepUnits, nx2 = 2 * kStepUnits;  // buffers of steps t, t + 1, t + 2
+        load(source());
+        put(buf + cur);
+        load(source());
+        put(buf + nx1);
+        load(source());
+        v4d an = *(const v4d *)(A + acol(K4[g]));
+        int xa = K4[(nks > 1 ? 4 : 0) + g];  // the next K-step's granule
+        __syncthreads();
+        v2d b0[kNMat];
+#pragma unroll
+        for (int m = 0; m < kNMat; m++) b0[m] = buf[cur + rd0 + m * 128];
 
-        // epilogue: for the f64 16x16x4 builtin, lane (g, c) holds
-        // Y_mat[row g + 4r][col c] of each block (checked by the MFMA
-        // layout self-test)
-        const double R[3] = {a.rf64[col], a.rf64[a.ncol_pad + col], a.rf64[2 * a.ncol_pad + col]};
+        for (int e = e0; e < e1; e++) {
+            // the epilogue's operands: the four functions of this lane's granule
+            const int xn = K4[4 * e + g];
+            const v4d ph = *(const v4d *)(A + acol(xn));
+            const v4d g0 = *(const v4d *)(G + acol(xn)), g1 = *(const v4d *)(G + gplane + acol(xn)),
+                      g2 = *(const v4d *)(G + 2 * gplane + acol(xn));
+            v4d acc[kNMat];
 #pragma unroll
-        for (int rb = 0; rb < 2; rb++) {
+            for (int m = 0; m < kNMat; m++) acc[m] = v4d{0.0, 0.0, 0.0, 0.0};
+            for (int ks = 0; ks < nks; ks++) {
+                const v4d av = an;
+                v2d b1[kNMat];
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int rl = wave * 32 + rb * 16 + g + 4 * r;
-                const size_t p = row0 + rl;
-                const bool valid = p < (size_t)a.npts;
-                const double rp[3] = {valid ? a.pts[3 * p] : 0.0, valid ? a.pts[3 * p + 1] : 0.0,
-                                      valid ? a.pts[3 * p + 2] : 0.0};
-                const double ph = live ? a.a64[p * lda + col] : 0.0;
-                const double G[3] = {live ? a.g64[p * lda + col] : 0.0,
-                                     live ? a.g64[gplane + p * lda + col] : 0.0,
-                                     live ? a.g64[2 * gplane + p * lda + col] : 0.0};
-                const double y0 = acc[rb][0][r];
-                double q[kNQ];
-                q[0] = y0 * ph;
+                for (int m = 0; m < kNMat; m++) b1[m] = buf[cur + rd1 + m * 128];
+                an = *(const v4d *)(A + acol(xa));
+                xa = K4[4 * (ks + 2 < nks ? ks + 2 : ks + 2 - nks < nks ? ks + 2 - nks : 0) + g];
 #pragma unroll
-                for (int d = 0; d < 3; d++) q[1 + d] = q[0] * (rp[d] - R[d]);
+                for (int m = 0; m < kNMat; m++)
+                    acc[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(b0[m].x, av[0], acc[m], 0, 0, 0);
+                const char *src = source();
 #pragma unroll
-                for (int bb = 0; bb < 3; bb++)
+                for (int m = 0; m < kNMat; m++)
+                    acc[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(b0[m].y, av[1], acc[m], 0, 0, 0);
+                put(buf + nx2);
+                load(src);
 #pragma unroll
-                    for (int m = 0; m < 3; m++) q[4 + m + 3 * bb] = acc[rb][1 + bb][r] * G[m];
+                for (int m = 0; m < kNMat; m++) b0[m] = buf[nx1 + rd0 + m * 128];
 #pragma unroll
-                for (int d = 0; d < 3; d++)
+                for (int m = 0; m < kNMat; m++)
+                    acc[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(b1[m].x, av[2], acc[m], 0, 0, 0);
 #pragma unroll
-                    for (int m = 0; m < 3; m++) q[13 + m + 3 * d] = G[m] * acc[rb][4 + d][r];
+                for (int m = 0; m < kNMat; m++)
+                    acc[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(b1[m].y, av[3], acc[m], 0, 0, 0);
+                // every wavefront has stored its part of step t + 2 and read
+                // buffer t (a bare barrier: a fence would wait for the loads)
+                __builtin_amdgcn_s_waitcnt(kWaitLds);
+                __builtin_amdgcn_s_barrier();
+                const int done = cur;
+                cur = nx1;
+                nx1 = nx2;
+                nx2 = done;
+            }
+
+            // lane (g, c) holds Y_mat of function i of granule g at point c in
+            // element i of each block (row g + 4 i of the block: the MFMA
+            // layout self-test); a padding granule's products are zero
+            const int fn = xn < 0 ? 0 : (xn >> 13) * 4;
+            const v4d R0 = *(const v4d *)(a.rf64 + fn), R1 = *(const v4d *)(a.rf64 + a.lda + fn),
+                      R2 = *(const v4d *)(a.rf64 + 2 * (size_t)a.lda + fn);
 #pragma unroll
-                for (int i = 0; i < kNQ; i++) q[i] = row16_sum(q[i]);
+            for (int i = 0; i < 4; i++) {
+                const double t = acc[0][i] * ph[i];
+                const double gr[3] = {g0[i], g1[i], g2[i]};
+                q[0] += t;
+                q[1] += t * (r[0] - R0[i]);
+                q[2] += t * (r[1] - R1[i]);
+                q[3] += t * (r[2] - R2[i]);
 #pragma unroll
-                for (int i = 0; i < kNQ; i++)
-                    if ((i & 15) == c) qs[rl * kNQ + i] += q[i];
+                for (int b = 0; b < 3; b++)
+#pragma unroll
+                    for (int m = 0; m < 3; m++) {
+                        q[4 + m + 3 * b] += acc[1 + b][i] * gr[m];
+                        q[13 + m + 3 * b] += gr[m] * acc[4 + b][i];
+                    }
             }
         }
     }
-    __syncthreads();
-    double *out = a.part + ((size_t)set * a.nsplit + split) * kNQ * rows + row0;
-    for (int i = tid; i < kRows * kNQ; i += 64 * WAVES) {
-        const int q = i / kRows, rl = i % kRows;
-        out[(size_t)q * rows + rl] = qs[rl * kNQ + q];
+
+    // add the four lane groups; group g stores sums g, g + 4, ...
+    double *out = a.part + ((size_t)set * a.nsplit + split) * kNQ * (size_t)a.rows + row;
+#pragma unroll
+    for (int j = 0; j < kNQ; j += 4) {
+        double s[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            s[i] = j + i < kNQ ? q[j + i < kNQ ? j + i : 0] : 0.0;
+            s[i] += __shfl_xor(s[i], 16);
+            s[i] += __shfl_xor(s[i], 32);
+        }
+        const double v = g == 0 ? s[0] : g == 1 ? s[1] : g == 2 ? s[2] : s[3];
+        if (j + g < kNQ) out[(size_t)(j + g) * a.rows] = v;
     }
 }
 
-hipError_t launch_contract_f64(const ContractArgs &a, int tile_rows, hipStream_t s) {
-    if (tile_rows != 64 && tile_rows != 128) return hipErrorInvalidValue;
-    if (a.rows % tile_rows) return hipErrorInvalidValue;
-    dim3 grid(a.rows / tile_rows, a.nsplit, a.nmatset);
-    if (tile_rows == 64)
-        hipLaunchKernelGGL(contract_f64_kernel<2>, grid, dim3(128), 0, s, a);
-    else
-        hipLaunchKernelGGL(contract_f64_kernel<4>, grid, dim3(256), 0, s, a);
+hipError_t launch_contract_f64(const ContractArgs &a, hipStream_t s) {
+    if ((a.tile_rows != 64 && a.tile_rows != 128) || a.rows % a.tile_rows || a.lda % 32 ||
+        a.ncol_pad != a.lda)
+        return hipErrorInvalidValue;
+    const long long nwg = 8LL * ((a.rows / a.tile_rows + 7) / 8) * a.nsplit * a.nmatset *
+                          (a.tile_rows / 64);
+    if (nwg > 0x7fffffffLL) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(contract_f64_kernel, dim3((unsigned)nwg), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -225,13 +225,13 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
     // N-tiles and K-steps of four live 8-function groups: entry = (global
     // group << 12) | position of the group in this tile's compressed rows;
     // -1 pads the last four (zero right operand)
-    const int *K8 = a.k8list + (size_t)rtile * a.nblk * 4;
-    const int nq = (a.k8count[rtile] + 3) >> 2;
+    const int *K8 = a.klist + (size_t)rtile * a.nblk * 4;
+    const int nq = (a.kcount[rtile] + 3) >> 2;
     // This tile's basis rows: dense [row][lda], or compressed to the live
     // groups (a.toff non-null: the basis kernel wrote only those, so A and
     // the gradients are addressed by list position)
     const bool cmp = a.toff != nullptr;
-    const size_t wcols = cmp ? (size_t)8 * a.k8count[rtile] : (size_t)lda;  // functions per row
+    const size_t wcols = cmp ? (size_t)8 * a.kcount[rtile] : (size_t)lda;  // functions per row
     const size_t arow = kAParts * wcols;                                     // BF16 per split row
     const __bf16 *Atile = cmp ? a.as3 + (size_t)a.toff[rtile] * kRows * (8 * kAParts)
                               : a.as3 + row0 * arow;

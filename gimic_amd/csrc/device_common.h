@@ -99,12 +99,12 @@ struct EvalArgs {
     size_t lds_image;    // bytes of its LDS image (set by the launcher)
     int lmax;            // largest shell l of the basis
     // Compressed split output (staged kernel, toff non-null): a row tile of
-    // tile_rows rows keeps only its k8count[t] live 8-function groups
-    // (k8list[t * 4 nblk ...], global group << 12 | place k in the row); its
+    // tile_rows rows keeps only its kcount[t] live 8-function groups
+    // (klist[t * 4 nblk ...], global group << 12 | place k in the row); its
     // rows start at element toff[t] * tile_rows * 8 kAParts of phis
     // ([row][k][kAParts][8]) and toff[t] * tile_rows * 24 of grad32
     // ([3][tile_rows][8 k])
-    const int *k8count, *k8list, *toff;
+    const int *kcount, *klist, *toff;
     int nblk, tile_rows;
 };
 hipError_t launch_basis_eval(const EvalArgs &a, int mode, hipStream_t s);
@@ -124,19 +124,24 @@ struct ContractArgs {
     const double *rf64;  // [3][ncol_pad] atom coordinate of each function
     const float *rf32;
     double *part;        // [nmatset][nsplit][kNQ][rows]; pre-split kernels: [nmatset][nsplit][rows][kNQ]
-    // screening lists per row tile (TileArgs): the live 8-function groups of
-    // the listed 32-function blocks, k8count[t] of them in k8list[t * 4 nblk
-    // ...]; the pre-split kernels take four per N-tile and K-step, the FP64
-    // kernel two (a zeroed 12 KiB buffer stands in for its padding groups);
+    // screening lists per row tile (TileArgs): its live groups of 8 functions
+    // (pre-split kernels) or 4 (FP64 kernel), four per N-tile and K-step;
     // split s of a tile takes N-tiles [s * count / nsplit, (s+1) * count / nsplit)
-    int nblk;
-    const int *k8count, *k8list;
-    const __bf16 *bzero;
+    int nblk, tile_rows;  // tile_rows: FP64 kernel only
+    const int *kcount, *klist;
     // compressed operands (pre-split kernels; see EvalArgs): null for dense
     const int *toff;
 };
-// FP64 kernel: row tiles of tile_rows = 64 or 128 points (a.rows a multiple)
-hipError_t launch_contract_f64(const ContractArgs &a, int tile_rows, hipStream_t s);
+// FP64 right operand in HBM: one pair block per (density set, 4-function
+// K-granule, 4-function N-granule) of 7 matrices x 4 x 4 elements,
+// [matrix][k / 2][n][k % 2]; K-granules major, each row ending in a zero pair
+// block and a zero row last (the padding entries of the granule lists)
+constexpr int kF64PairElems = kNMat * 16;
+__host__ __device__ constexpr size_t f64_set_elems(int lda) {
+    return (size_t)(lda / 4 + 1) * (size_t)(lda / 4 + 1) * kF64PairElems;
+}
+// FP64 kernel: row tiles of a.tile_rows = 64 or 128 points (a.rows a multiple)
+hipError_t launch_contract_f64(const ContractArgs &a, hipStream_t s);
 // Pre-split variant: both operands arrive as BF16 parts, the right operand in
 // pair blocks that the kernel gathers into its LDS buffers (see
 // contract_mx2.hip); nbuf 2 or 3 LDS buffers, krb 2 or 4 row blocks per
@@ -178,8 +183,8 @@ constexpr int kMx2BlockElems = (4 * kMx2GroupElems * 2 + 1023) / 1024 * 512;
 // `second` is set; element (mu, nu) in caller order at mu * n + nu (row_major)
 // or mu + n * nu; fun[i] is the caller's index of internal function i < n,
 // rf64 the centres [3][ld] by internal index.  One set's operand each:
-// launch_operand_f64 [matrix][nu][mu] with rows of ld, launch_operand_split the
-// pair blocks of mx2_set_elems(ld, ld) elements; padding is written as zeros.
+// the pair blocks of f64_set_elems(ld) and mx2_set_elems(ld, ld) elements;
+// padding is written as zeros.
 struct OperandArgs {
     const double *dens, *second;
     int subtract, row_major;
@@ -260,18 +265,20 @@ struct TileArgs {
     const double *spts;  // sorted chunk points
     int npts, rows;      // valid and padded rows
     int tile_rows;       // rows per contraction workgroup
-    int nblk;            // 32-function blocks (lda / 32)
-    const int *blk_beg;  // [nblk + 1] ranges into blk_sh
-    const int *blk_sh;   // shells with a function in each block
+    int nblk;            // 32-function blocks (lda / 32), at most 1024
+    int gran;            // functions per list entry: 8 (mixed) or 4 (FP64)
     const DevShell *shells;
+    int nshell;
     const double *coords;
-    int *bcount, *blist;  // [rows / tile_rows], [rows / tile_rows][nblk]
-    // 8-function groups of the listed blocks that screening leaves non-zero:
-    // k8count[t] groups, k8list[t * 4 nblk ...] = (global group << 12) |
-    // (place k of the group in this list: its place in the compressed rows), padded
-    // with -1 to a multiple of 4 (nblk <= 1024)
-    int *k8count, *k8list;
+    // per row tile: 32-function blocks and 8-function groups that screening
+    // can leave non-zero (statistics), and the list the contraction walks, the
+    // live groups of `gran` functions in ascending order: kcount[t] entries at
+    // klist[t * 32 nblk / gran ...], (global group << list_shift(gran)) | (place of the
+    // entry in this list: its place in compressed rows), padded with -1 to a
+    // multiple of 4
+    int *bcount, *k8count, *kcount, *klist;
 };
+constexpr int list_shift(int gran) { return gran == 8 ? 12 : 13; }
 hipError_t launch_block_lists(const TileArgs &a, hipStream_t s);
 // toff[t] = sum of cnt[0 .. t-1] for t = 0 .. ntiles (one workgroup)
 hipError_t launch_tile_offsets(const int *cnt, int ntiles, int *toff, hipStream_t s);

@@ -6,8 +6,7 @@
 // order (fun), combine the spin sets, form W_d(mu,nu) = D(mu,nu)
 // (R_nu - R_mu)_d, and write the layout a kernel reads.  One thread per
 // element (mu, nu) computes all seven matrices, so D and the centres are
-// loaded once; a wavefront covers 8 x 8 elements, whose stores are whole
-// 64- or 128-byte pieces.  Bound by memory: 32 bytes read and 56 (FP64) or 42
+// loaded once; the stores of a wavefront are whole 128-byte pieces.  Bound by memory: 32 bytes read and 56 (FP64) or 42
 // (split) bytes written per element.  Building them on the host and copying them
 // took most of a first evaluation: a whole run on the 60-atom cage (nbf 1800:
 // context, densities, one 140 x 140 plane in FP64) went from 214 to 101 ms, the
@@ -41,16 +40,20 @@ __device__ __forceinline__ void operand_values(const OperandArgs &a, int mu, int
         v[4 + d] = v[0] * (a.rf64[(size_t)d * a.ld + nu] - a.rf64[(size_t)d * a.ld + mu]);
 }
 
-// FP64: [matrix][nu][mu], rows of ld
+// FP64: 16 threads per pair block, 16 pair blocks of one K-granule row per
+// workgroup; a matrix's 16 elements are 128 contiguous bytes
 __global__ __launch_bounds__(256) void operand_f64_kernel(OperandArgs a, double *out) {
-    const int t = threadIdx.x;
-    const int mu = blockIdx.x * 64 + (t & 63), nu = blockIdx.y * 4 + (t >> 6);
-    if (mu >= a.ld || nu >= a.ld) return;
+    const int t = threadIdx.x & 15, ng = a.ld / 4;
+    const int gn = blockIdx.x * 16 + (threadIdx.x >> 4), gk = blockIdx.y;
+    if (gn > ng) return;
+    // consecutive threads take the elements in their order in the block
+    const int k = 2 * (t >> 3) + (t & 1), n = (t >> 1) & 3;
     double v[kNMat];
-    operand_values(a, mu, nu, v);
-    const size_t matsz = (size_t)a.ld * a.ld;
+    // (the zero blocks' indices are at least ld >= n: operand_values gives 0)
+    operand_values(a, gk * 4 + k, gn * 4 + n, v);
+    double *dst = out + ((size_t)gk * (ng + 1) + gn) * kF64PairElems + t;
 #pragma unroll
-    for (int m = 0; m < kNMat; m++) out[m * matsz + (size_t)nu * a.ld + mu] = v[m];
+    for (int m = 0; m < kNMat; m++) dst[m * 16] = v[m];
 }
 
 // split: the FP32 value of each element as kBParts BF16 parts (three parts:
@@ -62,7 +65,6 @@ __global__ __launch_bounds__(256) void operand_split_kernel(OperandArgs a, uint1
     if (gn > ng) return;
     const int nn = lane >> 3, kk = lane & 7;
     double v[kNMat];
-    // (the zero blocks' indices are at least ld >= n: operand_values gives 0)
     operand_values(a, gk * 8 + kk, gn * 8 + nn, v);
     uint16_t *dst = out + ((size_t)gk * (ng + 1) + gn) * kMx2PairElems + lane;
 #pragma unroll
@@ -80,9 +82,9 @@ __global__ __launch_bounds__(256) void operand_split_kernel(OperandArgs a, uint1
 }  // namespace
 
 hipError_t launch_operand_f64(const OperandArgs &a, double *out, hipStream_t s) {
-    if (a.n < 0 || a.ld < a.n || a.ld % 32 || (a.ld + 3) / 4 > 65535) return hipErrorInvalidValue;
-    if (a.ld == 0) return hipSuccess;
-    hipLaunchKernelGGL(operand_f64_kernel, dim3((a.ld + 63) / 64, a.ld / 4), dim3(256), 0, s, a, out);
+    if (a.n < 0 || a.ld < a.n || a.ld % 32 || a.ld / 4 + 1 > 65535) return hipErrorInvalidValue;
+    const int ng = a.ld / 4;
+    hipLaunchKernelGGL(operand_f64_kernel, dim3(ng / 16 + 1, ng + 1), dim3(256), 0, s, a, out);
     return hipGetLastError();
 }
 

@@ -15,10 +15,10 @@
 //     on every run); the basis, contraction and finalize kernels work on the
 //     sorted rows, and finalize writes each tensor back to its caller index.
 //  2. For every row tile of the contraction kernel, list in ascending order
-//     the blocks holding a function whose centre lies within its screening
-//     radius of the tile's bounding box (a conservative test: a block that
-//     is zero over the tile may be listed, one that is not is never left
-//     out).
+//     the groups of 8 or 4 functions touched by a shell whose centre lies
+//     within its screening radius of the tile's bounding box (a conservative
+//     test: a group that is zero over the tile may be listed, one that is
+//     not is never left out).
 #include "device_common.h"
 
 namespace gimic {
@@ -194,14 +194,17 @@ __global__ __launch_bounds__(256) void gather_points_kernel(const double *pts, c
     for (int d = 0; d < 3; d++) spts[3 * j + d] = pts[3 * (long long)i + d];
 }
 
-// One workgroup per row tile: bounding box of its valid rows, then the
-// ascending list of blocks with a function that may be non-zero there.
+// One workgroup per row tile: bounding box of its valid rows, the granules (4
+// functions) that a shell within reach of it touches, and the ascending list
+// of the live groups.  Threads take shells for the liveness test and blocks
+// for the list (positions by a prefix sum): one thread walking the blocks
+// took 12 us for a single tile, this 5.
 constexpr int kMaxBlk = 1024;  // 32-function blocks per row (32768 functions)
 
 __global__ __launch_bounds__(256) void block_list_kernel(TileArgs a) {
-    __shared__ double s[6][256];
-    __shared__ int wsum[4];
-    __shared__ unsigned char gmask[kMaxBlk];  // live 8-function groups of each block
+    __shared__ double box[4][6];
+    __shared__ int wsum[4][3];
+    __shared__ unsigned live[kMaxBlk];  // live granules of each block, 8 bits
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const long long r0 = (long long)blockIdx.x * a.tile_rows;
     double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
@@ -215,77 +218,89 @@ __global__ __launch_bounds__(256) void block_list_kernel(TileArgs a) {
                 hi[d] = fmax(hi[d], x);
             }
     }
+    for (int b = t; b < a.nblk; b += 256) live[b] = 0u;
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
-        s[d][t] = lo[d];
-        s[3 + d][t] = hi[d];
-    }
+    for (int w = 32; w > 0; w >>= 1)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            lo[d] = fmin(lo[d], __shfl_xor(lo[d], w));
+            hi[d] = fmax(hi[d], __shfl_xor(hi[d], w));
+        }
+    if (lane == 0)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            box[wave][d] = lo[d];
+            box[wave][3 + d] = hi[d];
+        }
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w)
+#pragma unroll
+    for (int w = 0; w < 4; w++)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            lo[d] = fmin(lo[d], box[w][d]);
+            hi[d] = fmax(hi[d], box[w][3 + d]);
+        }
+    if (r0 < a.npts)
+        for (int k = t; k < a.nshell; k += 256) {
+            const DevShell sh = a.shells[k];
+            const double *R = a.coords + 3 * sh.atom;
+            double d2 = 0.0;
 #pragma unroll
             for (int d = 0; d < 3; d++) {
-                s[d][t] = fmin(s[d][t], s[d][t + w]);
-                s[3 + d][t] = fmax(s[3 + d][t], s[3 + d][t + w]);
+                const double e = fmax(0.0, fmax(lo[d] - R[d], R[d] - hi[d]));
+                d2 += e * e;
             }
-        __syncthreads();
-    }
-    const double blo[3] = {s[0][0], s[1][0], s[2][0]}, bhi[3] = {s[3][0], s[4][0], s[5][0]};
-    const bool any = r0 < a.npts;
-    int *list = a.blist + (long long)blockIdx.x * a.nblk;
-    int base = 0;
-    const unsigned long long below = (1ull << lane) - 1ull;
+            // relative slack for rounding in the basis kernel's own distance
+            if (sqrt(d2) <= sh.radius * (1.0 + 1e-12) + 1e-12)
+                for (int q = sh.fout >> 2; q <= (sh.fout + sh.ncomp_out - 1) >> 2; q++)
+                    atomicOr(&live[q >> 3], 1u << (q & 7));
+        }
+    __syncthreads();
+    const int per = 32 / a.gran, shift = a.gran == 8 ? 12 : 13;
+    int *list = a.klist + (long long)blockIdx.x * a.nblk * per;
+    int base = 0, nb = 0, n8 = 0;
     for (int b0 = 0; b0 < a.nblk; b0 += 256) {
         const int b = b0 + t;
-        bool act = false;
-        unsigned m4 = 0;  // groups of 8 functions that a live shell touches
-        if (any && b < a.nblk) {
-            for (int k = a.blk_beg[b]; k < a.blk_beg[b + 1] && m4 != 15u; k++) {
-                const DevShell sh = a.shells[a.blk_sh[k]];
-                const double *R = a.coords + 3 * sh.atom;
-                double d2 = 0.0;
+        const unsigned m4 = b < a.nblk ? live[b] : 0u;   // granules of 4
+        const unsigned m8 = (m4 | m4 >> 1) & 0x55u;      // groups of 8, every second bit
+        const unsigned m = a.gran == 8 ? m8 : m4;
+        const int cnt = __popc(m);
+        int inc = cnt;
 #pragma unroll
-                for (int d = 0; d < 3; d++) {
-                    const double e = fmax(0.0, fmax(blo[d] - R[d], R[d] - bhi[d]));
-                    d2 += e * e;
-                }
-                // relative slack for rounding in the basis kernel's own distance
-                if (sqrt(d2) <= sh.radius * (1.0 + 1e-12) + 1e-12) {
-                    const int f0 = max(0, sh.fout - 32 * b);
-                    const int f1 = min(31, sh.fout + sh.ncomp_out - 1 - 32 * b);
-                    for (int gq = f0 >> 3; gq <= (f1 >> 3); gq++) m4 |= 1u << gq;
-                }
+        for (int d = 1; d < 64; d <<= 1) {
+            const int y = __shfl_up(inc, d);
+            if (lane >= d) inc += y;
+        }
+        int g8 = __popc(m8);
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) g8 += __shfl_xor(g8, d);
+        const int blocks = __popcll(__ballot(m4 != 0u));
+        if (lane == 63) {
+            wsum[wave][0] = inc;
+            wsum[wave][1] = g8;
+            wsum[wave][2] = blocks;
+        }
+        __syncthreads();
+        int pos = base + inc - cnt;
+        for (int w = 0; w < 4; w++) {
+            if (w < wave) pos += wsum[w][0];
+            base += wsum[w][0];
+            n8 += wsum[w][1];
+            nb += wsum[w][2];
+        }
+        for (int q = 0; q < per; q++)
+            if (m >> (a.gran == 8 ? 2 * q : q) & 1u) {
+                list[pos] = (per * b + q) << shift | pos;
+                pos++;
             }
-            act = m4 != 0u;
-        }
-        if (b < a.nblk) gmask[b] = (unsigned char)m4;
-        const unsigned long long m = __ballot(act);
-        if (lane == 0) wsum[wave] = __popcll(m);
-        __syncthreads();
-        int pos = base + __popcll(m & below);
-        for (int w = 0; w < wave; w++) pos += wsum[w];
-        if (act) list[pos] = b;
-        base += wsum[0] + wsum[1] + wsum[2] + wsum[3];
         __syncthreads();
     }
-    if (t == 0) a.bcount[blockIdx.x] = base;
-    // the live groups in list order, four per K-step (the last padded with -1)
-    __syncthreads();
     if (t == 0) {
-        int *kl = a.k8list + (long long)blockIdx.x * a.nblk * 4;
-        int k = 0;
-        for (int b = 0; b < a.nblk; b++) {
-            const unsigned m = gmask[b];
-            if (!m) continue;
-            for (int gq = 0; gq < 4; gq++)
-                if (m >> gq & 1u) {
-                    kl[k] = ((4 * b + gq) << 12) | k;
-                    k++;
-                }
-        }
-        a.k8count[blockIdx.x] = k;
-        while (k & 3) kl[k++] = -1;
+        a.bcount[blockIdx.x] = nb;
+        a.k8count[blockIdx.x] = n8;
+        a.kcount[blockIdx.x] = base;
     }
+    if (t < (-base & 3)) list[base + t] = -1;  // four per N-tile and K-step
 }
 
 // exclusive prefix sum of the tiles' live group counts, toff[0 .. n]
@@ -351,7 +366,8 @@ hipError_t launch_sort_points(const double *pts, int n, double *spts, int *perm,
 }
 
 hipError_t launch_block_lists(const TileArgs &a, hipStream_t s) {
-    if (a.tile_rows <= 0 || a.rows % a.tile_rows || a.nblk <= 0 || a.nblk > kMaxBlk)
+    if (a.tile_rows <= 0 || a.rows % a.tile_rows || a.nblk <= 0 || a.nblk > kMaxBlk ||
+        (a.gran != 8 && a.gran != 4))
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(block_list_kernel, dim3(a.rows / a.tile_rows), dim3(256), 0, s, a);
     return hipGetLastError();
