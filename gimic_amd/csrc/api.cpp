@@ -678,21 +678,22 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
         return round_up((rows_all + nmin - 1) / nmin, gran);
     };
     chunk = even_chunks(chunk);
-    // padding columns and rows of the basis buffers must read as zero: they
-    // are cleared when (re)allocated (every Scratch-mode call carves them
-    // afresh) and never written afterwards.  On an allocation failure in
-    // eager mode the other precision's basis buffers are released first, then
-    // the chunk is halved (smaller chunks change only the tiles' block lists,
-    // i.e. the results' last bits)
+    // Compressed rows are written whole; the dense FP64 rows of very wide bases
+    // have padding columns that must read as zero: cleared when (re)allocated
+    // and never written afterwards.  On an allocation failure in eager mode the
+    // other precision's basis buffers are released first, then the chunk is
+    // halved (smaller chunks change only the tiles' block lists, i.e. the
+    // results' last bits)
+    const bool dense = prec == GIMIC_PREC_FP64 && ld * 32 > kMaxRowBytes;
     for (;;) {
         const size_t rc = chunk;
         try {
             if (prec == GIMIC_PREC_FP64) {
-                grow(W.phi64, rc * ld * 8, W.phi64.bytes < rc * ld * 8);
-                grow(W.grad64, 3 * rc * ld * 8, W.grad64.bytes < 3 * rc * ld * 8);
+                grow(W.phi64, rc * ld * 8, dense && W.phi64.bytes < rc * ld * 8);
+                grow(W.grad64, 3 * rc * ld * 8, dense && W.grad64.bytes < 3 * rc * ld * 8);
             } else {
-                grow(W.phis, rc * ld * 2 * kAParts, W.phis.bytes < rc * ld * 2 * kAParts);
-                grow(W.grad32, 3 * rc * ld * 4, W.grad32.bytes < 3 * rc * ld * 4);
+                grow(W.phis, rc * ld * 2 * kAParts, false);
+                grow(W.grad32, 3 * rc * ld * 4, false);
             }
             break;
         } catch (const Error &e) {
@@ -841,14 +842,12 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
             if (variant == 0) plan(f64_tile_rows(n_c), kNT);
             else plan(mixed_tile_rows(variant), kMx2Cols / kNMat, split);
         };
-        // mixed kernels: row-major partial sums (written whole by the launch),
-        // and basis rows compressed to each row tile's live groups (lists
-        // and offsets built before the basis evaluation)
+        // row-major partial sums from the mixed kernels, written whole by the launch
+        const int tr64 = f64_tile_rows(n_c);
         auto run = [&](int variant, int split = -1) {
             plan_variant(variant, split);
-            if (variant == 0) lists(f64_tile_rows(n_c), 4);  // the FP64 kernel walks lists over dense rows
-            ca.toff = variant != 0 ? W.toff.as<int>() : nullptr;
-            ca.tile_rows = f64_tile_rows(n_c);
+            ca.toff = dense ? nullptr : W.toff.as<int>();
+            ca.tile_rows = tr64;
             if (variant == 0) hip_check(launch_contract_f64(ca, st), "contract_f64");
             else if (variant == 3) hip_check(launch_contract_mx2(ca, 2, 2, 4, st), "contract_mx2");
             else if (variant == 4) hip_check(launch_contract_mx2(ca, 3, 2, 4, st), "contract_mx2");
@@ -856,21 +855,19 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
             else if (variant == 8) hip_check(launch_contract_mx2(ca, 2, 2, 8, st), "contract_mx2");
             else hip_check(launch_contract_mx2(ca, 3, 2, 8, st), "contract_mx2");
         };
-        // basis evaluation: FP64 rows (mode 0), or the compressed split rows
-        // the mixed kernels read (mode 2)
+        // basis evaluation: FP64 rows (mode 0) or split rows (mode 2), compressed
+        // to each row tile's live groups (lists and offsets come first)
         auto eval = [&](int variant) {
-            ea.toff = nullptr;
-            if (variant != 0) {
-                const int tr = mixed_tile_rows(variant);
-                lists(tr, 8);
+            const int tr = variant == 0 ? tr64 : mixed_tile_rows(variant);
+            lists(tr, variant == 0 ? 4 : 8);
+            if (!dense)
                 hip_check(launch_tile_offsets(W.kcount.as<int>(), rows / tr, W.toff.as<int>(), st),
                           "tile_offsets");
-                ea.kcount = W.kcount.as<int>();
-                ea.klist = W.klist.as<int>();
-                ea.toff = W.toff.as<int>();
-                ea.nblk = nblk;
-                ea.tile_rows = tr;
-            }
+            ea.kcount = W.kcount.as<int>();
+            ea.klist = W.klist.as<int>();
+            ea.toff = dense ? nullptr : W.toff.as<int>();
+            ea.nblk = nblk;
+            ea.tile_rows = tr;
             hip_check(launch_basis_eval(ea, variant == 0 ? 0 : 2, st), "basis_eval");
         };
         // tensor assembly (and flux contributions) of this chunk from the

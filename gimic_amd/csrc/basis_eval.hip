@@ -13,13 +13,16 @@
 // ones.  Outputs: phi (the contraction's left operand) and its gradient in
 // FP64 for the FP64 path.
 //
-// The split output of the mixed kernels (phi as three BF16 parts plus FP32
-// gradients), and the FP64 rows of bases up to 4,800 functions, are
-// produced by basis_eval_staged_kernel: a workgroup
-// owns a tile of 1-32 whole point rows, its threads evaluate (point,
-// contraction) pairs into a zeroed LDS image of those rows, and the rows
-// then leave with 16-byte coalesced stores.  Written directly, every store
-// instruction of a wavefront scatters 64 short values over a whole row.
+// basis_eval_staged_kernel writes the rows that the contraction kernels read: a
+// workgroup owns 32 whole point rows, its threads evaluate (point,
+// contraction) pairs into a zeroed LDS image of some of those rows, and the
+// rows then leave with 16-byte coalesced stores.  Written directly, every
+// store instruction of a wavefront scatters 64 short values over a whole row;
+// that is left to the FP64 rows of bases too wide for the image
+// (basis_eval_kernel).
+#include <algorithm>
+#include <type_traits>
+
 #include "device_common.h"
 
 namespace gimic {
@@ -76,8 +79,14 @@ constexpr int kCandChunk = 1024;
 // sphere, per-wavefront counts
 constexpr size_t kCandBytes = kCandChunk * 2 + 4 * 8 + 4 * 4;
 
-// LDS image of a tile of rows for basis_eval_staged_kernel:
-//   [tile_points][lda/8][3][8] BF16 parts of phi, then [3][tile_points][lda] FP32 gradients
+// LDS for the place of each group of `gran` functions (nblk * 32 / gran shorts)
+__host__ __device__ constexpr size_t gpos_bytes(int nblk, int gran) {
+    return ((size_t)nblk * (64 / gran) + 15) / 16 * 16;
+}
+
+// LDS image of a pass's rows for basis_eval_staged_kernel, of width w: mixed
+// [rows][w/8][3][8] BF16 parts of phi, then [3][rows][w] FP32 gradients; FP64
+// [4][rows][w] (phi, then the gradient)
 extern __shared__ __align__(16) unsigned char basis_tile[];
 
 struct Comp {
@@ -277,13 +286,12 @@ __global__ __launch_bounds__(256) void basis_eval_kernel(EvalArgs a) {
     }
 }
 
-// Split output through LDS (see the file comment).  Grid: rows / tile_points
-// workgroups; tile_points divides 128 (the smallest row tile of the
-// contraction kernels) and the LDS image is
-// tile_points * lda * 18 bytes (then, compressed, 4 nblk shorts).
+// Rows staged through LDS (see the file comment).  Grid: rows / tile_points
+// workgroups of 32 rows, written in passes of as many rows as the LDS image
+// (36 KiB, or one dense row) holds.
 //
-// Compressed output (a.toff non-null): the workgroup's rows belong to row
-// tile t of a.tile_rows rows, which keeps only its live 8-function groups.
+// The workgroup's rows belong to row tile t of a.tile_rows rows, which keeps
+// only its live groups of 8 functions (mixed) or 4 (FP64), in list order.
 // A shell is evaluated only if its first group is live: a shell with a
 // function in a group that is not lies beyond its radius for every point
 // of the tile (the groups of every shell within reach of the tile are
@@ -291,10 +299,9 @@ __global__ __launch_bounds__(256) void basis_eval_kernel(EvalArgs a) {
 // groups, adjacent in the list, so its functions stay contiguous in the
 // compressed columns.
 //
-// F64: FP64 values and gradients of dense rows (the FP64 contraction's
-// input), 32 bytes per function in the image; no compression.  Staging
-// keeps the global stores contiguous whatever the function order: a
-// wavefront's shells (ordered by l) need not own adjacent columns.
+// F64: FP64 values and gradients, 32 bytes per function in the image; dense
+// rows of one per workgroup, written whole, took 13.7 ms where this takes
+// 5.8 ms for 857,375 points of the 60-atom cage.
 // (four wavefronts per SIMD for l <= 3: the LDS images of four workgroups
 // fit a CU, and the registers are held to 128)
 template <int LMAX, bool F64 = false, bool CAND = false>
@@ -303,26 +310,25 @@ void basis_eval_staged_kernel(EvalArgs a) {
     constexpr int kFunBytes = F64 ? 32 : 2 * kAParts + 12;  // image bytes per function
     const int tid = threadIdx.x, tp = a.tile_points;
     const size_t row0 = (size_t)blockIdx.x * tp;
-    int wt = a.lda;  // functions per row of this tile's output
-    short *gpos = nullptr;  // place of each 8-function group in the compressed rows
-    __bf16 *phi_dst = a.phis + row0 * kAParts * (size_t)a.lda;
-    float *grad_dst = a.grad32 + row0 * (size_t)a.lda;
-    size_t grad_plane = (size_t)a.gplane;
-    if (!F64 && a.toff) {
-        const int t = (int)(row0 / a.tile_rows);
-        const int kg = a.kcount[t];
-        if (kg == 0) return;  // nothing of this tile is read (uniform per workgroup)
-        wt = 8 * kg;
-        gpos = (short *)(basis_tile + a.lds_image);
-        for (int i = tid; i < 4 * a.nblk; i += 256) gpos[i] = -1;
-        __syncthreads();
-        for (int i = tid; i < kg; i += 256) gpos[a.klist[(size_t)t * a.nblk * 4 + i] >> 12] = (short)i;
-        const size_t base = (size_t)a.toff[t] * a.tile_rows * 8;
-        const size_t rin = row0 - (size_t)t * a.tile_rows;
-        phi_dst = a.phis + base * kAParts + rin * kAParts * (size_t)wt;
-        grad_dst = a.grad32 + base * 3 + rin * (size_t)wt;
-        grad_plane = (size_t)a.tile_rows * wt;
-    }
+    constexpr int kGran = F64 ? 4 : 8, kPer = 32 / kGran, kShift = list_shift(kGran);
+    // the tile's rows in the output, and the place of each group in them
+    const int t = (int)(row0 / a.tile_rows);
+    const int kg = a.kcount[t];
+    if (kg == 0) return;  // nothing of this tile is read (uniform per workgroup)
+    const int wt = kGran * kg;  // functions per row
+    short *gpos = (short *)(basis_tile + a.lds_image);
+    for (int i = tid; i < kPer * a.nblk; i += 256) gpos[i] = -1;
+    __syncthreads();
+    for (int i = tid; i < kg; i += 256)
+        gpos[a.klist[(size_t)t * a.nblk * kPer + i] >> kShift] = (short)i;
+    const size_t base = (size_t)a.toff[t] * a.tile_rows * kGran;
+    const size_t rin = row0 - (size_t)t * a.tile_rows;
+    typedef typename std::conditional<F64, double, __bf16>::type Value;
+    typedef typename std::conditional<F64, double, float>::type Grad;
+    constexpr int kParts = F64 ? 1 : kAParts;  // Values per function
+    Value *phi_dst = (F64 ? (Value *)a.phi64 : (Value *)a.phis) + base * kParts + rin * kParts * (size_t)wt;
+    Grad *grad_dst = (F64 ? (Grad *)a.grad64 : (Grad *)a.grad32) + base * 3 + rin * (size_t)wt;
+    const size_t grad_plane = (size_t)a.tile_rows * wt;
     // Candidate shells (CAND): the shells that can reach a row of this workgroup,
     // listed in shell order, kCandChunk at a time.  A shell is dropped only
     // if its group is not live (compressed output) or if it is beyond its
@@ -330,7 +336,7 @@ void basis_eval_staged_kernel(EvalArgs a) {
     // the per-row radius test below still decides each (row, shell) pair,
     // so the output is the same, but the lanes of a wavefront no longer
     // idle beside pairs that every row screens out.
-    short *cand = (short *)(basis_tile + a.lds_image + ((size_t)a.nblk * 8 + 15) / 16 * 16);
+    short *cand = (short *)(basis_tile + a.lds_image + gpos_bytes(a.nblk, kGran));
     double *sphere = (double *)(cand + kCandChunk);  // centre x, y, z and radius
     int *wcnt = (int *)(sphere + 4);                 // kept shells per wavefront
     if (CAND) {
@@ -375,7 +381,7 @@ void basis_eval_staged_kernel(EvalArgs a) {
             bool keep = false;
             if (i0 + tid < kCandChunk && si < a.nshell && sphere[3] >= 0.0) {
                 const DevShell sh = a.shells[si];
-                keep = !gpos || gpos[sh.fout >> 3] >= 0;
+                keep = gpos[sh.fout / kGran] >= 0;
                 if (keep) {
                     const double *R = a.coords + 3 * sh.atom;
                     const double dx = sphere[0] - R[0], dy = sphere[1] - R[1], dz = sphere[2] - R[2];
@@ -396,12 +402,9 @@ void basis_eval_staged_kernel(EvalArgs a) {
         return n;
     };
     // one chunk holds every shell of most bases: then the list is built once
-    // for all passes.  The FP64 rows (one or two per workgroup) keep the
-    // plain walk over every shell: for so few rows the list costs more than
-    // the idle lanes it saves (8.2 ms against 9.7 ms on the 60-atom cage)
-    constexpr bool kCand = CAND && !F64;
-    const bool one_chunk = !kCand || a.nshell <= kCandChunk;
-    const int ncand1 = kCand && one_chunk ? candidates(0) : 0;
+    // for all passes
+    const bool one_chunk = !CAND || a.nshell <= kCandChunk;
+    const int ncand1 = CAND && one_chunk ? candidates(0) : 0;
     // rows per pass: as many as the LDS image holds at this width (at least
     // one: the image holds a dense row)
     const int rpp = max(1, min(tp, (int)(a.lds_image / ((size_t)wt * kFunBytes))));
@@ -424,11 +427,9 @@ void basis_eval_staged_kernel(EvalArgs a) {
             const size_t row = row0 + r0 + lp;
             if (row >= (size_t)a.npts) return;  // padding rows stay zero
             DevShell sh = a.shells[si];
-            if (gpos) {
-                const int cg = gpos[sh.fout >> 3];
-                if (cg < 0) return;  // zero over the whole tile
-                sh.fout = cg * 8 + (sh.fout & 7);
-            }
+            const int cg = gpos[sh.fout / kGran];
+            if (cg < 0) return;  // zero over the whole tile
+            sh.fout = cg * kGran + sh.fout % kGran;
             const double *r = a.pts + 3 * row;
             const double *R = a.coords + 3 * sh.atom;
             double rr[3] = {r[0] - R[0], r[1] - R[1], r[2] - R[2]};
@@ -445,7 +446,7 @@ void basis_eval_staged_kernel(EvalArgs a) {
                 else dispatch_l<M, false, false, LMAX>(b, lp, sh, rr, g, h);
             }
         };
-        if constexpr (kCand) {
+        if constexpr (CAND) {
             for (int s0 = 0; s0 < a.nshell; s0 += kCandChunk) {
                 const int ncand = one_chunk ? ncand1 : candidates(s0);
                 for (int it = tid; it < nr * ncand; it += 256) pair(it % nr, s0 + cand[it / nr]);
@@ -456,26 +457,16 @@ void basis_eval_staged_kernel(EvalArgs a) {
         }
         __syncthreads();
         // this pass's rows are contiguous in both outputs
-        if (F64) {
-            const size_t n16 = (size_t)nr * wt / 2;  // 16-byte units per plane
-            for (int d = 0; d < 4; d++) {
-                const uint4 *src = (const uint4 *)(basis_tile + (size_t)d * nr * wt * 8);
-                double *base = d == 0 ? a.phi64 : a.grad64 + (size_t)(d - 1) * a.gplane;
-                uint4 *dst = (uint4 *)(base + (row0 + r0) * (size_t)wt);
-                for (size_t i = tid; i < n16; i += 256) dst[i] = src[i];
-            }
-            __syncthreads();
-            continue;
-        }
         {
             const uint4 *src = (const uint4 *)basis_tile;
-            uint4 *dst = (uint4 *)(phi_dst + (size_t)r0 * kAParts * wt);
+            uint4 *dst = (uint4 *)(phi_dst + (size_t)r0 * kParts * wt);
             for (size_t i = tid; i < phi_bytes / 16; i += 256) dst[i] = src[i];
         }
         for (int d = 0; d < 3; d++) {
-            const uint4 *src = (const uint4 *)(basis_tile + phi_bytes + (size_t)d * nr * wt * 4);
+            const size_t plane = grad_bytes / 3;
+            const uint4 *src = (const uint4 *)(basis_tile + phi_bytes + d * plane);
             uint4 *dst = (uint4 *)(grad_dst + d * grad_plane + (size_t)r0 * wt);
-            for (size_t i = tid; i < (size_t)nr * wt / 4; i += 256) dst[i] = src[i];
+            for (size_t i = tid; i < plane / 16; i += 256) dst[i] = src[i];
         }
         __syncthreads();  // the image is read out before the next pass clears it
     }
@@ -489,88 +480,51 @@ hipError_t upload_basis_tables(const double *sph, int nsph, hipStream_t s) {
 
 hipError_t launch_basis_eval(const EvalArgs &a, int mode, hipStream_t s) {
     const long long total = (long long)a.rows * a.nshell;
-    const unsigned nblk = (unsigned)((total + 255) / 256);
     if (total <= 0) return hipSuccess;
-    if (mode == 0 && (size_t)a.lda * 32 <= 150 * 1024 && a.lmax >= 0 && a.lmax <= kDevMaxL) {
-        // FP64 rows staged through LDS: the largest tile of 1, 2, 4 or 8 rows
-        // within 72 KiB (or one row up to 150 KiB)
-        EvalArgs b = a;
-        const size_t row_bytes = (size_t)a.lda * 32;
-        int tp = 8;
-        while (tp > 1 && tp * row_bytes > 72 * 1024) tp >>= 1;
-        if (a.rows % tp) return hipErrorInvalidValue;
-        b.tile_points = tp;
-        b.lds_image = tp * row_bytes;
-        b.toff = nullptr;
-        b.nblk = 0;  // no block positions: the candidate list follows the image
-        const size_t lds = b.lds_image;
-        auto launch = [&](auto kernel) -> hipError_t {
-            hipError_t e = hipFuncSetAttribute((const void *)kernel,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)std::max<size_t>(lds, 72 * 1024));
-            if (e != hipSuccess) return e;
-            hipLaunchKernelGGL(kernel, dim3((unsigned)(a.rows / tp)), dim3(256), lds, s, b);
-            return hipGetLastError();
-        };
-        if (a.lmax <= 1) return launch(basis_eval_staged_kernel<1, true>);
-        if (a.lmax == 2) return launch(basis_eval_staged_kernel<2, true>);
-        if (a.lmax == 3) return launch(basis_eval_staged_kernel<3, true>);
-        return launch(basis_eval_staged_kernel<5, true>);
+    if (a.lmax < 0 || a.lmax > kDevMaxL) return hipErrorInvalidValue;
+    const bool f64 = mode == 0;
+    if (f64 && !a.toff) {
+        // dense rows of a basis too wide for the LDS image
+        hipLaunchKernelGGL(basis_eval_kernel<0>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
+                           s, a);
+        return hipGetLastError();
     }
-    if (mode == 0)
-        hipLaunchKernelGGL(basis_eval_kernel<0>, dim3(nblk), dim3(256), 0, s, a);
-    else {
-        // dense: the largest tile of 1, 2, 4 or 8 rows whose LDS image fits in
-        // 72 KiB (two workgroups per CU).  Compressed: 32 rows per workgroup
-        // staged in passes through an image of 36 KiB or one dense row,
-        // whichever is larger (four workgroups per CU at nbf <= 2048); 32
-        // rows rather than 8 spread the workgroup's fixed work (block
-        // positions, candidate list) over more rows: 6-8% on the cage's and
-        // the tetracene scan's basis evaluation, 64 rows no better
-        EvalArgs b = a;
-        const size_t row_bytes = (size_t)a.lda * (2 * kAParts + 12);
-        int tp = a.toff ? 32 : 8;
-        size_t image;
-        if (a.toff) {
-            image = std::max<size_t>(36 * 1024, row_bytes);
-        } else {
-            while (tp > 1 && tp * row_bytes > 72 * 1024) tp >>= 1;
-            image = tp * row_bytes;
-        }
-        if (row_bytes > 150 * 1024) return hipErrorInvalidValue;
-        b.tile_points = tp;
-        b.lds_image = image;
-        // the image, the group positions (16-byte aligned) and, for bases of
-        // kCandMinShells shells or more, the candidate list
-        const bool cand = a.nshell >= kCandMinShells;
-        const size_t lds = image + ((size_t)a.nblk * 8 + 15) / 16 * 16 + (cand ? kCandBytes : 0);
-        // (the candidate list's bounding sphere takes one row per lane of a wavefront)
-        if (a.rows % tp || tp > 64 || a.lmax < 0 || a.lmax > kDevMaxL) return hipErrorInvalidValue;
-        if (a.toff && (a.tile_rows % tp || a.rows % a.tile_rows || a.nblk * 32 != a.lda))
-            return hipErrorInvalidValue;
-        auto launch = [&](auto kernel) -> hipError_t {
-            hipError_t e = hipFuncSetAttribute((const void *)kernel,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)std::max<size_t>(lds, 72 * 1024));
-            if (e != hipSuccess) return e;
-            hipLaunchKernelGGL(kernel, dim3((unsigned)(a.rows / tp)), dim3(256), lds, s, b);
-            return hipGetLastError();
-        };
-        hipError_t e;
-        if (cand) {
-            if (a.lmax <= 1) e = launch(basis_eval_staged_kernel<1, false, true>);
-            else if (a.lmax == 2) e = launch(basis_eval_staged_kernel<2, false, true>);
-            else if (a.lmax == 3) e = launch(basis_eval_staged_kernel<3, false, true>);
-            else e = launch(basis_eval_staged_kernel<5, false, true>);
-        } else {
-            if (a.lmax <= 1) e = launch(basis_eval_staged_kernel<1>);
-            else if (a.lmax == 2) e = launch(basis_eval_staged_kernel<2>);
-            else if (a.lmax == 3) e = launch(basis_eval_staged_kernel<3>);
-            else e = launch(basis_eval_staged_kernel<5>);
-        }
+    // 32 rows per workgroup, staged in passes through an image of 36 KiB or
+    // one dense row, whichever is larger (four workgroups per CU at nbf <=
+    // 2048); 32 rows rather than 8 spread the workgroup's fixed work (group
+    // positions, candidate list) over more rows: 6-8% on the cage's and the
+    // tetracene scan's mixed basis evaluation, 64 rows no better
+    EvalArgs b = a;
+    const size_t row_bytes = (size_t)a.lda * (f64 ? 32 : 2 * kAParts + 12);
+    if (row_bytes > kMaxRowBytes || !a.toff) return hipErrorInvalidValue;
+    b.tile_points = 32;
+    b.lds_image = std::max<size_t>(36 * 1024, row_bytes);
+    // the image, the group positions (16-byte aligned) and, for bases of
+    // kCandMinShells shells or more, the candidate list
+    const bool cand = a.nshell >= kCandMinShells;
+    const size_t lds = b.lds_image + gpos_bytes(a.nblk, f64 ? 4 : 8) + (cand ? kCandBytes : 0);
+    // (the candidate list's bounding sphere takes one row per lane of a wavefront)
+    if (a.tile_rows % b.tile_points || a.rows % a.tile_rows || a.nblk * 32 != a.lda)
+        return hipErrorInvalidValue;
+    auto launch = [&](auto kernel) -> hipError_t {
+        hipError_t e = hipFuncSetAttribute((const void *)kernel,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           (int)std::max<size_t>(lds, 72 * 1024));
         if (e != hipSuccess) return e;
-    }
-    return hipGetLastError();
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(a.rows / b.tile_points)), dim3(256), lds, s, b);
+        return hipGetLastError();
+    };
+    auto pick = [&](auto f, auto c) -> hipError_t {
+        constexpr bool F = decltype(f)::value, C = decltype(c)::value;
+        if (a.lmax <= 1) return launch(basis_eval_staged_kernel<1, F, C>);
+        if (a.lmax == 2) return launch(basis_eval_staged_kernel<2, F, C>);
+        if (a.lmax == 3) return launch(basis_eval_staged_kernel<3, F, C>);
+        return launch(basis_eval_staged_kernel<5, F, C>);
+    };
+    using T = std::true_type;
+    using N = std::false_type;
+    if (f64) return cand ? pick(T{}, T{}) : pick(T{}, N{});
+    return cand ? pick(N{}, T{}) : pick(N{}, N{});
 }
 
 }  // namespace gimic

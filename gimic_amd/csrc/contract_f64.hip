@@ -83,15 +83,20 @@ __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
     const int ng = a.lda / 4;  // granules per row; index ng: the zero blocks
     const v2d *B = (const v2d *)(a.b64 + (size_t)set * f64_set_elems(a.lda));
     const size_t rowst = (size_t)(ng + 1) * kUnits;
-    const size_t row = (size_t)rtile * a.tile_rows + (blockIdx.x >> 3) % parts * kRows + wave * 16 + c;
-    const double *A = a.a64 + row * a.lda;
-    const double *G = a.g64 + row * a.lda;
-    const size_t gplane = (size_t)a.gplane;
+    const int rin = (blockIdx.x >> 3) % parts * kRows + wave * 16 + c;
+    const size_t row = (size_t)rtile * a.tile_rows + rin;
+    // the point's values and gradients: dense, or compressed to the tile's granules
+    const bool cmp = a.toff != nullptr;
+    const size_t w = cmp ? (size_t)a.kcount[rtile] * 4 : (size_t)a.lda;
+    const size_t base = cmp ? (size_t)a.toff[rtile] * a.tile_rows * 4 : (size_t)rtile * a.tile_rows * w;
+    const double *A = a.a64 + base + rin * w;
+    const double *G = a.g64 + (cmp ? 3 * base : base) + rin * w;
+    const size_t gplane = cmp ? (size_t)a.tile_rows * w : (size_t)a.gplane;
     const bool valid = row < (size_t)a.npts;
     const double r[3] = {valid ? a.pts[3 * row] : 0.0, valid ? a.pts[3 * row + 1] : 0.0,
                          valid ? a.pts[3 * row + 2] : 0.0};
     // a padding entry (-1) reads the row's first granule against zero blocks
-    auto acol = [&](int v) { return v < 0 ? 0 : (v >> 13) * 4; };
+    auto acol = [&](int v) { return v < 0 ? 0 : (cmp ? v & 8191 : v >> 13) * 4; };
 
     // Element pair sp of matrix m for lane l is at (2 m + sp) * 64 +
     // (l ^ (l >> 3 & 1) ^ 2 sp): eight consecutive lanes of a read (c fixed in

@@ -28,6 +28,9 @@ constexpr int kNT = 16;
 // K padding granularity (FP64 K-step 16, BF16 K-step 32)
 constexpr int kKPad = 32;
 
+// bits of a screening list entry that hold its place (TileArgs)
+__host__ __device__ constexpr int list_shift(int gran) { return gran == 8 ? 12 : 13; }
+
 struct DevShell {
     int atom;
     int l;
@@ -98,15 +101,16 @@ struct EvalArgs {
     int tile_points;     // points per workgroup of the LDS-staged kernel (set by the launcher)
     size_t lds_image;    // bytes of its LDS image (set by the launcher)
     int lmax;            // largest shell l of the basis
-    // Compressed split output (staged kernel, toff non-null): a row tile of
-    // tile_rows rows keeps only its kcount[t] live 8-function groups
-    // (klist[t * 4 nblk ...], global group << 12 | place k in the row); its
-    // rows start at element toff[t] * tile_rows * 8 kAParts of phis
-    // ([row][k][kAParts][8]) and toff[t] * tile_rows * 24 of grad32
-    // ([3][tile_rows][8 k])
+    // Compressed rows (toff non-null): a row tile of tile_rows rows keeps only
+    // its kcount[t] live groups of gran = 8 (mixed) or 4 (FP64) functions
+    // (TileArgs); its rows start at function toff[t] * tile_rows * gran: split
+    // values [row][place][kAParts][8] or FP64 values [row][gran place], and
+    // gradients [3][tile_rows][gran kcount] from three times that.  Only FP64
+    // rows of more than kMaxRowBytes are dense.
     const int *kcount, *klist, *toff;
     int nblk, tile_rows;
 };
+constexpr size_t kMaxRowBytes = 150 * 1024;
 hipError_t launch_basis_eval(const EvalArgs &a, int mode, hipStream_t s);
 hipError_t upload_basis_tables(const double *sph, int nsph, hipStream_t s);
 
@@ -129,7 +133,7 @@ struct ContractArgs {
     // split s of a tile takes N-tiles [s * count / nsplit, (s+1) * count / nsplit)
     int nblk, tile_rows;  // tile_rows: FP64 kernel only
     const int *kcount, *klist;
-    // compressed operands (pre-split kernels; see EvalArgs): null for dense
+    // compressed operands (see EvalArgs): null for dense rows
     const int *toff;
 };
 // FP64 right operand in HBM: one pair block per (density set, 4-function
@@ -278,7 +282,7 @@ struct TileArgs {
     // multiple of 4
     int *bcount, *k8count, *kcount, *klist;
 };
-constexpr int list_shift(int gran) { return gran == 8 ? 12 : 13; }
+
 hipError_t launch_block_lists(const TileArgs &a, hipStream_t s);
 // toff[t] = sum of cnt[0 .. t-1] for t = 0 .. ntiles (one workgroup)
 hipError_t launch_tile_offsets(const int *cnt, int ntiles, int *toff, hipStream_t s);
