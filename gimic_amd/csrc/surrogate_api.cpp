@@ -11,38 +11,17 @@
 #include <vector>
 
 #include "../../include/gimic_hip.h"
+#include "surrogate.h"
 
 namespace gimic {
-hipError_t mlp_gemm(const __bf16 *A, long long sam, long long sak, const __bf16 *B, long long sbk,
-                    long long sbn, float *C, long long ldc, int M, int N, int K, int ksplit,
-                    hipStream_t s);
-hipError_t mlp_features(const double *r, long long npts, const float *Bfreq, int F,
-                        const float *cs, __bf16 *X, int K0, hipStream_t s);
-hipError_t mlp_bias_silu(float *Z, const float *b, __bf16 *H, long long total, int N,
-                         hipStream_t s);
-hipError_t mlp_loss(const float *Z, const float *b, const double *target, const float *out_scale,
-                    float eps2, long long npts, int NO, float *dY, __bf16 *dYb, float *loss,
-                    hipStream_t s);
-hipError_t mlp_dsilu(const float *dH, const float *Z, float *dZ, __bf16 *dZb, long long total,
-                     hipStream_t s);
-hipError_t mlp_colsum(const float *dZ, long long npts, int N, float *db, hipStream_t s);
-hipError_t mlp_adam(float *p, const float *grad, float *m, float *v, long long n, float lr,
-                    float b1, float b2, float eps, float bc1, float bc2, __bf16 *pb,
-                    hipStream_t s);
-hipError_t mlp_cast(const float *p, __bf16 *pb, long long n, hipStream_t s);
-hipError_t mlp_output(const float *Z, const float *b, const float *out_scale, long long npts,
-                      int NO, double *J, hipStream_t s);
-hipError_t mlp_infer(const double *r, long long npts, const float *Bfreq, int F, const float *cs,
-                     const __bf16 *const *W, const float *const *bias, const float *out_scale,
-                     double *J, hipStream_t s);
 std::string &error_slot();
-}  // namespace gimic
+}
 
 using namespace gimic;
 
 namespace {
 
-constexpr int kF = 64, kK0 = 160, kH = 128, kD = 4, kNO = 16;
+constexpr int kF = kMlpF, kK0 = kMlpK0, kH = kMlpH, kD = kMlpD, kNO = kMlpNO;
 
 struct MlpError : std::runtime_error {
     int code;
@@ -80,8 +59,8 @@ struct gimic_mlp {
     long long np = 0;                 // parameter count
     long long woff[kD + 1], boff[kD + 1];
     int kin[kD + 1], nout[kD + 1];
-    Buf params, params_b, grad, adam_m, adam_v, freq, cs, oscale, ptrs;
-    Buf X[kD + 1], Z[kD + 1], dH, dZ, dZb, dY, dYb, loss;
+    Buf params, params_b, params_t, grad, adam_m, adam_v, freq, cs, oscale, ptrs;
+    Buf X[kD + 1], dZ[kD], dY, part, bpart, loss;
     long long cap = 0;  // batch capacity of the work buffers
     long long step = 0;
     ~gimic_mlp() {
@@ -115,63 +94,53 @@ int guard(F &&f) {
 
 void reserve(gimic_mlp *n, long long P) {
     if (P <= n->cap) return;
-    for (int l = 0; l <= kD; l++) {
-        n->X[l].need((size_t)P * n->kin[l] * 2);
-        n->Z[l].need((size_t)P * n->nout[l] * 4);
-    }
-    n->dH.need((size_t)P * kK0 * 4);
-    n->dZ.need((size_t)P * kH * 4);
-    n->dZb.need((size_t)P * kH * 2);
-    n->dY.need((size_t)P * kNO * 4);
-    n->dYb.need((size_t)P * kNO * 2);
+    const size_t rows = (size_t)(P + 63) / 64 * 64;  // whole tiles
+    for (int l = 0; l <= kD; l++) n->X[l].need(rows * n->kin[l] * 2);
+    for (int l = 0; l < kD; l++) n->dZ[l].need(rows * kH * 2);
+    n->dY.need(rows * kNO * 2);
+    n->part.need((size_t)kMlpMaxRanges * kMlpParams * 4);
+    n->bpart.need((size_t)mlp_tile_groups(1ll << 30) * kMlpBiasPart * 4);
     n->cap = P;
 }
 
-// forward pass of a batch (training form: activations kept)
-void forward(gimic_mlp *n, long long P, const double *d_r, hipStream_t s) {
-    float *prm = n->params.as<float>();
-    __bf16 *pb = n->params_b.as<__bf16>();
-    chk(mlp_features(d_r, P, n->freq.as<float>(), kF, n->cs.as<float>(), n->X[0].as<__bf16>(), kK0,
-                     s), "features");
-    for (int l = 0; l <= kD; l++) {
-        const int K = n->kin[l], N = n->nout[l];
-        chk(mlp_gemm(n->X[l].as<__bf16>(), K, 1, pb + n->woff[l], 1, K, n->Z[l].as<float>(), N,
-                     (int)P, N, K, 1, s), "gemm fwd");
-        if (l < kD)
-            chk(mlp_bias_silu(n->Z[l].as<float>(), prm + n->boff[l], n->X[l + 1].as<__bf16>(),
-                              P * N, N, s), "bias_silu");
-    }
+MlpTileArgs tile_args(gimic_mlp *n, long long P, const double *d_r) {
+    MlpTileArgs a{};
+    a.r = d_r;
+    a.npts = P;
+    a.freq = n->freq.as<float>();
+    a.cs = n->cs.as<float>();
+    a.oscale = n->oscale.as<float>();
+    a.prm = n->params.as<float>();
+    a.W = n->params_b.as<__bf16>();
+    a.WT = n->params_t.as<__bf16>();
+    return a;
 }
 
-void backward(gimic_mlp *n, long long P, const double *d_target, float eps2, hipStream_t s) {
-    float *prm = n->params.as<float>();
-    __bf16 *pb = n->params_b.as<__bf16>();
-    float *gr = n->grad.as<float>();
-    chk(hipMemsetAsync(gr, 0, (size_t)n->np * 4, s), "memset grad");
-    chk(hipMemsetAsync(n->loss.p, 0, 4, s), "memset loss");
-    chk(mlp_loss(n->Z[kD].as<float>(), prm + n->boff[kD], d_target, n->oscale.as<float>(), eps2, P,
-                 kNO, n->dY.as<float>(), n->dYb.as<__bf16>(), n->loss.as<float>(), s), "loss");
-    const int ks = (int)std::max<long long>(1, std::min<long long>(64, P / 1024));
-    // output layer
-    {
-        const int l = kD, K = n->kin[l], N = n->nout[l];
-        chk(mlp_gemm(n->dYb.as<__bf16>(), 1, N, n->X[l].as<__bf16>(), K, 1, gr + n->woff[l], K, N,
-                     K, (int)P, ks, s), "gemm dW out");
-        chk(mlp_colsum(n->dY.as<float>(), P, N, gr + n->boff[l], s), "colsum");
-        chk(mlp_gemm(n->dYb.as<__bf16>(), N, 1, pb + n->woff[l], K, 1, n->dH.as<float>(), K,
-                     (int)P, K, N, 1, s), "gemm dX out");
-    }
-    for (int l = kD - 1; l >= 0; l--) {
-        const int K = n->kin[l], N = n->nout[l];
-        chk(mlp_dsilu(n->dH.as<float>(), n->Z[l].as<float>(), n->dZ.as<float>(),
-                      n->dZb.as<__bf16>(), P * N, s), "dsilu");
-        chk(mlp_gemm(n->dZb.as<__bf16>(), 1, N, n->X[l].as<__bf16>(), K, 1, gr + n->woff[l], K, N,
-                     K, (int)P, ks, s), "gemm dW");
-        chk(mlp_colsum(n->dZ.as<float>(), P, N, gr + n->boff[l], s), "colsum");
-        if (l > 0)
-            chk(mlp_gemm(n->dZb.as<__bf16>(), N, 1, pb + n->woff[l], K, 1, n->dH.as<float>(), K,
-                         (int)P, K, N, 1, s), "gemm dX");
-    }
+// one batch: forward, backward, and the gradient (adam == 0) or an Adam step
+void batch(gimic_mlp *n, long long P, const double *d_r, const double *d_target, float eps2,
+           MlpAdamArgs o, hipStream_t s) {
+    reserve(n, P);
+    MlpTileArgs a = tile_args(n, P, d_r);
+    a.target = d_target;
+    a.eps2 = eps2;
+    for (int l = 0; l <= kD; l++) a.X[l] = n->X[l].as<__bf16>();
+    for (int l = 0; l < kD; l++) a.dZ[l] = n->dZ[l].as<__bf16>();
+    a.dY = n->dY.as<__bf16>();
+    a.bpart = n->bpart.as<float>();
+    chk(mlp_tiles(a, true, s), "tiles");
+    chk(mlp_dw(a, n->part.as<float>(), s), "dW");
+    o.part = n->part.as<float>();
+    o.bpart = n->bpart.as<float>();
+    o.ranges = mlp_ranges(P);
+    o.groups = mlp_tile_groups(P);
+    o.grad = n->grad.as<float>();
+    o.loss = n->loss.as<float>();
+    o.prm = n->params.as<float>();
+    o.m = n->adam_m.as<float>();
+    o.v = n->adam_v.as<float>();
+    o.W = n->params_b.as<__bf16>();
+    o.WT = n->params_t.as<__bf16>();
+    chk(mlp_adam(o, s), "adam");
 }
 
 }  // namespace
@@ -213,6 +182,7 @@ int gimic_mlp_create(gimic_mlp **out, double sigma, const double *center_scale,
             hipStream_t s = work_stream(n);
             n->params.need(off * 4);
             n->params_b.need(off * 2);
+            n->params_t.need((size_t)kMlpTransposed * 2);
             n->grad.need(off * 4);
             n->adam_m.need(off * 4);
             n->adam_v.need(off * 4);
@@ -226,7 +196,8 @@ int gimic_mlp_create(gimic_mlp **out, double sigma, const double *center_scale,
             chk(hipMemcpyAsync(n->freq.p, fr.data(), fr.size() * 4, hipMemcpyHostToDevice, s), "copy");
             chk(hipMemcpyAsync(n->cs.p, cs, 16, hipMemcpyHostToDevice, s), "copy");
             chk(hipMemcpyAsync(n->oscale.p, os, 36, hipMemcpyHostToDevice, s), "copy");
-            chk(mlp_cast(n->params.as<float>(), n->params_b.as<__bf16>(), off, s), "cast");
+            chk(mlp_cast(n->params.as<float>(), n->params_b.as<__bf16>(), n->params_t.as<__bf16>(), s),
+                "cast");
             // device table of layer pointers for the fused inference kernel
             std::vector<void *> tab(2 * (kD + 1));
             for (int l = 0; l <= kD; l++) {
@@ -271,7 +242,8 @@ int gimic_mlp_params(gimic_mlp *n, float *host, int set) {
         hipStream_t s = work_stream(n);
         if (set) {
             chk(hipMemcpyAsync(n->params.p, host, n->np * 4, hipMemcpyHostToDevice, s), "copy");
-            chk(mlp_cast(n->params.as<float>(), n->params_b.as<__bf16>(), n->np, s), "cast");
+            chk(mlp_cast(n->params.as<float>(), n->params_b.as<__bf16>(), n->params_t.as<__bf16>(), s),
+                "cast");
         } else {
             chk(hipMemcpyAsync(host, n->params.p, n->np * 4, hipMemcpyDeviceToHost, s), "copy");
         }
@@ -284,9 +256,7 @@ int gimic_mlp_loss_grad(gimic_mlp *n, long long npts, const double *d_r, const d
     return guard([&] {
         if (!n || npts <= 0 || !d_r || !d_target) throw MlpError(GIMIC_EINVAL, "bad argument");
         hipStream_t s = work_stream(n);
-        reserve(n, npts);
-        forward(n, npts, d_r, s);
-        backward(n, npts, d_target, (float)(eps * eps), s);
+        batch(n, npts, d_r, d_target, (float)(eps * eps), MlpAdamArgs{}, s);
         float l = 0.f;
         chk(hipMemcpyAsync(&l, n->loss.p, 4, hipMemcpyDeviceToHost, s), "copy");
         if (host_grad)
@@ -301,15 +271,18 @@ int gimic_mlp_train_step(gimic_mlp *n, long long npts, const double *d_r, const 
     return guard([&] {
         if (!n || npts <= 0 || !d_r || !d_target) throw MlpError(GIMIC_EINVAL, "bad argument");
         hipStream_t s = work_stream(n);
-        reserve(n, npts);
-        forward(n, npts, d_r, s);
-        backward(n, npts, d_target, (float)(eps * eps), s);
-        n->step++;
         const float b1 = 0.9f, b2 = 0.999f;
-        const float bc1 = 1.f - std::pow(b1, (float)n->step), bc2 = 1.f - std::pow(b2, (float)n->step);
-        chk(mlp_adam(n->params.as<float>(), n->grad.as<float>(), n->adam_m.as<float>(),
-                     n->adam_v.as<float>(), n->np, (float)lr, b1, b2, 1e-8f, bc1, bc2,
-                     n->params_b.as<__bf16>(), s), "adam");
+        const float t = (float)(n->step + 1);
+        MlpAdamArgs o{};
+        o.adam = 1;
+        o.lr = (float)lr;
+        o.b1 = b1;
+        o.b2 = b2;
+        o.eps = 1e-8f;
+        o.bc1 = 1.f - std::pow(b1, t);
+        o.bc2 = 1.f - std::pow(b2, t);
+        batch(n, npts, d_r, d_target, (float)(eps * eps), o, s);
+        n->step++;
         if (loss) {
             float l = 0.f;
             chk(hipMemcpyAsync(&l, n->loss.p, 4, hipMemcpyDeviceToHost, s), "copy");
@@ -334,10 +307,9 @@ int gimic_mlp_predict_unfused(gimic_mlp *n, long long npts, const double *d_r, d
     return guard([&] {
         if (!n || npts <= 0 || !d_r || !d_J) throw MlpError(GIMIC_EINVAL, "bad argument");
         hipStream_t s = work_stream(n);
-        reserve(n, npts);
-        forward(n, npts, d_r, s);
-        chk(mlp_output(n->Z[kD].as<float>(), n->params.as<float>() + n->boff[kD],
-                       n->oscale.as<float>(), npts, kNO, d_J, s), "output");
+        MlpTileArgs a = tile_args(n, npts, d_r);
+        a.J = d_J;
+        chk(mlp_tiles(a, false, s), "tiles");
         chk(hipStreamSynchronize(s), "sync");
     });
 }
