@@ -42,8 +42,7 @@ hipError_t mlp_tiles(const MlpTileArgs &a, bool train, hipStream_t s);
 hipError_t mlp_dw(const MlpTileArgs &a, float *part, hipStream_t s);
 hipError_t mlp_adam(const MlpAdamArgs &a, hipStream_t s);
 hipError_t mlp_cast(const float *p, __bf16 *W, __bf16 *WT, hipStream_t s);
-hipError_t mlp_infer(const double *r, long long npts, const float *Bfreq, int F, const float *cs,
-                     const __bf16 *const *W, const float *const *bias, const float *out_scale,
-                     double *J, hipStream_t s);
+hipError_t mlp_infer(const double *r, long long npts, const float *freq, const float *cs,
+                     const __bf16 *W, const float *prm, const float *oscale, double *J, hipStream_t s);
 
 }  // namespace gimic

@@ -14,7 +14,7 @@
 // (direction and log magnitude fitted separately, so every point weighs the
 // same whatever the size of its current; the prediction y e^{y_9} then has
 // relative error ~ |y - u| + |y_9 - log n|).
-// Inference: one fused kernel per 64-point tile, activations in LDS.
+// Inference: one fused kernel, activations in registers, weights in LDS.
 //
 // Training (mlp_tile_kernel, mlp_dw_kernel, mlp_adam_kernel): three launches a
 // step.  The first takes 64-point tiles through the whole network and back:
@@ -531,92 +531,174 @@ __global__ __launch_bounds__(256) void mlp_cast_kernel(const float *p, __bf16 *W
     if (i < kMlpParams) store_bf16(i, param_at(i), p[i], W, WT);
 }
 
-// ---- fused inference: one 64-point tile per workgroup ----
-// weights bf16, layout W_l[n][k]; activations in LDS [64][width + 8]
-template <int K0, int H, int D>
-__global__ __launch_bounds__(256) void mlp_infer_kernel(const double *r, long long npts,
-                                                        const float *Bfreq, int F,
-                                                        const float *ctr_scale,
-                                                        const __bf16 *const *W, const float *const *bias,
-                                                        const float *out_scale, double *J) {
-    constexpr int P = 64;
-    constexpr int LD = (K0 > H ? K0 : H) + 8;
-    __shared__ __align__(16) __bf16 act[2][P][LD];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+// ---- fused inference ----
+
+namespace {
+
+// weights, biases and frequencies in LDS, weight rows of K + 8
+constexpr int kInferW(int l) { return l == 0 ? 0 : kInferW(l - 1) + nout(l - 1) * (kin(l - 1) + 8); }
+constexpr int kInferElems = kInferW(kD) + kNO * (kH + 8);
+constexpr int kInferThreads = 1024;
+constexpr size_t kInferLds = (size_t)kInferElems * 2 + (kBiasN + 4 * kF) * 4;
+typedef unsigned short v2us __attribute__((ext_vector_type(2)));
+
+// (bf16)(z / (1 + e^-z)) of four values, bit for bit that of the exact
+// division: z times the hardware reciprocal (1 ulp) is within 3 ulp of the
+// correctly rounded quotient, so the BF16 values agree unless one of the four
+// lies that close to the middle between two BF16 values (or the divisor's
+// reciprocal is denormal, z < -80), where the wavefront divides: 3% of the
+// time.
+__device__ __forceinline__ v4bf silu_bf16(v4f z) {
+    float h[4];
+    v2us near = {0xffff, 0xffff};
+#pragma unroll
+    for (int i = 0; i < 4; i++) h[i] = z[i] * __builtin_amdgcn_rcpf(1.f + __expf(-z[i]));
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+        // the halves that rounding drops, 0x7ffd .. 0x8003 -> 0 .. 6
+        const uint32_t lo = __builtin_amdgcn_perm(__float_as_uint(h[i + 1]), __float_as_uint(h[i]), 0x05040100u);
+        v2us d;
+        __builtin_memcpy(&d, &lo, 4);
+        d = d - (v2us){0x7ffd, 0x7ffd};
+        near = __builtin_elementwise_min(near, d);
+    }
+    const float low = fminf(fminf(z[0], z[1]), fminf(z[2], z[3]));
+    const bool redo = near[0] <= 6 || near[1] <= 6 || !(low >= -80.f);
+    if (__builtin_expect(__any(redo), 0)) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) h[i] = silu(z[i]);
+    }
+    v4bf r;
+#pragma unroll
+    for (int i = 0; i < 4; i++) r[i] = (__bf16)h[i];
+    return r;
+}
+
+}  // namespace
+
+// 16 points per wavefront, all in registers; 16 wavefronts share the weights
+// in LDS (152 KB) and step through the points without a barrier.  With the
+// weights as the first MFMA operand the lane (g, c) holds rows 4 g .. + 3 of
+// every 16-row block of point c; the next layer wants 8 g .. + 7 of every 32,
+// two lane-group swaps away.  Bound by VALU: 512 SiLU and 64 sine-cosine pairs
+// a point.
+__global__ __launch_bounds__(kInferThreads, 1) void mlp_infer_kernel(
+    const double *r, long long npts, const float *freq, const float *cs, const __bf16 *W,
+    const float *prm, const float *oscale, double *J) {
+    extern __shared__ __align__(16) unsigned char infer_lds[];
+    __bf16 *w = (__bf16 *)infer_lds;
+    float *bias = (float *)(w + kInferElems);  // the layers' biases one after another
+    float *fr = bias + kBiasN;                 // [f][4]
+    const int tid = threadIdx.x, lane = tid & 63;
     const int g = lane >> 4, c = lane & 15;
-    const long long p0 = (long long)blockIdx.x * P;
-    // features: 4 threads per point
-    {
-        const int pl = tid >> 2, part = tid & 3;
-        const long long p = p0 + pl;
-        const float inv = 1.f / ctr_scale[3];
-        float u[3] = {0.f, 0.f, 0.f};
-        if (p < npts) {
-            u[0] = (float)(r[3 * p] - ctr_scale[0]) * inv;
-            u[1] = (float)(r[3 * p + 1] - ctr_scale[1]) * inv;
-            u[2] = (float)(r[3 * p + 2] - ctr_scale[2]) * inv;
-        }
-        for (int f = part; f < F; f += 4) {
-            const float t = 6.283185307179586f *
-                            (Bfreq[3 * f] * u[0] + Bfreq[3 * f + 1] * u[1] + Bfreq[3 * f + 2] * u[2]);
-            float s, co;
-            sincosf(t, &s, &co);
-            act[0][pl][f] = (__bf16)s;
-            act[0][pl][F + f] = (__bf16)co;
-        }
-        if (part == 0) {
-            act[0][pl][2 * F] = (__bf16)u[0];
-            act[0][pl][2 * F + 1] = (__bf16)u[1];
-            act[0][pl][2 * F + 2] = (__bf16)u[2];
-            for (int k = 2 * F + 3; k < K0; k++) act[0][pl][k] = (__bf16)0.f;
-        }
-    }
+    auto stage = [&](auto lc) {
+        constexpr int l = decltype(lc)::value, K = kin(l), N = nout(l);
+        for (int u = tid; u < N * K / 8; u += kInferThreads)
+            *(v4u *)(w + kInferW(l) + u / (K / 8) * (K + 8) + u % (K / 8) * 8) =
+                *(const v4u *)(W + woff(l) + u * 8);
+        for (int n = tid; n < N; n += kInferThreads) bias[l * kH + n] = prm[boff(l) + n];
+    };
+    stage(std::integral_constant<int, 0>{});
+    stage(std::integral_constant<int, 1>{});
+    stage(std::integral_constant<int, 2>{});
+    stage(std::integral_constant<int, 3>{});
+    stage(std::integral_constant<int, 4>{});
+    for (int i = tid; i < 4 * kF; i += kInferThreads) fr[i] = (i & 3) < 3 ? freq[3 * (i >> 2) + (i & 3)] : 0.f;
     __syncthreads();
-    int cur = 0;
-    // hidden layers: each wave computes 16 rows x H columns
-#pragma unroll 1
-    for (int l = 0; l < D; l++) {
-        const int K = l == 0 ? K0 : H;
-        const __bf16 *Wl = W[l];
-        const float *bl = bias[l];
-        v4f acc[H / 16];
-#pragma unroll
-        for (int j = 0; j < H / 16; j++) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
-        for (int k0 = 0; k0 < K; k0 += 32) {
-            const v8bf a = *(const v8bf *)&act[cur][wave * 16 + c][k0 + 8 * g];
-#pragma unroll
-            for (int j = 0; j < H / 16; j++) {
-                const v8bf b = *(const v8bf *)(Wl + (long long)(16 * j + c) * K + k0 + 8 * g);
-                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[j], 0, 0, 0);
-            }
+    const float inv = 1.f / cs[3];
+    const long long step = (long long)gridDim.x * (kInferThreads / 64) * 16;
+    for (long long p0 = ((long long)blockIdx.x * (kInferThreads / 64) + (tid >> 6)) * 16; p0 < npts;
+         p0 += step) {
+        const long long p = p0 + c;
+        const bool valid = p < npts;
+        float u[3] = {0.f, 0.f, 0.f};
+        if (valid) {
+            u[0] = (float)(r[3 * p] - cs[0]) * inv;
+            u[1] = (float)(r[3 * p + 1] - cs[1]) * inv;
+            u[2] = (float)(r[3 * p + 2] - cs[2]) * inv;
         }
+        // features 32 q + 8 g .. + 7 in x[q]: sines, cosines, the coordinates
+        v8bf x[kK0 / 32];
+        const float *fq = fr + fresh(32 * g, 4 * kF);
 #pragma unroll
-        for (int j = 0; j < H / 16; j++)
+        for (int q = 0; q < 2; q++)
 #pragma unroll
-            for (int rr = 0; rr < 4; rr++) {
-                const int n = 16 * j + c;
-                act[cur ^ 1][wave * 16 + 4 * g + rr][n] = (__bf16)silu(acc[j][rr] + bl[n]);
+            for (int i = 0; i < 8; i++) {
+                const v4f b = *(const v4f *)(fq + 4 * (32 * q + i));
+                const float t = 6.283185307179586f * (b[0] * u[0] + b[1] * u[1] + b[2] * u[2]);
+                float s, co;
+                sincosf(t, &s, &co);
+                x[q][i] = (__bf16)s;
+                x[2 + q][i] = (__bf16)co;
             }
-        __syncthreads();
-        cur ^= 1;
-    }
-    // output layer (16 columns: 9 used + the log amplitude in column 9)
-    {
-        const __bf16 *Wo = W[D];
-        const float *bo = bias[D];
+        x[4] = v8bf{};
+        if (g == 0) {
+            x[4][0] = (__bf16)u[0];
+            x[4][1] = (__bf16)u[1];
+            x[4][2] = (__bf16)u[2];
+        }
+        auto layer = [&](auto lc) {
+            constexpr int l = decltype(lc)::value, K = kin(l);
+            // (else the loads of all weights move out of the loop over points)
+            const __bf16 *wl = w + fresh(kInferW(l) + c * (K + 8) + 8 * g, kInferElems);
+            const float *bl = bias + fresh(l * kH + 4 * g, kBiasN);
+            v8bf nx[kH / 32];
+#pragma unroll
+            for (int q = 0; q < kH / 32; q++) {
+                union {
+                    v4bf h;
+                    uint32_t d[2];
+                } b[2];
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    v4f acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int k = 0; k < K / 32; k++)
+                        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            *(const v8bf *)(wl + (32 * q + 16 * j) * (K + 8) + 32 * k), x[k], acc, 0, 0, 0);
+                    const v4f bb = *(const v4f *)(bl + 32 * q + 16 * j);
+                    v4f z;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) z[i] = acc[i] + bb[i];
+                    b[j].h = silu_bf16(z);
+                }
+                // rows 4 g' of two blocks to rows 8 g of the 32: groups (0, 1,
+                // 2, 3) of block A and B become (A0 A1), (A2 A3), (B0 B1), (B2 B3)
+                union {
+                    v8bf v;
+                    uint32_t d[4];
+                } o;
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    const auto s = __builtin_amdgcn_permlane32_swap(b[0].d[e], b[1].d[e], false, false);
+                    const auto t = __builtin_amdgcn_permlane16_swap(s[0], s[1], false, false);
+                    o.d[e] = t[0];
+                    o.d[2 + e] = t[1];
+                }
+                nx[q] = o.v;
+            }
+#pragma unroll
+            for (int q = 0; q < kH / 32; q++) x[q] = nx[q];
+        };
+        layer(std::integral_constant<int, 0>{});
+        layer(std::integral_constant<int, 1>{});
+        layer(std::integral_constant<int, 2>{});
+        layer(std::integral_constant<int, 3>{});
         v4f acc = {0.f, 0.f, 0.f, 0.f};
-        for (int k0 = 0; k0 < H; k0 += 32) {
-            const v8bf a = *(const v8bf *)&act[cur][wave * 16 + c][k0 + 8 * g];
-            const v8bf b = *(const v8bf *)(Wo + (long long)c * H + k0 + 8 * g);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-        }
+        const __bf16 *wo = w + fresh(kInferW(kD) + c * (kH + 8) + 8 * g, kInferElems);
 #pragma unroll
-        for (int rr = 0; rr < 4; rr++) {
-            const long long p = p0 + wave * 16 + 4 * g + rr;
-            const float y = acc[rr] + bo[c];
-            // lane (g, 9) holds the log amplitude of the same point
-            const float e = amp(__shfl(y, (lane & ~15) | 9));
-            if (c < 9 && p < npts) J[9 * p + c] = (double)(y * e * out_scale[c]);
+        for (int k = 0; k < kH / 32; k++)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const v8bf *)(wo + 32 * k), x[k], acc, 0, 0, 0);
+        const v4f bb = *(const v4f *)(bias + fresh(kD * kH + 4 * g, kBiasN));
+        float y[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) y[i] = acc[i] + bb[i];
+        // row 9, the log amplitude, is element 1 of lane group 2
+        const float e = amp(__shfl(y[1], 32 + c));
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int n = 4 * g + i;
+            if (n < 9 && valid) J[9 * p + n] = (double)(y[i] * e * oscale[n]);
         }
     }
 }
@@ -664,12 +746,16 @@ hipError_t mlp_cast(const float *p, __bf16 *W, __bf16 *WT, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t mlp_infer(const double *r, long long npts, const float *Bfreq, int F, const float *cs,
-                     const __bf16 *const *W, const float *const *bias, const float *out_scale,
-                     double *J, hipStream_t s) {
+hipError_t mlp_infer(const double *r, long long npts, const float *freq, const float *cs,
+                     const __bf16 *W, const float *prm, const float *oscale, double *J, hipStream_t s) {
     if (npts <= 0) return hipSuccess;
-    hipLaunchKernelGGL((mlp_infer_kernel<160, 128, 4>), dim3(blocks(npts, 64)), dim3(256), 0, s, r,
-                       npts, Bfreq, F, cs, W, bias, out_scale, J);
+    hipError_t e = hipFuncSetAttribute((const void *)mlp_infer_kernel,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kInferLds);
+    if (e != hipSuccess) return e;
+    // one workgroup per CU at most, 256 points at a time
+    const unsigned groups = (unsigned)std::min<long long>((npts + 255) / 256, 256);
+    hipLaunchKernelGGL(mlp_infer_kernel, dim3(groups), dim3(kInferThreads), kInferLds, s, r, npts, freq,
+                       cs, W, prm, oscale, J);
     return hipGetLastError();
 }
 

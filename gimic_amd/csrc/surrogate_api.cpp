@@ -59,7 +59,7 @@ struct gimic_mlp {
     long long np = 0;                 // parameter count
     long long woff[kD + 1], boff[kD + 1];
     int kin[kD + 1], nout[kD + 1];
-    Buf params, params_b, params_t, grad, adam_m, adam_v, freq, cs, oscale, ptrs;
+    Buf params, params_b, params_t, grad, adam_m, adam_v, freq, cs, oscale;
     Buf X[kD + 1], dZ[kD], dY, part, bpart, loss;
     long long cap = 0;  // batch capacity of the work buffers
     long long step = 0;
@@ -198,15 +198,6 @@ int gimic_mlp_create(gimic_mlp **out, double sigma, const double *center_scale,
             chk(hipMemcpyAsync(n->oscale.p, os, 36, hipMemcpyHostToDevice, s), "copy");
             chk(mlp_cast(n->params.as<float>(), n->params_b.as<__bf16>(), n->params_t.as<__bf16>(), s),
                 "cast");
-            // device table of layer pointers for the fused inference kernel
-            std::vector<void *> tab(2 * (kD + 1));
-            for (int l = 0; l <= kD; l++) {
-                tab[l] = n->params_b.as<__bf16>() + n->woff[l];
-                tab[kD + 1 + l] = n->params.as<float>() + n->boff[l];
-            }
-            n->ptrs.need(tab.size() * sizeof(void *));
-            chk(hipMemcpyAsync(n->ptrs.p, tab.data(), tab.size() * sizeof(void *),
-                               hipMemcpyHostToDevice, s), "copy");
             chk(hipStreamSynchronize(s), "sync");
         } catch (...) {
             delete n;
@@ -296,10 +287,8 @@ int gimic_mlp_predict(gimic_mlp *n, long long npts, const double *d_r, double *d
     return guard([&] {
         if (!n || npts < 0 || (npts > 0 && (!d_r || !d_J))) throw MlpError(GIMIC_EINVAL, "bad argument");
         hipStream_t s = stream ? (hipStream_t)stream : work_stream(n);
-        const __bf16 *const *W = (const __bf16 *const *)n->ptrs.p;
-        const float *const *B = (const float *const *)((void **)n->ptrs.p + kD + 1);
-        chk(mlp_infer(d_r, npts, n->freq.as<float>(), kF, n->cs.as<float>(), W, B,
-                      n->oscale.as<float>(), d_J, s), "infer");
+        chk(mlp_infer(d_r, npts, n->freq.as<float>(), n->cs.as<float>(), n->params_b.as<__bf16>(),
+                      n->params.as<float>(), n->oscale.as<float>(), d_J, s), "infer");
     });
 }
 
