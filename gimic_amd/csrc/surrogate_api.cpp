@@ -51,6 +51,13 @@ struct Buf {
     T *as() const { return (T *)p; }
 };
 
+// a range of a Buf
+struct Part {
+    void *p = nullptr;
+    template <class T>
+    T *as() const { return (T *)p; }
+};
+
 }  // namespace
 
 struct gimic_mlp {
@@ -59,8 +66,9 @@ struct gimic_mlp {
     long long np = 0;                 // parameter count
     long long woff[kD + 1], boff[kD + 1];
     int kin[kD + 1], nout[kD + 1];
-    Buf params, params_b, params_t, grad, adam_m, adam_v, freq, cs, oscale;
-    Buf X[kD + 1], dZ[kD], dY, part, bpart, loss;
+    Buf state;  // the parts below in one allocation (each costs about 1 ms)
+    Part params, params_b, params_t, grad, adam_m, adam_v, freq, cs, oscale, loss;
+    Buf X[kD + 1], dZ[kD], dY, part, bpart;
     long long cap = 0;  // batch capacity of the work buffers
     long long step = 0;
     ~gimic_mlp() {
@@ -180,16 +188,21 @@ int gimic_mlp_create(gimic_mlp **out, double sigma, const double *center_scale,
             float os[9];
             for (int i = 0; i < 9; i++) os[i] = (float)out_scale[i];
             hipStream_t s = work_stream(n);
-            n->params.need(off * 4);
-            n->params_b.need(off * 2);
-            n->params_t.need((size_t)kMlpTransposed * 2);
-            n->grad.need(off * 4);
-            n->adam_m.need(off * 4);
-            n->adam_v.need(off * 4);
-            n->freq.need(fr.size() * 4);
-            n->cs.need(16);
-            n->oscale.need(36);
-            n->loss.need(4);
+            struct {
+                Part *q;
+                size_t bytes;
+            } parts[] = {{&n->params, (size_t)off * 4}, {&n->params_b, (size_t)off * 2},
+                         {&n->params_t, (size_t)kMlpTransposed * 2}, {&n->grad, (size_t)off * 4},
+                         {&n->adam_m, (size_t)off * 4}, {&n->adam_v, (size_t)off * 4},
+                         {&n->freq, fr.size() * 4}, {&n->cs, 16}, {&n->oscale, 36}, {&n->loss, 4}};
+            size_t total = 0;
+            for (auto &x : parts) total += (x.bytes + 255) / 256 * 256;
+            n->state.need(total);
+            total = 0;
+            for (auto &x : parts) {
+                x.q->p = n->state.as<unsigned char>() + total;
+                total += (x.bytes + 255) / 256 * 256;
+            }
             chk(hipMemcpyAsync(n->params.p, p.data(), off * 4, hipMemcpyHostToDevice, s), "copy");
             chk(hipMemsetAsync(n->adam_m.p, 0, off * 4, s), "memset");
             chk(hipMemsetAsync(n->adam_v.p, 0, off * 4, s), "memset");
