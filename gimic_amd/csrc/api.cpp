@@ -129,7 +129,7 @@ struct Workspace {
     DevBuf phi64, grad64, phis, grad32, part;
     // spatial tiles of a chunk: sorted points, their caller indices, sort
     // scratch, and the screening block list of every contraction row tile
-    DevBuf spts, perm, bpart, sortscr, bcount, k8count, toff, kcount, klist;
+    DevBuf spts, perm, bpart, sortscr, bcount, k8count, kcount, klist;
     // FP64 pass near nuclei: selection index list, their points, selection
     // scratch and count
     DevBuf near_idx, near_pts, near_scr, near_cnt;
@@ -327,7 +327,7 @@ struct gimic_ctx {
     std::map<std::pair<std::vector<int>, int>, std::unique_ptr<Mats>> mats;
     // evaluation workspace, and host-array staging of the batch calls
     Workspace ws;
-    DevBuf pts_tmp, jt_tmp, contrib, planes, pparams, offs, outs;
+    DevBuf pts_tmp, jt_tmp, contrib, planes, pparams, outs;
     // internal function order (see setup_device): fun_orig[i] is the caller's
     // index of internal function i
     std::vector<int> fun_orig;
@@ -635,7 +635,7 @@ size_t scratch_eval_bytes(const gimic_ctx *c, int prec, int nmatset, size_t rows
     size_t n = prec == GIMIC_PREC_FP64 ? r(rows * ld * 8) + r(3 * rows * ld * 8)
                                        : r(rows * ld * 2 * kAParts) + r(3 * rows * ld * 4);
     n += r(rows * 24) + r(rows * 4) + r(256 * 6 * 8) + r((size_t)sort_scratch_ints((int)rows) * 4);
-    n += 3 * r(t * 4) + r((t + 1) * 4) + r(t * nblk * 32);
+    n += 3 * r(t * 4) + r(t * nblk * 32);
     n += r((size_t)nmatset * split * kNQ * rows * 8);
     return n;
 }
@@ -779,7 +779,6 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
     grow(W.sortscr, (size_t)sort_scratch_ints((int)rows_cap) * 4, false);
     grow(W.bcount, rows_cap / kMinTileRows * 4, false);
     grow(W.k8count, rows_cap / kMinTileRows * 4, false);
-    grow(W.toff, (rows_cap / kMinTileRows + 1) * 4, false);
     grow(W.kcount, rows_cap / kMinTileRows * 4, false);
     grow(W.klist, rows_cap / kMinTileRows * nblk * 8 * 4, false);  // granules of 4 at most
     const int nmatset = M.nmatset;
@@ -902,7 +901,7 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
         const int tr64 = f64_tile_rows(n_c);
         auto run = [&](int variant, int split = -1) {
             plan_variant(variant, split);
-            ca.toff = dense ? nullptr : W.toff.as<int>();
+            ca.compressed = !dense;
             ca.tile_rows = tr64;
             if (variant == 0) hip_check(launch_contract_f64(ca, st), "contract_f64");
             else if (variant == 3) hip_check(launch_contract_mx2(ca, 2, 2, 4, st), "contract_mx2");
@@ -912,16 +911,13 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
             else hip_check(launch_contract_mx2(ca, 3, 2, 8, st), "contract_mx2");
         };
         // basis evaluation: FP64 rows (mode 0) or split rows (mode 2), compressed
-        // to each row tile's live groups (lists and offsets come first)
+        // to each row tile's live groups (the lists come first)
         auto eval = [&](int variant) {
             const int tr = variant == 0 ? tr64 : mixed_tile_rows(variant);
             lists(tr, variant == 0 ? 4 : 8);
-            if (!dense)
-                hip_check(launch_tile_offsets(W.kcount.as<int>(), rows / tr, W.toff.as<int>(), st),
-                          "tile_offsets");
             ea.kcount = W.kcount.as<int>();
             ea.klist = W.klist.as<int>();
-            ea.toff = dense ? nullptr : W.toff.as<int>();
+            ea.compressed = !dense;
             ea.nblk = nblk;
             ea.tile_rows = tr;
             hip_check(launch_basis_eval(ea, variant == 0 ? 0 : 2, st), "basis_eval");
@@ -1553,9 +1549,8 @@ void flux_buffers(gimic_ctx *c, int64_t npts, int nplanes) {
     c->jt_tmp.alloc(np * 72, st, false);
     c->contrib.alloc(np * 24, st, false);
     c->planes.alloc(np * 4, st, false);
-    c->pparams.alloc((size_t)nplanes * 80, st, false);
-    c->offs.alloc((size_t)(nplanes + 1) * 8, st, false);
-    c->outs.alloc((size_t)nplanes * 72, st, false);
+    c->pparams.alloc((size_t)nplanes * 88 + 8, st, false);
+    c->outs.alloc((size_t)nplanes * 72 * (1 + plane_parts(npts, nplanes)), st, false);
 }
 
 // Plane flux over the points, weights and plane indices that `prepare(st)`
@@ -1568,7 +1563,11 @@ void flux_run(gimic_ctx *c, int64_t npts, int nplanes, const int64_t *offs, cons
               int precision, double *out, double *out_mod, double *out_acid, double *jt,
               std::vector<uintptr_t> source, Prep &&prepare) {
     hipStream_t st = c->stream;
-    std::vector<double> params(10 * (size_t)nplanes);
+    // plane offsets, then per-plane parameters, in one copy
+    const size_t no = (size_t)nplanes + 1;
+    std::vector<double> head(no + 10 * (size_t)nplanes);
+    std::memcpy(head.data(), offs, no * 8);
+    double *params = head.data() + no;
     for (int k = 0; k < nplanes; k++) {
         for (int d = 0; d < 3; d++) {
             params[3 * k + d] = normals[3 * k + d];
@@ -1579,14 +1578,13 @@ void flux_run(gimic_ctx *c, int64_t npts, int nplanes, const int64_t *offs, cons
     }
     const size_t np = (size_t)std::max<int64_t>(npts, 1);
     double *d_r = c->pts_tmp.as<double>(), *d_w = d_r + 3 * np;
-    hip_check(hipMemcpyAsync(c->pparams.p, params.data(), params.size() * 8,
-                             hipMemcpyHostToDevice, st), "copy params");
-    hip_check(hipMemcpyAsync(c->offs.p, offs, (size_t)(nplanes + 1) * 8, hipMemcpyHostToDevice, st),
-              "copy offs");
+    hip_check(hipMemcpyAsync(c->pparams.p, head.data(), head.size() * 8, hipMemcpyHostToDevice, st),
+              "copy plane parameters");
+    const long long *d_offs = (const long long *)c->pparams.p;
     FluxDev fd;
     fd.w = d_w;
     fd.plane = c->planes.as<int>();
-    const double *pp = c->pparams.as<double>();
+    const double *pp = c->pparams.as<double>() + no;
     fd.pnorm = pp;
     fd.pbfield = pp + 3 * nplanes;
     fd.pcenter = pp + 6 * nplanes;
@@ -1594,14 +1592,15 @@ void flux_run(gimic_ctx *c, int64_t npts, int nplanes, const int64_t *offs, cons
     fd.contrib = c->contrib.as<double>();
     fd.contrib_mod = out_mod ? c->contrib.as<double>() + np : nullptr;
     fd.contrib_acid = out_acid ? c->contrib.as<double>() + 2 * np : nullptr;
+    // sums of the arrays asked for, in order: current, modulus, ACID
+    int kind[3] = {0, 0, 0}, kinds = 1;
+    if (out_mod) kind[kinds++] = 1;
+    if (out_acid) kind[kinds++] = 2;
+    double *d_out = c->outs.as<double>();
     auto reduce = [&] {
-        for (int k = 0; k < 3; k++) {
-            if ((k == 1 && !out_mod) || (k == 2 && !out_acid)) continue;
-            hip_check(launch_plane_reduce(c->contrib.as<double>() + k * np,
-                                          (const long long *)c->offs.p, nplanes,
-                                          c->outs.as<double>() + 3 * k * nplanes, st),
-                      "plane_reduce");
-        }
+        hip_check(launch_plane_reduce(c->contrib.as<double>(), (long long)np, kind, kinds, d_offs, npts,
+                                      nplanes, d_out + 9 * (size_t)nplanes, d_out, st),
+                  "plane_reduce");
     };
     // the FP64 pass over points next to a nucleus runs eagerly after a
     // captured mixed evaluation, and the reductions after it
@@ -1624,12 +1623,12 @@ void flux_run(gimic_ctx *c, int64_t npts, int nplanes, const int64_t *offs, cons
             (uintptr_t)c->giao, (uintptr_t)c->diamag, (uintptr_t)c->paramag,
             (uintptr_t)c->mixed_variant, (uintptr_t)st, (uintptr_t)c->pts_tmp.p,
             (uintptr_t)c->jt_tmp.p, (uintptr_t)c->contrib.p, (uintptr_t)c->planes.p,
-            (uintptr_t)c->pparams.p, (uintptr_t)c->offs.p, (uintptr_t)c->outs.p,
+            (uintptr_t)c->pparams.p, (uintptr_t)c->outs.p,
             (uintptr_t)c->ws.phi64.p, (uintptr_t)c->ws.grad64.p, (uintptr_t)c->ws.grad32.p,
             (uintptr_t)c->ws.part.p, (uintptr_t)M.b64.p, (uintptr_t)c->ws.phis.p,
             (uintptr_t)M.bs3.p, (uintptr_t)c->mixed_split, (uintptr_t)c->ws.spts.p,
             (uintptr_t)c->ws.perm.p, (uintptr_t)c->ws.bpart.p, (uintptr_t)c->ws.sortscr.p,
-            (uintptr_t)c->ws.bcount.p, (uintptr_t)c->ws.k8count.p, (uintptr_t)c->ws.toff.p,
+            (uintptr_t)c->ws.bcount.p, (uintptr_t)c->ws.k8count.p,
             (uintptr_t)c->ws.kcount.p, (uintptr_t)c->ws.klist.p,
             (uintptr_t)refine,
             (uintptr_t)c->chunk_bytes};
@@ -1666,17 +1665,18 @@ void flux_run(gimic_ctx *c, int64_t npts, int nplanes, const int64_t *offs, cons
             reduce();
         }
     }
-    std::vector<double> res(9 * (size_t)nplanes);
+    std::vector<double> res(3 * (size_t)kinds * nplanes);
     hip_check(hipMemcpyAsync(res.data(), c->outs.p, res.size() * 8, hipMemcpyDeviceToHost, st),
               "copy out");
     if (jt && npts > 0)
         hip_check(hipMemcpyAsync(jt, c->jt_tmp.p, (size_t)npts * 72, hipMemcpyDeviceToHost, st),
                   "copy jt");
     hip_check(hipStreamSynchronize(st), "hipStreamSynchronize");
-    std::copy(res.begin(), res.begin() + 3 * nplanes, out);
-    if (out_mod) std::copy(res.begin() + 3 * nplanes, res.begin() + 6 * nplanes, out_mod);
+    auto sums = [&](int k) { return res.begin() + 3 * (size_t)k * nplanes; };
+    std::copy(sums(0), sums(1), out);
+    if (out_mod) std::copy(sums(1), sums(2), out_mod);
     if (out_acid)
-        for (int k = 0; k < nplanes; k++) out_acid[k] = res[6 * (size_t)nplanes + 3 * k];
+        for (int k = 0; k < nplanes; k++) out_acid[k] = sums(kinds - 1)[3 * k];
 }
 
 }  // namespace
@@ -1705,7 +1705,7 @@ int gimic_flux_planes(gimic_ctx *c, int nplanes, const int64_t *offs, const doub
         }
         flux_run(c, npts, nplanes, offs, normals, bfields, centers, radii, spin, precision, out,
                  out_mod, out_acid, jt, {(uintptr_t)0}, [&](hipStream_t s) {
-                     hip_check(launch_plane_index((const long long *)c->offs.p, nplanes, npts,
+                     hip_check(launch_plane_index((const long long *)c->pparams.p, nplanes, npts,
                                                   c->planes.as<int>(), s),
                                "plane_index");
                  });

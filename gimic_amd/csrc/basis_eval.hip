@@ -70,9 +70,11 @@ __device__ __forceinline__ void radial_parts(const EvalArgs &a, const DevShell &
 }
 
 // Candidate lists (below) for bases of at least this many shells: with fewer,
-// nearly every shell reaches every tile (tetracene, 144 shells: 6% slower
-// with the list, which costs registers and a pass over the shells)
-constexpr int kCandMinShells = 400;
+// nearly every shell reaches every tile and the list costs registers and a
+// pass over the shells.  Tetracene (144 shells): its mixed scan is 6% slower
+// with the list, its FP64 scan 6% faster (basis 1.66 to 1.35 ms: the pass holds
+// three rows instead of seven, so screened pairs cost more there).
+constexpr int kCandMinShells = 400, kCandMinShellsF64 = 64;
 // Shells whose candidacy the staged kernel settles per pass of its loop
 constexpr int kCandChunk = 1024;
 // LDS beyond the image and the block positions: candidate list, bounding
@@ -311,6 +313,7 @@ void basis_eval_staged_kernel(EvalArgs a) {
     const int tid = threadIdx.x, tp = a.tile_points;
     const size_t row0 = (size_t)blockIdx.x * tp;
     constexpr int kGran = F64 ? 4 : 8, kPer = 32 / kGran, kShift = list_shift(kGran);
+    if (row0 >= (size_t)a.npts) return;  // padding rows: nobody reads their sums
     // the tile's rows in the output, and the place of each group in them
     const int t = (int)(row0 / a.tile_rows);
     const int kg = a.kcount[t];
@@ -321,7 +324,7 @@ void basis_eval_staged_kernel(EvalArgs a) {
     __syncthreads();
     for (int i = tid; i < kg; i += 256)
         gpos[a.klist[(size_t)t * a.nblk * kPer + i] >> kShift] = (short)i;
-    const size_t base = (size_t)a.toff[t] * a.tile_rows * kGran;
+    const size_t base = (size_t)t * a.tile_rows * a.lda;
     const size_t rin = row0 - (size_t)t * a.tile_rows;
     typedef typename std::conditional<F64, double, __bf16>::type Value;
     typedef typename std::conditional<F64, double, float>::type Grad;
@@ -483,7 +486,7 @@ hipError_t launch_basis_eval(const EvalArgs &a, int mode, hipStream_t s) {
     if (total <= 0) return hipSuccess;
     if (a.lmax < 0 || a.lmax > kDevMaxL) return hipErrorInvalidValue;
     const bool f64 = mode == 0;
-    if (f64 && !a.toff) {
+    if (f64 && !a.compressed) {
         // dense rows of a basis too wide for the LDS image
         hipLaunchKernelGGL(basis_eval_kernel<0>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
                            s, a);
@@ -496,12 +499,12 @@ hipError_t launch_basis_eval(const EvalArgs &a, int mode, hipStream_t s) {
     // tetracene scan's mixed basis evaluation, 64 rows no better
     EvalArgs b = a;
     const size_t row_bytes = (size_t)a.lda * (f64 ? 32 : 2 * kAParts + 12);
-    if (row_bytes > kMaxRowBytes || !a.toff) return hipErrorInvalidValue;
+    if (row_bytes > kMaxRowBytes || !a.compressed) return hipErrorInvalidValue;
     b.tile_points = 32;
     b.lds_image = std::max<size_t>(36 * 1024, row_bytes);
     // the image, the group positions (16-byte aligned) and, for bases of
-    // kCandMinShells shells or more, the candidate list
-    const bool cand = a.nshell >= kCandMinShells;
+    // kCandMinShells (F64) shells or more, the candidate list
+    const bool cand = a.nshell >= (f64 ? kCandMinShellsF64 : kCandMinShells);
     const size_t lds = b.lds_image + gpos_bytes(a.nblk, f64 ? 4 : 8) + (cand ? kCandBytes : 0);
     // (the candidate list's bounding sphere takes one row per lane of a wavefront)
     if (a.tile_rows % b.tile_points || a.rows % a.tile_rows || a.nblk * 32 != a.lda)

@@ -86,9 +86,9 @@ __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
     const int rin = (blockIdx.x >> 3) % parts * kRows + wave * 16 + c;
     const size_t row = (size_t)rtile * a.tile_rows + rin;
     // the point's values and gradients: dense, or compressed to the tile's granules
-    const bool cmp = a.toff != nullptr;
+    const bool cmp = a.compressed;
     const size_t w = cmp ? (size_t)a.kcount[rtile] * 4 : (size_t)a.lda;
-    const size_t base = cmp ? (size_t)a.toff[rtile] * a.tile_rows * 4 : (size_t)rtile * a.tile_rows * w;
+    const size_t base = (size_t)rtile * a.tile_rows * a.lda;
     const double *A = a.a64 + base + rin * w;
     const double *G = a.g64 + (cmp ? 3 * base : base) + rin * w;
     const size_t gplane = cmp ? (size_t)a.tile_rows * w : (size_t)a.gplane;

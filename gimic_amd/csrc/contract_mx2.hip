@@ -227,16 +227,13 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
     // -1 pads the last four (zero right operand)
     const int *K8 = a.klist + (size_t)rtile * a.nblk * 4;
     const int nq = (a.kcount[rtile] + 3) >> 2;
-    // This tile's basis rows: dense [row][lda], or compressed to the live
-    // groups (a.toff non-null: the basis kernel wrote only those, so A and
-    // the gradients are addressed by list position)
-    const bool cmp = a.toff != nullptr;
-    const size_t wcols = cmp ? (size_t)8 * a.kcount[rtile] : (size_t)lda;  // functions per row
-    const size_t arow = kAParts * wcols;                                     // BF16 per split row
-    const __bf16 *Atile = cmp ? a.as3 + (size_t)a.toff[rtile] * kRows * (8 * kAParts)
-                              : a.as3 + row0 * arow;
-    const float *Gtile = cmp ? a.g32 + (size_t)a.toff[rtile] * kRows * 24 : a.g32 + row0 * wcols;
-    const size_t gpl = cmp ? (size_t)kRows * wcols : (size_t)a.gplane;  // gradient plane stride
+    // This tile's basis rows hold only its live groups, in list order
+    // (EvalArgs): A and the gradients are addressed by list position
+    const size_t wcols = (size_t)8 * a.kcount[rtile];  // functions per row
+    const size_t arow = kAParts * wcols;                // BF16 per split row
+    const __bf16 *Atile = a.as3 + row0 * lda * kAParts;
+    const float *Gtile = a.g32 + row0 * lda * 3;
+    const size_t gpl = (size_t)kRows * wcols;           // gradient plane stride
     const int np = pieces_of(wave, WAVES);  // pieces this wavefront copies per block
     // this workgroup's partial sums, row-major [row][kNQ]
     double *pout = a.part + ((size_t)set * a.nsplit + split) * kNQ * rows;
@@ -253,7 +250,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
     const __bf16 *Arow = Atile + (size_t)(wave * 16 * kRB + c) * arow;
     auto a_off = [&](int4 v) -> size_t {  // this lane's group of a K-step, in BF16 of a row
         const int x = g == 0 ? v.x : g == 1 ? v.y : g == 2 ? v.z : v.w;
-        return x < 0 ? 0 : (size_t)(cmp ? (x & 4095) : (x >> 12)) * (8 * kAParts);
+        return x < 0 ? 0 : (size_t)(x & 4095) * (8 * kAParts);
     };
     // pair blocks of this density set: rows of K-groups (nkg: the zero row)
     // of ngn + 1 N-groups (ngn: the zero block)
@@ -384,7 +381,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
         for (int h = 0; h < 2; h++) {
             const int x = pick4(en, 2 * h + (c >> 3));
             const int fn = x < 0 ? 0 : (x >> 12) * 8 + (c & 7);
-            acol[h] = x < 0 ? 0 : (cmp ? (x & 4095) : (x >> 12)) * 8 + (c & 7);
+            acol[h] = x < 0 ? 0 : (x & 4095) * 8 + (c & 7);
 #pragma unroll
             for (int d = 0; d < 3; d++) R[h][d] = a.rf32[(size_t)d * a.ncol_pad + fn];
         }

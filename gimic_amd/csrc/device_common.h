@@ -101,13 +101,13 @@ struct EvalArgs {
     int tile_points;     // points per workgroup of the LDS-staged kernel (set by the launcher)
     size_t lds_image;    // bytes of its LDS image (set by the launcher)
     int lmax;            // largest shell l of the basis
-    // Compressed rows (toff non-null): a row tile of tile_rows rows keeps only
-    // its kcount[t] live groups of gran = 8 (mixed) or 4 (FP64) functions
-    // (TileArgs); its rows start at function toff[t] * tile_rows * gran: split
-    // values [row][place][kAParts][8] or FP64 values [row][gran place], and
-    // gradients [3][tile_rows][gran kcount] from three times that.  Only FP64
-    // rows of more than kMaxRowBytes are dense.
-    const int *kcount, *klist, *toff;
+    // Compressed rows: a row tile of tile_rows rows keeps only its kcount[t]
+    // live groups of gran = 8 (mixed) or 4 (FP64) functions (TileArgs), from
+    // where its dense rows would start: split values [row][place][kAParts][8] or
+    // FP64 values [row][gran place], and gradients [3][tile_rows][gran kcount]
+    // (three times as far).  Only FP64 rows of more than kMaxRowBytes are dense.
+    int compressed;
+    const int *kcount, *klist;
     int nblk, tile_rows;
 };
 constexpr size_t kMaxRowBytes = 150 * 1024;
@@ -133,8 +133,7 @@ struct ContractArgs {
     // split s of a tile takes N-tiles [s * count / nsplit, (s+1) * count / nsplit)
     int nblk, tile_rows;  // tile_rows: FP64 kernel only
     const int *kcount, *klist;
-    // compressed operands (see EvalArgs): null for dense rows
-    const int *toff;
+    int compressed;      // FP64 kernel: rows as in EvalArgs
 };
 // FP64 right operand in HBM: one pair block per (density set, 4-function
 // K-granule, 4-function N-granule) of 7 matrices x 4 x 4 elements,
@@ -254,8 +253,12 @@ hipError_t launch_plane_index(const long long *offs, int nplanes, long long npts
 hipError_t launch_plane_grid(const PlaneGridArgs &a, double *r, double *w, int *plane,
                              hipStream_t s);
 
-// deterministic per-plane sums of contributions: out[3*plane] = net, pos, neg
-hipError_t launch_plane_reduce(const double *contrib, const long long *offs, int nplanes,
+// Per-plane sums, in a fixed order, of `kinds` arrays of contributions `stride`
+// apart: out[3 * (k * nplanes + plane)] = net, pos, neg of array kind[k].  part:
+// 9 * nplanes * plane_parts(npts, nplanes) doubles.
+int plane_parts(long long npts, int nplanes);
+hipError_t launch_plane_reduce(const double *contrib, long long stride, const int *kind, int kinds,
+                               const long long *offs, long long npts, int nplanes, double *part,
                                double *out, hipStream_t s);
 
 // Spatial tiles (tiles.hip).  launch_sort_points orders n points along a
@@ -284,8 +287,6 @@ struct TileArgs {
 };
 
 hipError_t launch_block_lists(const TileArgs &a, hipStream_t s);
-// toff[t] = sum of cnt[0 .. t-1] for t = 0 .. ntiles (one workgroup)
-hipError_t launch_tile_offsets(const int *cnt, int ntiles, int *toff, hipStream_t s);
 
 hipError_t run_mfma_layout_probe(double *h_f64, float *h_bf16);
 hipError_t run_mfma32_layout_probe(float *h_out);  // 2048 floats

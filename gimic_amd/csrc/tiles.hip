@@ -10,9 +10,9 @@
 //
 // Two steps per chunk of points:
 //  1. Order the points along a Morton curve of 32^3 cubic cells over their
-//     bounding box (a stable LSD radix sort with 4-bit digits of the 15-bit
-//     cell key, so the order - and with it every result bit - is the same
-//     on every run); the basis, contraction and finalize kernels work on the
+//     bounding box (a stable LSD radix sort with two 8-bit digits of the
+//     15-bit cell key, so the order - and with it every result bit - is the
+//     same on every run); the basis, contraction and finalize kernels work on the
 //     sorted rows, and finalize writes each tensor back to its caller index.
 //  2. For every row tile of the contraction kernel, list in ascending order
 //     the groups of 8 or 4 functions touched by a shell whose centre lies
@@ -26,8 +26,10 @@ namespace gimic {
 namespace {
 
 constexpr int kSortBlock = 1024;  // elements per radix block (4 rounds of 256)
-constexpr int kBins = 16;         // 4-bit digits
-constexpr int kCellBits = 5;      // 32 cells per axis
+constexpr int kBins = 256;        // 8-bit digits
+constexpr int kCellBits = 5;      // 32 cells per axis: a 15-bit key, two digits
+constexpr int kSmallSort = 2048;  // points that one workgroup sorts by itself
+constexpr int kSmallBits = 11;    // of their index
 
 __device__ __forceinline__ unsigned spread3(unsigned v) {
     // bits b0..b4 -> positions 0, 3, 6, 9, 12
@@ -67,131 +69,217 @@ __global__ __launch_bounds__(256) void bbox_partial_kernel(const double *pts, in
     if (t < 6) out[blockIdx.x * 6 + t] = s[t][0];
 }
 
-// Morton key of each point's cell; keys[i] = key, idx[i] = i
-__global__ __launch_bounds__(256) void cell_key_kernel(const double *pts, int n, const double *bpart,
-                                                       int nbpart, unsigned *keys, int *idx) {
-    __shared__ double s[6][256];
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-        s[d][t] = t < nbpart ? bpart[t * 6 + d] : INFINITY;
-        s[3 + d][t] = t < nbpart ? bpart[t * 6 + 3 + d] : -INFINITY;
-    }
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w)
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                s[d][t] = fmin(s[d][t], s[d][t + w]);
-                s[3 + d][t] = fmax(s[3 + d][t], s[3 + d][t + w]);
-            }
-        __syncthreads();
-    }
-    const double lo[3] = {s[0][0], s[1][0], s[2][0]};
-    double h = fmax(fmax(s[3][0] - lo[0], s[4][0] - lo[1]), s[5][0] - lo[2]) / (1 << kCellBits);
+// Morton key of the cell of a point in the box [lo, hi]
+__device__ __forceinline__ unsigned cell_key(const double *pt, const double (&lo)[3],
+                                             const double (&hi)[3]) {
+    double h = fmax(fmax(hi[0] - lo[0], hi[1] - lo[1]), hi[2] - lo[2]) / (1 << kCellBits);
     if (!(h > 0.0) || !isfinite(h)) h = 1.0;
-    const long long i = (long long)blockIdx.x * 256 + t;
-    if (i >= n) return;
     unsigned key = 0;
 #pragma unroll
     for (int d = 0; d < 3; d++) {
         // fmax/fmin map NaN to the first cell
-        const double c = fmin(fmax((pts[3 * i + d] - lo[d]) / h, 0.0), (double)((1 << kCellBits) - 1));
+        const double c = fmin(fmax((pt[d] - lo[d]) / h, 0.0), (double)((1 << kCellBits) - 1));
         key |= spread3((unsigned)c) << d;
     }
-    keys[i] = key;
-    idx[i] = (int)i;
+    return key;
 }
 
-// per radix block digit counts, digit-major: hist[d * nb + b]
-__global__ __launch_bounds__(256) void radix_hist_kernel(const unsigned *keys, int n, int shift,
+// box of the lanes' boxes, left in every lane of the wavefront
+__device__ __forceinline__ void wave_box(double (&lo)[3], double (&hi)[3]) {
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            lo[d] = fmin(lo[d], __shfl_xor(lo[d], w));
+            hi[d] = fmax(hi[d], __shfl_xor(hi[d], w));
+        }
+}
+
+// Up to kSmallSort points in one workgroup and launch: box, keys, a bitonic
+// sort of (key, index) in LDS (unique keys, so the order is the stable one),
+// and the sorted points.  A single point took 14 launches of the general sort,
+// half of the time of its tensor.
+__global__ __launch_bounds__(1024) void small_sort_kernel(const double *pts, int n, double *spts,
+                                                          int *perm) {
+    __shared__ unsigned v[kSmallSort];
+    __shared__ double box[16][6];
+    const int t = threadIdx.x, nt = blockDim.x, lane = t & 63, wave = t >> 6;
+    double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (int i = t; i < n; i += nt)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            lo[d] = fmin(lo[d], pts[3 * i + d]);
+            hi[d] = fmax(hi[d], pts[3 * i + d]);
+        }
+    wave_box(lo, hi);
+    if (lane == 0)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            box[wave][d] = lo[d];
+            box[wave][3 + d] = hi[d];
+        }
+    __syncthreads();
+    for (int w = 0; w < nt / 64; w++)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            lo[d] = fmin(lo[d], box[w][d]);
+            hi[d] = fmax(hi[d], box[w][3 + d]);
+        }
+    int m = 1;
+    while (m < n) m <<= 1;
+    for (int i = t; i < m; i += nt)
+        v[i] = i < n ? cell_key(pts + 3 * i, lo, hi) << kSmallBits | (unsigned)i : ~0u;
+    for (int k = 2; k <= m; k <<= 1)
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            __syncthreads();
+            for (int q = t; q < m / 2; q += nt) {
+                const int i = (q & ~(j - 1)) << 1 | (q & (j - 1)), o = i | j;
+                const unsigned x = v[i], y = v[o];
+                if ((x > y) == ((i & k) == 0)) {
+                    v[i] = y;
+                    v[o] = x;
+                }
+            }
+        }
+    __syncthreads();
+    for (int j = t; j < n; j += nt) {
+        const int i = (int)(v[j] & ((1u << kSmallBits) - 1));
+        perm[j] = i;
+#pragma unroll
+        for (int d = 0; d < 3; d++) spts[3 * j + d] = pts[3 * i + d];
+    }
+}
+
+// Counts of digit `shift` of 1024 keys, digit-major: hist[d * nb + b].  FIRST:
+// the keys come from the points and the partial boxes, and are stored.
+template <bool FIRST>
+__global__ __launch_bounds__(256) void radix_hist_kernel(const double *pts, const double *bpart,
+                                                         int nbpart, unsigned *keys, int n, int shift,
                                                          int *hist) {
     __shared__ int cnt[kBins];
+    __shared__ double box[4][6];
     const int t = threadIdx.x, b = blockIdx.x, nb = gridDim.x;
-    if (t < kBins) cnt[t] = 0;
+    double lo[3], hi[3];
+    cnt[t] = 0;
+    if (FIRST) {
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            lo[d] = t < nbpart ? bpart[t * 6 + d] : INFINITY;
+            hi[d] = t < nbpart ? bpart[t * 6 + 3 + d] : -INFINITY;
+        }
+        wave_box(lo, hi);
+        if ((t & 63) == 0)
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                box[t >> 6][d] = lo[d];
+                box[t >> 6][3 + d] = hi[d];
+            }
+    }
     __syncthreads();
+    if (FIRST)
+        for (int w = 0; w < 4; w++)
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                lo[d] = fmin(lo[d], box[w][d]);
+                hi[d] = fmax(hi[d], box[w][3 + d]);
+            }
     for (int r = 0; r < kSortBlock / 256; r++) {
         const long long i = (long long)b * kSortBlock + r * 256 + t;
-        if (i < n) atomicAdd(&cnt[(keys[i] >> shift) & (kBins - 1)], 1);
+        if (i >= n) break;
+        unsigned key;
+        if (FIRST) keys[i] = key = cell_key(pts + 3 * i, lo, hi);
+        else key = keys[i];
+        atomicAdd(&cnt[(key >> shift) & (kBins - 1)], 1);
     }
     __syncthreads();
-    if (t < kBins) hist[t * nb + b] = cnt[t];
+    hist[t * nb + b] = cnt[t];
 }
 
-// exclusive scan of m counts in place (one workgroup of 1024): the counts
-// are read in coalesced passes of 1024, each scanned within wavefronts
-// (shuffles), then across the 16 wavefronts, plus the running total
-__global__ __launch_bounds__(1024) void radix_scan_kernel(int *v, int m) {
-    __shared__ int wsum[16];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    int carry = 0;
-    for (int base = 0; base < m; base += 1024) {
-        const int i = base + t;
-        const int x = i < m ? v[i] : 0;
-        int inc = x;
+// exclusive scan over the 256 threads of a workgroup; wsum: 4 ints of LDS
+__device__ __forceinline__ int scan256(int x, int *wsum, int &total) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int inc = x;
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int y = __shfl_up(inc, d);
-            if (lane >= d) inc += y;
-        }
-        if (lane == 63) wsum[wave] = inc;
-        __syncthreads();
-        int before = carry, total = carry;
-#pragma unroll
-        for (int w = 0; w < 16; w++) {
-            const int ws = wsum[w];
-            if (w < wave) before += ws;
-            total += ws;
-        }
-        if (i < m) v[i] = before + inc - x;
-        carry = total;
-        __syncthreads();  // wsum is rewritten by the next pass
+    for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(inc, d);
+        if (lane >= d) inc += y;
     }
+    __syncthreads();  // wsum may still be read from an earlier scan
+    if (lane == 63) wsum[wave] = inc;
+    __syncthreads();
+    int before = 0;
+    total = 0;
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+        if (w < wave) before += wsum[w];
+        total += wsum[w];
+    }
+    return before + inc - x;
 }
 
-// stable scatter by digit: element order within a digit is kept
+// workgroup d: exclusive scan of digit d's counts over the radix blocks in
+// place, their sum into digits[d]
+__global__ __launch_bounds__(256) void radix_scan_kernel(int *hist, int nb, int *digits) {
+    __shared__ int wsum[4];
+    int *v = hist + (long long)blockIdx.x * nb;
+    int carry = 0;
+    for (int base = 0; base < nb; base += 256) {
+        const int i = base + threadIdx.x, x = i < nb ? v[i] : 0;
+        int total;
+        const int before = scan256(x, wsum, total);
+        if (i < nb) v[i] = carry + before;
+        carry += total;
+    }
+    if (threadIdx.x == 0) digits[blockIdx.x] = carry;
+}
+
+// stable scatter by digit: element order within a digit is kept.  LAST: the
+// output is the permutation and the points in its order
+template <bool LAST>
 __global__ __launch_bounds__(256) void radix_scatter_kernel(const unsigned *kin, const int *iin, int n,
-                                                            int shift, const int *off, unsigned *kout,
-                                                            int *iout) {
+                                                            int shift, const int *hist,
+                                                            const int *digits, unsigned *kout, int *iout,
+                                                            const double *pts, double *spts) {
     __shared__ int wcnt[4][kBins];
     __shared__ int run[kBins];
+    __shared__ int wsum[4];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, b = blockIdx.x, nb = gridDim.x;
-    if (t < kBins) run[t] = off[t * nb + b];
+    int total;
+    run[t] = scan256(digits[t], wsum, total) + hist[(long long)t * nb + b];
     const unsigned long long below = (1ull << lane) - 1ull;
     for (int r = 0; r < kSortBlock / 256; r++) {
         const long long i = (long long)b * kSortBlock + r * 256 + t;
         const bool valid = i < n;
         const unsigned key = valid ? kin[i] : 0u;
         const int dig = (int)((key >> shift) & (kBins - 1));
-        int rank = 0;
 #pragma unroll
-        for (int v = 0; v < kBins; v++) {
-            const unsigned long long m = __ballot(valid && dig == v);
-            if (dig == v) rank = __popcll(m & below);
-            if (lane == 0) wcnt[wave][v] = __popcll(m);
+        for (int w = 0; w < 4; w++) wcnt[w][t] = 0;
+        // lanes of this wavefront with the same digit
+        unsigned long long same = __ballot(valid);
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const unsigned long long m = __ballot((dig >> k) & 1);
+            same &= (dig >> k) & 1 ? m : ~m;
         }
-        __syncthreads();  // wcnt written, run up to date
+        const int rank = __popcll(same & below);
+        __syncthreads();  // wcnt cleared, run up to date
+        if (valid && rank == 0) wcnt[wave][dig] = __popcll(same);
+        __syncthreads();
         if (valid) {
             int pos = run[dig] + rank;
             for (int w = 0; w < wave; w++) pos += wcnt[w][dig];
-            kout[pos] = key;
-            iout[pos] = iin[i];
+            const int idx = LAST ? iin[i] : (int)i;
+            iout[pos] = idx;
+            if (LAST) {
+#pragma unroll
+                for (int d = 0; d < 3; d++) spts[3 * (long long)pos + d] = pts[3 * (long long)idx + d];
+            } else {
+                kout[pos] = key;
+            }
         }
         __syncthreads();  // every thread has read run and wcnt
-        if (t < kBins) run[t] += wcnt[0][t] + wcnt[1][t] + wcnt[2][t] + wcnt[3][t];
-        __syncthreads();  // run updated before the next round's wcnt is written
+        run[t] += wcnt[0][t] + wcnt[1][t] + wcnt[2][t] + wcnt[3][t];
     }
-}
-
-// sorted points and their caller indices
-__global__ __launch_bounds__(256) void gather_points_kernel(const double *pts, const int *idx, int n,
-                                                            double *spts, int *perm) {
-    const long long j = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (j >= n) return;
-    const int i = idx[j];
-    perm[j] = i;
-#pragma unroll
-    for (int d = 0; d < 3; d++) spts[3 * j + d] = pts[3 * (long long)i + d];
 }
 
 // One workgroup per row tile: bounding box of its valid rows, the granules (4
@@ -219,13 +307,7 @@ __global__ __launch_bounds__(256) void block_list_kernel(TileArgs a) {
             }
     }
     for (int b = t; b < a.nblk; b += 256) live[b] = 0u;
-#pragma unroll
-    for (int w = 32; w > 0; w >>= 1)
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            lo[d] = fmin(lo[d], __shfl_xor(lo[d], w));
-            hi[d] = fmax(hi[d], __shfl_xor(hi[d], w));
-        }
+    wave_box(lo, hi);
     if (lane == 0)
 #pragma unroll
         for (int d = 0; d < 3; d++) {
@@ -303,65 +385,38 @@ __global__ __launch_bounds__(256) void block_list_kernel(TileArgs a) {
     if (t < (-base & 3)) list[base + t] = -1;  // four per N-tile and K-step
 }
 
-// exclusive prefix sum of the tiles' live group counts, toff[0 .. n]
-__global__ __launch_bounds__(256) void tile_offsets_kernel(const int *cnt, int n, int *toff) {
-    __shared__ int s[256];
-    const int t = threadIdx.x;
-    const int per = (n + 255) / 256;
-    const int beg = min(n, t * per), end = min(n, beg + per);
-    int sum = 0;
-    for (int i = beg; i < end; i++) sum += cnt[i];
-    s[t] = sum;
-    __syncthreads();
-    for (int w = 1; w < 256; w <<= 1) {
-        const int x = t >= w ? s[t - w] : 0;
-        __syncthreads();
-        s[t] += x;
-        __syncthreads();
-    }
-    int run = s[t] - sum;
-    for (int i = beg; i < end; i++) {
-        toff[i] = run;
-        run += cnt[i];
-    }
-    if (t == 255) toff[n] = s[255];
-}
-
 }  // namespace
-
-hipError_t launch_tile_offsets(const int *cnt, int ntiles, int *toff, hipStream_t s) {
-    if (ntiles <= 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(tile_offsets_kernel, dim3(1), dim3(256), 0, s, cnt, ntiles, toff);
-    return hipGetLastError();
-}
 
 int sort_scratch_ints(int n) {
     const int nb = (n + kSortBlock - 1) / kSortBlock;
-    return 4 * n + kBins * nb;  // two key/index ping-pong pairs + digit counts
+    return 3 * n + kBins * nb + kBins;  // keys twice, indices, digit counts
 }
 
 hipError_t launch_sort_points(const double *pts, int n, double *spts, int *perm, double *bpart,
                               int *scratch, hipStream_t s) {
     if (n <= 0) return hipSuccess;
+    if (n <= kSmallSort) {
+        const int threads = n <= 128 ? 64 : n <= 512 ? 256 : 1024;
+        hipLaunchKernelGGL(small_sort_kernel, dim3(1), dim3(threads), 0, s, pts, n, spts, perm);
+        return hipGetLastError();
+    }
     const int nb = (n + kSortBlock - 1) / kSortBlock;
     unsigned *k0 = (unsigned *)scratch, *k1 = k0 + n;
-    int *i0 = scratch + 2 * n, *i1 = i0 + n, *hist = scratch + 4 * n;
+    int *i1 = scratch + 2 * (long long)n, *hist = i1 + n, *digits = hist + (long long)kBins * nb;
     const int npart = n < 256 * 256 ? (n + 255) / 256 : 256;
     hipLaunchKernelGGL(bbox_partial_kernel, dim3(npart), dim3(256), 0, s, pts, n, bpart);
-    hipLaunchKernelGGL(cell_key_kernel, dim3((n + 255) / 256), dim3(256), 0, s, pts, n,
-                       (const double *)bpart, npart, k0, i0);
-    for (int pass = 0; pass < 4; pass++) {
-        const int shift = 4 * pass;
-        unsigned *kin = pass & 1 ? k1 : k0, *kout = pass & 1 ? k0 : k1;
-        int *iin = pass & 1 ? i1 : i0, *iout = pass & 1 ? i0 : i1;
-        hipLaunchKernelGGL(radix_hist_kernel, dim3(nb), dim3(256), 0, s, (const unsigned *)kin, n,
-                           shift, hist);
-        hipLaunchKernelGGL(radix_scan_kernel, dim3(1), dim3(1024), 0, s, hist, kBins * nb);
-        hipLaunchKernelGGL(radix_scatter_kernel, dim3(nb), dim3(256), 0, s, (const unsigned *)kin,
-                           (const int *)iin, n, shift, (const int *)hist, kout, iout);
-    }
-    hipLaunchKernelGGL(gather_points_kernel, dim3((n + 255) / 256), dim3(256), 0, s, pts,
-                       (const int *)i0, n, spts, perm);
+    hipLaunchKernelGGL(radix_hist_kernel<true>, dim3(nb), dim3(256), 0, s, pts, (const double *)bpart,
+                       npart, k0, n, 0, hist);
+    hipLaunchKernelGGL(radix_scan_kernel, dim3(kBins), dim3(256), 0, s, hist, nb, digits);
+    hipLaunchKernelGGL(radix_scatter_kernel<false>, dim3(nb), dim3(256), 0, s, (const unsigned *)k0,
+                       (const int *)nullptr, n, 0, (const int *)hist, (const int *)digits, k1, i1,
+                       (const double *)nullptr, (double *)nullptr);
+    hipLaunchKernelGGL(radix_hist_kernel<false>, dim3(nb), dim3(256), 0, s, (const double *)nullptr,
+                       (const double *)nullptr, 0, k1, n, 8, hist);
+    hipLaunchKernelGGL(radix_scan_kernel, dim3(kBins), dim3(256), 0, s, hist, nb, digits);
+    hipLaunchKernelGGL(radix_scatter_kernel<true>, dim3(nb), dim3(256), 0, s, (const unsigned *)k1,
+                       (const int *)i1, n, 8, (const int *)hist, (const int *)digits,
+                       (unsigned *)nullptr, perm, pts, spts);
     return hipGetLastError();
 }
 

@@ -1,0 +1,87 @@
+"""GPU: point counts around the edges of the point sort and the plane sums.
+
+Up to 2,048 points one workgroup sorts them (64, 256 or 1,024 threads), more
+go through two radix passes of 1,024-point blocks; a plane of more than 65,536
+points is summed in parts.
+"""
+import numpy as np
+import pytest
+
+from conftest import rel_err
+from oracle import oracle, sph
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ring():
+    from gimic_amd import synth
+    s = synth.ring12()
+    ctx = s.context(screening=1e-8)
+    yield s, ctx
+    ctx.close()
+
+
+def _points(n, seed=1):
+    return np.random.default_rng(seed).uniform(-6.0, 6.0, (n, 3))
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 63, 64, 65, 128, 129, 512, 513, 2047, 2048, 2049, 3072, 5000])
+def test_point_counts_around_the_sort(ring, n):
+    s, ctx = ring
+    pts = _points(n)
+    pts[n // 2] = pts[0]  # a repeated point
+    print("case sort of", n, flush=True)
+    J = ctx.jtensor(pts, precision="fp64")
+    sub = np.unique(np.r_[0, n // 2, n - 1, np.random.default_rng(n).integers(0, n, 20)])
+    ref = oracle.jtensor(s.arrays(), sph.to_cartesian(s.dens, s.shell_l), pts[sub], screening=1e-8)
+    # the scale of the error floor is that of the whole set
+    scale = max(np.linalg.norm(J, axis=1).max(), 1e-300)
+    e = np.linalg.norm(J[sub] - ref, axis=1) / np.maximum(np.linalg.norm(ref, axis=1), 1e-3 * scale)
+    assert e.max() <= 1e-10, e.max()
+    assert np.array_equal(ctx.jtensor(pts, precision="fp64"), J)
+
+
+def test_points_in_one_cell_and_not_a_number(ring):
+    """all points in one Morton cell (equal keys keep their order), and a point
+    that is not a number (it gets a cell, and only its own tensor)"""
+    s, ctx = ring
+    for n in (100, 3000):
+        pts = np.tile([1.0, 0.5, 0.3], (n, 1))
+        J = ctx.jtensor(pts, precision="fp64")
+        assert np.array_equal(J, np.tile(J[0], (n, 1)))
+        pts = _points(n, 3)
+        J = ctx.jtensor(pts, precision="fp64")
+        bad = pts.copy()
+        bad[n // 3, 1] = np.nan
+        K = ctx.jtensor(bad, precision="fp64")
+        keep = np.arange(n) != n // 3
+        assert rel_err(K[keep], J[keep]).max() <= 1e-12
+
+
+@pytest.mark.parametrize("sizes", [[65535], [65536], [200000], [150000, 3, 0, 90000]])
+def test_plane_sums_in_parts(ring, sizes):
+    s, ctx = ring
+    rng = np.random.default_rng(len(sizes))
+    planes = []
+    for n in sizes:
+        planes.append(dict(points=rng.uniform(-5.0, 5.0, (n, 3)), weights=rng.uniform(0.0, 1.0, n),
+                           normal=[0.6, 0.0, 0.8], bfield=[0.0, 0.0, 1.0], center=[0.0, 0.0, 0.0]))
+    print("case plane sums", sizes, flush=True)
+    flux, mod, acid, jt = ctx.flux_planes(planes, return_jt=True, modulus=True, acid=True)
+    at = 0
+    for k, p in enumerate(planes):
+        n = sizes[k]
+        T = jt[at:at + n].reshape(-1, 3, 3).transpose(0, 2, 1)
+        at += n
+        jv = T @ np.asarray(p["bfield"])
+        v = p["weights"] * (jv @ np.asarray(p["normal"]))
+        m = p["weights"] * np.sign(jv @ np.asarray(p["normal"])) * np.linalg.norm(jv, axis=1)
+        for got, w in ((flux[k], v), (mod[k], m)):
+            ref = np.array([w.sum(), w[w > 0].sum(), w[w <= 0].sum()])
+            # rounding of sums of n terms in another order
+            assert np.abs(got - ref).max() <= 1e-15 * max(n, 1) ** 0.5 * 100 * np.abs(w).sum() + 1e-300
+        assert (acid[k] > 0.0) == (n > 0)
+    plain = ctx.flux_planes(planes)
+    assert np.array_equal(plain, flux)
+    assert np.array_equal(ctx.flux_planes(planes, acid=True)[1], acid)
