@@ -352,6 +352,7 @@ struct gimic_ctx {
     // (variant 0 here), walks the screening block lists
     int mixed_variant = -1;
     int mixed_split = 0;  // N-split count of the pre-split kernel (0: by workgroup count)
+    bool split_fixed = false;  // set by the caller: small launches keep it too
     // block-list statistics (gimic_ctx_set_tile_stats): tiles, sum n, sum n^2, rows per tile
     bool tile_stats = false;
     double tile_acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
@@ -627,6 +628,11 @@ constexpr int kMinTileRows = 64;
 constexpr size_t kSmallF64Points = 131072;
 int f64_tile_rows(size_t points) { return points <= kSmallF64Points ? 64 : kWgRows; }
 
+// Ranges of a row tile that the assembly adds by itself (launch_split_sum
+// otherwise): it reads them one after another, so fewer where its workgroups
+// do not fill the chip
+constexpr int kMaxAssemblySplit = 16, kMaxSmallSplit = 4, kSmallAssembly = 65536;
+
 // Arena bytes one Scratch-mode chunk of `rows` rows carves (every carve
 // rounded to 256 bytes), with `split` N-ranges per row tile
 size_t scratch_eval_bytes(const gimic_ctx *c, int prec, int nmatset, size_t rows, int split) {
@@ -878,29 +884,44 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
         // wants some 32 K-steps in each, though, and a tile of a small basis has
         // few: then half as many pairs (ring12, 64,000 points: 0.183 ms at
         // 2048 against 0.227 at 4096 and 0.266 at 8192)
-        auto plan = [&](int wg_rows, int tile_cols, int want_split = 0) {
+        // A tuned mixed count is that of a full chip: launches of few tiles take
+        // more ranges (1,331 points of the 60-atom cage, 6 tiles, dealt to all
+        // XCDs besides: 1.93 to 0.43 ms; 29,791 points 2.92 to 2.34 ms).
+        auto plan = [&](int wg_rows, int tile_cols, int want_split = 0, bool at_least = false) {
             ca.ntiles = c->ncol_pad / tile_cols;
             const long long per = (long long)(rows / wg_rows) * nmatset, nt = ca.ntiles;
             auto pairs = [&](long long n) { return std::max<long long>(1, (n + per - 1) / per); };
             int nsplit = (int)std::min(nt, pairs(prec == GIMIC_PREC_FP64 ? 4096 : 8192));
             if (prec == GIMIC_PREC_FP64)
                 nsplit = (int)std::min<long long>(nsplit, std::max(pairs(2048), nt * nt / 128));
-            if (want_split > 0) nsplit = std::min(want_split, ca.ntiles);
+            if (want_split > 0)
+                nsplit = (int)std::min<long long>(
+                    at_least ? std::max<long long>(want_split, pairs(1024)) : want_split, nt);
             if (scratch) nsplit = std::min(nsplit, kScratchMaxSplit);
-            ca.tiles_per_split = (ca.ntiles + nsplit - 1) / nsplit;
-            ca.nsplit = (ca.ntiles + ca.tiles_per_split - 1) / ca.tiles_per_split;
+            const int per_split = (ca.ntiles + nsplit - 1) / nsplit;
+            ca.nsplit = (ca.ntiles + per_split - 1) / per_split;
+            // a few tiles of a large basis: one N-tile a range still leaves CUs
+            // idle and a long walk over K, so K is split too, four steps or more
+            // a range
+            ca.ksplit = 1;
+            if (prec == GIMIC_PREC_FP64 && !scratch && ca.nsplit == ca.ntiles)
+                ca.ksplit = (int)std::max<long long>(
+                    1, std::min<long long>(std::min<long long>(8, nt / 4), 1024 / (per * nt)));
+            ca.nsplit *= ca.ksplit;
             grow(W.part, (size_t)nmatset * ca.nsplit * kNQ * rows * 8, false);
             ca.part = W.part.as<double>();
         };
         auto plan_variant = [&](int variant, int split = -1) {
-            if (split < 0) split = msplit;
             if (variant == 0) plan(f64_tile_rows(n_c), kNT);
-            else plan(mixed_tile_rows(variant), kMx2Cols / kNMat, split);
+            else
+                plan(mixed_tile_rows(variant), kMx2Cols / kNMat, split < 0 ? msplit : split,
+                     split < 0 && !c->split_fixed && !scratch);
         };
         // row-major partial sums from the mixed kernels, written whole by the launch
         const int tr64 = f64_tile_rows(n_c);
         auto run = [&](int variant, int split = -1) {
             plan_variant(variant, split);
+            ca.spread = split < 0;
             ca.compressed = !dense;
             ca.tile_rows = tr64;
             if (variant == 0) hip_check(launch_contract_f64(ca, st), "contract_f64");
@@ -927,7 +948,12 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
         auto finalize = [&](int variant) {
             FinalizeArgs fa{};
             fa.part = W.part.as<double>();
-            fa.nsplit = ca.nsplit;
+            fa.nsplit = fa.nsum = ca.nsplit;
+            if (ca.spread && ca.nsplit > (rows <= kSmallAssembly ? kMaxSmallSplit : kMaxAssemblySplit)) {
+                hip_check(launch_split_sum(W.part.as<double>(), nmatset, ca.nsplit,
+                                           (long long)kNQ * rows, st), "split_sum");
+                fa.nsum = 1;
+            }
             fa.part_rows = variant != 0 ? 1 : 0;
             fa.rows = rows;
             fa.npts = n_c;
@@ -979,7 +1005,9 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
             // fastest run counts.  The fastest candidate replaces the
             // default only when it is faster by more than 1%: near-ties are
             // noise, and a chance pick of a near-tie ran 4% slower in the
-            // steady state than the default on the 60-atom cage.
+            // steady state than the default on the 60-atom cage.  Candidates
+            // are timed at their own split and plain order whatever the size of
+            // this chunk: the choice is for every later one.
             const int cand[][2] = {{3, 4}, {4, 4}, {5, 4}, {8, 2}, {8, 4}, {8, 8},
                                    {9, 2}, {9, 4}, {9, 8}};
             c->tune_log.clear();
@@ -1812,6 +1840,7 @@ int gimic_ctx_set_mixed_kernel(gimic_ctx *c, int variant, int split) {
         if (split < 0) throw Error(GIMIC_EINVAL, "split count must be >= 0");
         c->mixed_variant = variant == 0 ? -1 : variant;
         c->mixed_split = variant >= 3 ? split : 0;
+        c->split_fixed = variant != 0;
         for (auto &e : c->tune_ms) e = 0.f;
     });
 }

@@ -75,6 +75,8 @@ __device__ __forceinline__ void radial_parts(const EvalArgs &a, const DevShell &
 // with the list, its FP64 scan 6% faster (basis 1.66 to 1.35 ms: the pass holds
 // three rows instead of seven, so screened pairs cost more there).
 constexpr int kCandMinShells = 400, kCandMinShellsF64 = 64;
+// Workgroups a launch should have before they take 32 rows each
+constexpr int kMinBasisGroups = 512;
 // Shells whose candidacy the staged kernel settles per pass of its loop
 constexpr int kCandChunk = 1024;
 // LDS beyond the image and the block positions: candidate list, bounding
@@ -500,7 +502,10 @@ hipError_t launch_basis_eval(const EvalArgs &a, int mode, hipStream_t s) {
     EvalArgs b = a;
     const size_t row_bytes = (size_t)a.lda * (f64 ? 32 : 2 * kAParts + 12);
     if (row_bytes > kMaxRowBytes || !a.compressed) return hipErrorInvalidValue;
-    b.tile_points = 32;
+    // fewer where the launch would leave CUs idle
+    int tp = 32;
+    while (tp > 1 && (a.npts + tp - 1) / tp < kMinBasisGroups) tp >>= 1;
+    b.tile_points = tp;
     b.lds_image = std::max<size_t>(36 * 1024, row_bytes);
     // the image, the group positions (16-byte aligned) and, for bases of
     // kCandMinShells (F64) shells or more, the candidate list

@@ -20,7 +20,9 @@
 // or two workgroups) is visited, in granules of four functions, the K of one
 // v_mfma_f64_16x16x4: an N-tile is four of the tile's live granules (16
 // functions x 7 matrices), a K-step another four (lane group g owns the g-th).
-// The N-tiles of a row tile are split evenly over nsplit ranges.
+// The N-tiles of a row tile are split evenly over ranges and, where a launch
+// has too few of these for the chip, the K-steps over ksplit ranges too (the
+// sums are linear in Y): nsplit pairs of ranges in all.
 //
 // The matrices are the first MFMA operand and the points the second, so the
 // lane (g, c) of an output block holds Y of the four functions of granule g
@@ -44,7 +46,8 @@
 // operand load redirected to one cached block it ran within 1% of that.
 //
 // Workgroup order: the ranges of a row tile run back to back on one XCD
-// (workgroup i goes to XCD i mod 8), so its basis rows come from that L2.
+// (workgroup i goes to XCD i mod 8), so its basis rows come from that L2; with
+// few tiles they go to all XCDs in turn (a.spread).
 #include "device_common.h"
 
 namespace gimic {
@@ -70,20 +73,26 @@ __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, c = lane & 15;
     const int parts = a.tile_rows / kRows;  // workgroups that share a list and a range
-    const int xcd = blockIdx.x & 7, slot = (blockIdx.x >> 3) / parts;
-    const int ntile = a.rows / a.tile_rows, per_set = (ntile + 7) / 8 * a.nsplit;
-    const int set = slot / per_set, split = slot % a.nsplit;
-    const int rtile = slot % per_set / a.nsplit * 8 + xcd;
+    const int part = (a.spread ? blockIdx.x : blockIdx.x >> 3) % parts;
+    const int slot = (a.spread ? blockIdx.x : blockIdx.x >> 3) / parts;
+    const int ntile = a.rows / a.tile_rows, tiles = a.spread ? ntile : (ntile + 7) / 8;
+    const int set = slot / (tiles * a.nsplit), split = slot % a.nsplit;
+    const int rt = slot % (tiles * a.nsplit) / a.nsplit;
+    const int rtile = a.spread ? rt : rt * 8 + (blockIdx.x & 7);
     if (rtile >= ntile) return;
     const int *K4 = a.klist + (size_t)rtile * a.nblk * 8;
     const int nks = (a.kcount[rtile] + 3) >> 2;
-    const int e0 = (int)((long long)split * nks / a.nsplit);
-    const int e1 = (int)((long long)(split + 1) * nks / a.nsplit);
+    // this workgroup's N-tiles e0 .. e1 and, of each, kn K-steps from k0 on
+    const int nsn = a.nsplit / a.ksplit, sn = split / a.ksplit, sk = split % a.ksplit;
+    const int e0 = (int)((long long)sn * nks / nsn), e1 = (int)((long long)(sn + 1) * nks / nsn);
+    const int k0 = (int)((long long)sk * nks / a.ksplit);
+    const int kn = (int)((long long)(sk + 1) * nks / a.ksplit) - k0;
+    const int *KK = K4 + 4 * k0;
 
     const int ng = a.lda / 4;  // granules per row; index ng: the zero blocks
     const v2d *B = (const v2d *)(a.b64 + (size_t)set * f64_set_elems(a.lda));
     const size_t rowst = (size_t)(ng + 1) * kUnits;
-    const int rin = (blockIdx.x >> 3) % parts * kRows + wave * 16 + c;
+    const int rin = part * kRows + wave * 16 + c;
     const size_t row = (size_t)rtile * a.tile_rows + rin;
     // the point's values and gradients: dense, or compressed to the tile's granules
     const bool cmp = a.compressed;
@@ -113,7 +122,7 @@ __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
 #pragma unroll
     for (int i = 0; i < kNQ; i++) q[i] = 0.0;
 
-    if (e0 < e1) {
+    if (e0 < e1 && kn > 0) {
         // The K-steps of all N-tiles form one sequence t.  During step t the
         // workgroup computes on buffer t mod 3, stores step t + 2 (loaded
         // during step t - 1) and loads step t + 3; one barrier ends a step.
@@ -135,7 +144,7 @@ __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
         nxt = *(const int4 *)(K4 + 4 * min(fe + 1, e1 - 1));
         v2d st[4];
         const int wv = tid >> 6;
-        int kent = K4[wv];
+        int kent = KK[wv];
         auto source = [&] {
             const int x = __builtin_amdgcn_readfirstlane(kent);
             return (const char *)(B + (size_t)(x < 0 ? ng : x >> 13) * rowst);
@@ -143,13 +152,13 @@ __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
         auto load = [&](const char *src) {
 #pragma unroll
             for (int i = 0; i < 4; i++) st[i] = *(const v2d *)(src + noff[i]);
-            if (++fk == nks) {  // on to the next N-tile (past the last: it again)
+            if (++fk == kn) {  // on to the next N-tile (past the last: it again)
                 fk = 0;
                 fe = min(fe + 1, e1 - 1);
                 offsets();
                 nxt = *(const int4 *)(K4 + 4 * min(fe + 1, e1 - 1));
             }
-            kent = K4[4 * fk + wv];  // for the next step's load
+            kent = KK[4 * fk + wv];  // for the next step's load
         };
         auto put = [&](v2d *b) {
             if (lane < kUnits)
@@ -162,8 +171,8 @@ __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
         load(source());
         put(buf + nx1);
         load(source());
-        v4d an = *(const v4d *)(A + acol(K4[g]));
-        int xa = K4[(nks > 1 ? 4 : 0) + g];  // the next K-step's granule
+        v4d an = *(const v4d *)(A + acol(KK[g]));
+        int xa = KK[(kn > 1 ? 4 : 0) + g];  // the next K-step's granule
         __syncthreads();
         v2d b0[kNMat];
 #pragma unroll
@@ -178,13 +187,13 @@ __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
             v4d acc[kNMat];
 #pragma unroll
             for (int m = 0; m < kNMat; m++) acc[m] = v4d{0.0, 0.0, 0.0, 0.0};
-            for (int ks = 0; ks < nks; ks++) {
+            for (int ks = 0; ks < kn; ks++) {
                 const v4d av = an;
                 v2d b1[kNMat];
 #pragma unroll
                 for (int m = 0; m < kNMat; m++) b1[m] = buf[cur + rd1 + m * 128];
                 an = *(const v4d *)(A + acol(xa));
-                xa = K4[4 * (ks + 2 < nks ? ks + 2 : ks + 2 - nks < nks ? ks + 2 - nks : 0) + g];
+                xa = KK[4 * (ks + 2 < kn ? ks + 2 : ks + 2 - kn < kn ? ks + 2 - kn : 0) + g];
 #pragma unroll
                 for (int m = 0; m < kNMat; m++)
                     acc[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(b0[m].x, av[0], acc[m], 0, 0, 0);
@@ -255,12 +264,15 @@ __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
 
 hipError_t launch_contract_f64(const ContractArgs &a, hipStream_t s) {
     if ((a.tile_rows != 64 && a.tile_rows != 128) || a.rows % a.tile_rows || a.lda % 32 ||
-        a.ncol_pad != a.lda)
+        a.ncol_pad != a.lda || a.ksplit < 1 || a.nsplit % a.ksplit)
         return hipErrorInvalidValue;
-    const long long nwg = 8LL * ((a.rows / a.tile_rows + 7) / 8) * a.nsplit * a.nmatset *
+    ContractArgs b = a;
+    const int ntile = a.rows / a.tile_rows;
+    b.spread = a.spread && ntile < kSpreadTiles;
+    const long long nwg = (b.spread ? ntile : 8LL * ((ntile + 7) / 8)) * a.nsplit * a.nmatset *
                           (a.tile_rows / 64);
     if (nwg > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(contract_f64_kernel, dim3((unsigned)nwg), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(contract_f64_kernel, dim3((unsigned)nwg), dim3(256), 0, s, b);
     return hipGetLastError();
 }
 

@@ -67,7 +67,8 @@
 // their lists mostly agree, and spread enough that its workgroups do not
 // all stream the same B groups at once.  On the 60-atom cage, runs of 2, 4
 // and 32 tiles were 0.3%, 1.3% and 12% slower; runs of 8 were 1-5% slower
-// (two boxes).
+// (two boxes).  A launch of few tiles deals its workgroups to all XCDs in turn
+// instead (a.spread).
 #include "device_common.h"
 
 namespace gimic {
@@ -211,13 +212,14 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, c = lane & 15;
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int groups = tile_groups(a.rows / kRows);  // row tiles per XCD
+    const int xcd = blockIdx.x & 7, slot = a.spread ? blockIdx.x : blockIdx.x >> 3;
+    const int groups = a.spread ? a.rows / kRows : tile_groups(a.rows / kRows);  // row tiles per XCD
     const int per_set = groups * a.nsplit;
     const int set = slot / per_set;
     const int split = slot % a.nsplit;
     const int jt = (slot % per_set) / a.nsplit;
-    const int rtile = (jt / kTileRun) * 8 * kTileRun + xcd * kTileRun + jt % kTileRun;
+    const int rtile =
+        a.spread ? jt : (jt / kTileRun) * 8 * kTileRun + xcd * kTileRun + jt % kTileRun;
     if (rtile >= a.rows / kRows) return;  // padding of the last run
     const size_t row0 = (size_t)rtile * kRows;
     const int lda = a.lda;
@@ -481,11 +483,13 @@ static hipError_t launch_one(const ContractArgs &a, hipStream_t s) {
     }
     if (a.rows % rows || a.lda % 32 || a.ncol_pad != a.lda || a.ntiles * kNu != a.ncol_pad)
         return hipErrorInvalidValue;
-    const long long groups = tile_groups(a.rows / rows);
-    const long long nwg = 8 * groups * a.nsplit * a.nmatset;
+    ContractArgs b = a;
+    b.spread = a.spread && a.rows / rows < kSpreadTiles;
+    const long long groups = b.spread ? a.rows / rows : 8LL * tile_groups(a.rows / rows);
+    const long long nwg = groups * a.nsplit * a.nmatset;
     if (nwg > 0x7fffffffLL) return hipErrorInvalidValue;
     hipLaunchKernelGGL((contract_mx2_kernel<NBUF, KRB, WAVES>), dim3((unsigned)nwg),
-                       dim3(64 * WAVES), lds, s, a);
+                       dim3(64 * WAVES), lds, s, b);
     return hipGetLastError();
 }
 

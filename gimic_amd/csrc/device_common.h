@@ -117,7 +117,8 @@ hipError_t upload_basis_tables(const double *sph, int nsph, hipStream_t s);
 struct ContractArgs {
     int rows, lda, ncol_pad;
     long long gplane;    // elements between the three gradient planes
-    int ntiles, nsplit, tiles_per_split;
+    int ntiles, nsplit;
+    int ksplit;       // FP64 kernel: K-ranges among the nsplit (1: N-ranges only)
     int nmatset;      // density sets packed side by side (7 matrices each)
     const double *pts;   // chunk points (3 per row, npts valid rows)
     int npts;
@@ -132,6 +133,7 @@ struct ContractArgs {
     // (pre-split kernels) or 4 (FP64 kernel), four per N-tile and K-step;
     // split s of a tile takes N-tiles [s * count / nsplit, (s+1) * count / nsplit)
     int nblk, tile_rows;  // tile_rows: FP64 kernel only
+    int spread;           // workgroups of fewer than kSpreadTiles row tiles to all XCDs in turn
     const int *kcount, *klist;
     int compressed;      // FP64 kernel: rows as in EvalArgs
 };
@@ -143,6 +145,10 @@ constexpr int kF64PairElems = kNMat * 16;
 __host__ __device__ constexpr size_t f64_set_elems(int lda) {
     return (size_t)(lda / 4 + 1) * (size_t)(lda / 4 + 1) * kF64PairElems;
 }
+// Row tiles from which the ranges of one tile stay on one XCD: with fewer, some
+// XCDs would have one tile more than others or none (24 points of the 60-atom
+// cage, one tile: the FP64 call takes 496 us on one XCD, 120 on all)
+constexpr int kSpreadTiles = 64;
 // FP64 kernel: row tiles of a.tile_rows = 64 or 128 points (a.rows a multiple)
 hipError_t launch_contract_f64(const ContractArgs &a, hipStream_t s);
 // Pre-split variant: both operands arrive as BF16 parts, the right operand in
@@ -202,6 +208,7 @@ struct FinalizeArgs {
     const double *part;  // [nmatset][nsplit][kNQ][rows], or [nmatset][nsplit][rows][kNQ] if part_rows
     int part_rows;
     int nsplit, rows, npts, nmatset;
+    int nsum;            // of the nsplit blocks of a set, the first nsum are added
     const double *pts;   // chunk points in row order
     const int *perm;     // caller index (within the chunk) of each row, or null
     const long long *pidx;  // output index of each caller index (subset runs), or null
@@ -217,6 +224,8 @@ struct FinalizeArgs {
     double *contrib_acid; // ACID contribution w_p dT^2 or null
 };
 hipError_t launch_finalize(const FinalizeArgs &a, hipStream_t s);
+// per set, the sum of nsplit blocks of `count` partial sums, in order, into the first
+hipError_t launch_split_sum(double *part, int nmatset, int nsplit, long long count, hipStream_t s);
 // Shielding (per nucleus) and magnetizability sums per point partition:
 // out[(k * npart + p) * 5 + q], k < nnuc shielding of nucleus k, k == nnuc
 // magnetizability; q = sum w s_x, s_y, s_z, positive part, negative part.

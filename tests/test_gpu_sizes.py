@@ -85,3 +85,36 @@ def test_plane_sums_in_parts(ring, sizes):
     plain = ctx.flux_planes(planes)
     assert np.array_equal(plain, flux)
     assert np.array_equal(ctx.flux_planes(planes, acid=True)[1], acid)
+
+
+@pytest.fixture(scope="module")
+def cage():
+    from gimic_amd import synth
+    s = synth.cage60()
+    ctx = s.context(screening=1e-8)
+    yield s, ctx
+    ctx.close()
+
+
+@pytest.mark.parametrize("n", [1, 5, 64, 65, 257, 4000])
+def test_small_launches_split_over_k_and_all_xcds(cage, n):
+    """few row tiles of a large basis: N- and K-ranges on every XCD, their sums
+    added by a launch of their own"""
+    s, ctx = cage
+    # spread over the whole cage, so the tiles list most functions
+    pts = np.random.default_rng(n).uniform(-8.0, 8.0, (n, 3))
+    print("case cage60 small launch", n, flush=True)
+    J = ctx.jtensor(pts, precision="fp64")
+    sub = np.random.default_rng(2).integers(0, n, min(n, 16))
+    ref = oracle.jtensor(s.arrays(), sph.to_cartesian(s.dens, s.shell_l), pts[sub], screening=1e-8)
+    scale = np.linalg.norm(J, axis=1).max()
+    e = np.linalg.norm(J[sub] - ref, axis=1) / np.maximum(np.linalg.norm(ref, axis=1), 1e-3 * scale)
+    assert e.max() <= 1e-10, e.max()
+    assert np.array_equal(ctx.jtensor(pts, precision="fp64"), J)
+    M = ctx.jtensor(pts, precision="mixed")
+    assert rel_err(M, J).max() <= 1e-5
+    assert np.array_equal(ctx.jtensor(pts, precision="mixed"), M)
+    # the same points in a full launch: other tiles, fewer ranges
+    far = np.random.default_rng(9).uniform(-8.0, 8.0, (60000, 3))
+    K = ctx.jtensor(np.concatenate([pts, far]), precision="fp64")[:n]
+    assert rel_err(K, J).max() <= 1e-12
