@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstdio>
 #include <condition_variable>
@@ -615,6 +616,15 @@ struct EvalWork {
 constexpr int kDefaultVariant = 9, kDefaultSplit = 4;
 constexpr int kScratchMaxSplit = 32;
 
+// How much faster the mixed kernels of 256-row tiles have to be than those of
+// 128 rows to be taken: 1.06, or 1.11 for the few tiles of a small chunk.
+// Screening follows the tile, so the results of the two differ by some 2e-8 of
+// their norm.  The lines lie where the two were equally fast (within 1% in
+// nine of ten of 230 timed sizes) when wavefronts waited for each K-step's
+// list entries, which cost the 8-wavefront kernels twice as much: a faster
+// kernel does not move a program's results between the two
+float wide_tile_gain(int points) { return points <= 16384 ? 1.11f : 1.06f; }
+
 // Row tile of the mixed kernels: 128 rows (4 wavefronts x 32), 256 (4 x 64
 // or 8 x 32)
 int mixed_tile_rows(int variant) { return variant == 5 || variant >= 8 ? 256 : 128; }
@@ -917,11 +927,12 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
                 plan(mixed_tile_rows(variant), kMx2Cols / kNMat, split < 0 ? msplit : split,
                      split < 0 && !c->split_fixed && !scratch);
         };
-        // row-major partial sums from the mixed kernels, written whole by the launch
+        // row-major partial sums from the mixed kernels
         const int tr64 = f64_tile_rows(n_c);
-        auto run = [&](int variant, int split = -1) {
+        auto run = [&](int variant, int split = -1, bool plain = false) {
             plan_variant(variant, split);
             ca.spread = split < 0;
+            ca.plain = plain;
             ca.compressed = !dense;
             ca.tile_rows = tr64;
             if (variant == 0) hip_check(launch_contract_f64(ca, st), "contract_f64");
@@ -949,11 +960,16 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
             FinalizeArgs fa{};
             fa.part = W.part.as<double>();
             fa.nsplit = fa.nsum = ca.nsplit;
+            const int *kc = variant != 0 && !ca.plain ? W.kcount.as<int>() : nullptr;
+            const int tr = variant != 0 ? mixed_tile_rows(variant) : tr64;
             if (ca.spread && ca.nsplit > (rows <= kSmallAssembly ? kMaxSmallSplit : kMaxAssemblySplit)) {
                 hip_check(launch_split_sum(W.part.as<double>(), nmatset, ca.nsplit,
-                                           (long long)kNQ * rows, st), "split_sum");
+                                           rows, kc, tr, st), "split_sum");
                 fa.nsum = 1;
+                kc = nullptr;
             }
+            fa.kcount = kc;
+            fa.tile_rows = tr;
             fa.part_rows = variant != 0 ? 1 : 0;
             fa.rows = rows;
             fa.npts = n_c;
@@ -1002,19 +1018,19 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
             // share each row tile's A through L2, fewer give each workgroup
             // more N-tiles to amortise its start, and fewer partial sums to
             // assemble); every candidate is timed three times and its
-            // fastest run counts.  The fastest candidate replaces the
-            // default only when it is faster by more than 1%: near-ties are
-            // noise, and a chance pick of a near-tie ran 4% slower in the
-            // steady state than the default on the 60-atom cage.  Candidates
-            // are timed at their own split and plain order whatever the size of
-            // this chunk: the choice is for every later one.
-            const int cand[][2] = {{3, 4}, {4, 4}, {5, 4}, {8, 2}, {8, 4}, {8, 8},
-                                   {9, 2}, {9, 4}, {9, 8}};
-            c->tune_log.clear();
-            float best = 0.f, def_ms = 0.f;
-            int best_v = -1, best_split = 0;
-            for (auto &cv : cand) {
-                const int v = cv[0], sp = cv[1];
+            // fastest run counts.  The row tile decides which functions are
+            // screened together, and so the last digits of the results, and
+            // is chosen first, in the plain form (every range written); then
+            // the kernel and split of that tile, as they will run.  Within a
+            // tile the default is replaced only by a candidate faster by more
+            // than 1%: near-ties are noise, and a chance pick of a near-tie ran
+            // 4% slower in the steady state than the default on the 60-atom
+            // cage.  Candidates are timed at their own split and plain order
+            // whatever the size of this chunk: the choice is for every later one.
+            const int cand[][2] = {{3, 4}, {4, 4}, {9, 2}, {9, 4}, {9, 8},
+                                   {5, 4}, {8, 2}, {8, 4}, {8, 8}};
+            const int ntile = 5;  // candidates that stand for their tile
+            auto time = [&](int v, int sp, bool plain) {
                 hipEvent_t e0, e1;
                 hip_check(hipEventCreate(&e0), "hipEventCreate");
                 hip_check(hipEventCreate(&e1), "hipEventCreate");
@@ -1023,7 +1039,7 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
                 for (int rep = 0; rep < 3; rep++) {
                     hip_check(hipEventRecord(e0, st), "hipEventRecord");
                     eval(v);
-                    run(v, sp);
+                    run(v, sp, plain);
                     finalize(v);
                     hip_check(hipEventRecord(e1, st), "hipEventRecord");
                     hip_check(hipEventSynchronize(e1), "hipEventSynchronize");
@@ -1033,21 +1049,33 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
                 }
                 (void)hipEventDestroy(e0);
                 (void)hipEventDestroy(e1);
+                return ms;
+            };
+            float fine = FLT_MAX, wide = FLT_MAX;  // the fastest of each row tile
+            for (int k = 0; k < ntile; k++) {
+                float &b = mixed_tile_rows(cand[k][0]) == 128 ? fine : wide;
+                b = std::min(b, time(cand[k][0], cand[k][1], true));
+            }
+            const int tile = fine <= wide_tile_gain(n_c) * wide ? 128 : 256;
+            c->tune_log.clear();
+            float best = FLT_MAX, def_ms = FLT_MAX;
+            for (auto &cv : cand) {
+                const int v = cv[0], sp = cv[1];
+                if (mixed_tile_rows(v) != tile) continue;
+                const float ms = time(v, sp, false);
                 c->tune_log.push_back({v * 100 + sp, ms});
                 if (c->tune_ms[v - 1] == 0.f || ms < c->tune_ms[v - 1]) c->tune_ms[v - 1] = ms;
                 if (v == kDefaultVariant && sp == kDefaultSplit) def_ms = ms;
-                if (best_v < 0 || ms < best) {
+                if (ms < best) {
                     best = ms;
-                    best_v = v;
-                    best_split = sp;
+                    c->mixed_variant = v;
+                    c->mixed_split = sp;
                 }
             }
-            if (def_ms > 0.f && def_ms <= 1.01f * best) {
-                best_v = kDefaultVariant;
-                best_split = kDefaultSplit;
+            if (def_ms <= 1.01f * best) {
+                c->mixed_variant = kDefaultVariant;
+                c->mixed_split = kDefaultSplit;
             }
-            c->mixed_variant = best_v;
-            c->mixed_split = best_split;
             mv = c->mixed_variant;
             msplit = c->mixed_split;
             if (mode == EvalMode::Reserve) {

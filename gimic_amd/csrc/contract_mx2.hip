@@ -31,13 +31,30 @@
 // wavefront's MFMA chains run while the other waits on a dependency or a
 // load, and each staged block feeds twice the rows.
 //
+// Nothing in the K-loop waits for a load of its own step: list entries are
+// read a step before their first use, by each lane its own group's (the
+// copy takes them from four lanes), the B fragments of a column block while
+// the one before it is multiplied, and the A fragments a step ahead; the
+// first blocks and fragments of the next N-tile are loaded during the
+// epilogue.  When each step waited for its entries and, with NBUF = 3, for
+// the copy that was to stay in flight, 256 planes of the 30-atom sheet took
+// 2 x 1.54 ms of contraction against 2 x 1.18, the open-shell sheet (2620
+// functions, 4 launches) 6.87 against 6.22 each, the 60-atom cage (2.1M
+// points) 72.7 against 69.6 in all.  The cage runs at 1183 TFLOP/s of listed
+// work, the rate of a large library product on this chip.  Small bases are
+// bound by the epilogue (40% of the sheet's time) and the A rows' way from
+// memory.  An epilogue on transposed blocks (a lane holds functions of one
+// point: half the instructions, the same sums bit for bit) was no faster for
+// the sheet and 4% slower for the cage.
+//
 // Per-point partial sums.  After the butterfly over the 16 columns of a lane
 // group every lane holds all kNQ sums of its row; lane c writes sums c and
 // c + 16 (FP64) to the row-major partial buffer [set][split][row][kNQ],
 // 16 lanes of a group covering 128 contiguous bytes: an atomic store for
 // the workgroup's first N-tile, no-return atomic adds for the later ones
-// (one thread's atomics on one address keep program order), zeros from a
-// workgroup without N-tiles.  Each address belongs to one lane of one
+// (one thread's atomics on one address keep program order).  A tile of fewer
+// N-tiles than nsplit fills one range with each, and the assembly reads only
+// the filled ones (in the plain form the others write zeros).  Each address belongs to one lane of one
 // workgroup, which adds its N-tiles in order, so the sums are the same, bit
 // for bit, on every run, no clearing pass is needed, and no LDS holds them
 // (three K-step buffers fit with 256-row tiles).
@@ -47,7 +64,7 @@
 // tile (tiles.hip: the groups of the listed 32-function blocks in which
 // screening leaves some function of the tile non-zero), on both sides of
 // the product: an N-tile is four of them (their 32 functions x 7 matrices),
-// the N-tiles are split evenly over the nsplit workgroups of the row tile,
+// the N-tiles are split evenly over the row tile's filled ranges,
 // and the K-loop walks the same groups, four per K-step (an MFMA's K of
 // 32).  On the 60-atom cage that is a fifth fewer (N-tile, K-step) pairs
 // than N-tiles of whole 32-function blocks.  Each lane group of a wavefront
@@ -81,68 +98,63 @@ constexpr int kCB = kCols / 16;             // 14 column blocks
 constexpr int kBlk = kMx2BlockElems;        // BF16 per block / LDS buffer
 constexpr size_t kBufBytes = (size_t)kBlk * 2;
 // A K-step's LDS buffer is [group slot j][part][column][8]: slot j holds one
-// K-group (kBParts x 3584 bytes), copied in kPPG 1 KiB pieces per slot, the
-// last one partial when the slot does not fill it (three parts: 10752
-// bytes, eleven pieces, the last for lanes 0-31).  Lane l of piece t of a
-// slot fills unit u = 64 t + l of the slot: [part p][column], column =
-// matrix m * 32 + 8 * N-slot + n.  As 224 = 7 * 32, the 32-unit chunk
-// w = u / 32 = 2 t + l / 32 is p * 7 + m, and column % 32 = l % 32, so the
+// K-group (kBParts x 3584 bytes = kSlotHalves half pieces of 512 bytes), and
+// the buffer is copied in 1 KiB pieces, 64 lanes x 16 bytes, without regard
+// to the slots: piece q holds half pieces 2q (lanes 0-31) and 2q + 1, and
+// half piece h is chunk w = h % kSlotHalves of slot h / kSlotHalves.  A
+// chunk holds 32 units [part p][column], column = matrix m * 32 + 8 * N-slot
+// + n: as 224 = 7 * 32, chunk w is p * 7 + m, and column % 32 = l % 32, so the
 // lane's N-slot (l / 8) % 4 and function n = l % 8 are the same in every
-// piece: the unit is element (p * 7 + m) * 64 + 8 n of the pair block of the
-// slot's K-group and the lane's N-group, at lane offset nlo + 128 t
+// piece: the unit is element w * 64 + 8 n of the pair block of the slot's
+// K-group and the lane's N-group
 constexpr int kGroupBytes = kMx2GroupElems * 2;
-constexpr int kPPG = (kGroupBytes + 1023) / 1024;           // pieces per group slot
-constexpr int kLastLanes = (kGroupBytes - (kPPG - 1) * 1024) / 16;  // lanes of its last piece
-constexpr int kPieces = 4 * kPPG;                            // pieces per K-step
+constexpr int kSlotHalves = kGroupBytes / 512;
+constexpr int kPieces = 4 * kGroupBytes / 1024;             // pieces per K-step
 constexpr int kPartElems = kCols * 8;                       // BF16 per part of a group
-static_assert(4 * kGroupBytes <= kBlk * 2 && kGroupBytes % 16 == 0, "piece layout");
+static_assert(kPieces * 1024 == kBlk * 2 && kGroupBytes % 512 == 0, "piece layout");
 
-// pieces a wavefront copies of each block: wavefront w copies w, w + WAVES, ...
+// Pieces a wavefront copies of each block: wavefront w copies w, w + WAVES,
+// ...; what is beyond the block repeats its last piece (the same bytes to the
+// same place), so that every wavefront issues the same number of copies
+// with no branch between them.  With branches the compiler's own count of the
+// loads in flight held for none of them, and it waited for the whole copy at
+// the top of every K-step
 template <int WAVES>
 constexpr int pieces_max() { return (kPieces + WAVES - 1) / WAVES; }
-__device__ __forceinline__ int pieces_of(int wave, int waves) {
-    return (kPieces - wave + waves - 1) / waves;
-}
 
 typedef __attribute__((address_space(3))) void lds_void;
 
-__device__ __forceinline__ int pick4(int4 v, int i) {
-    return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
-}
-
 // the lane's offset, within a K-group's row of pair blocks, of its unit in
-// piece 0 of a slot (fixed for an N-tile): pair block gn of its N-slot's
-// group (ngn, a zero block, for padding), chunk l / 32, function l % 8
-__device__ __forceinline__ int lane_offset(int4 en, int ngn, int lane) {
-    const int x = pick4(en, (lane >> 3) & 3);
+// chunk 0 (fixed for an N-tile): pair block gn of its N-slot's group, entry x
+// (ngn, a zero block, for padding), function l % 8
+__device__ __forceinline__ int lane_offset(int x, int ngn, int lane) {
     const int gn = x < 0 ? ngn : x >> 12;
-    return gn * kMx2PairElems + (lane >> 5) * 64 + (lane & 7) * 8;
+    return gn * kMx2PairElems + (lane & 7) * 8;
 }
 
-// piece i of this wavefront's share of a K-step's buffer (64 lanes x 16
-// bytes per instruction, LDS base in M0): piece q = kPPG j + t fills bytes
-// [1024 t, 1024 t + 1024) of slot j from the row of K-group ek[j] >> 12
-// (ek[j] < 0: the zero row nkg), each lane from its offset nlo + 128 t
+// piece i of this wavefront's share of a K-step's buffer (LDS base in M0):
+// the half pieces' rows are those of K-group ek[j] >> 12 of their slots j
+// (ek[j] < 0: the zero row nkg; lane 16 j holds entry j)
 template <int WAVES>
-__device__ __forceinline__ void stage_piece_k8(const __bf16 *Bset, size_t rowst, int nkg, int4 ek,
+__device__ __forceinline__ void stage_piece_k8(const __bf16 *Bset, size_t rowst, int nkg, int ek,
                                                int nlo, unsigned char *buf, int wave, int lane,
                                                int i) {
-    const int piece = wave + WAVES * i;
-    const int j = piece / kPPG, t = piece - kPPG * j;
-    const int v = pick4(ek, j);
-    const __bf16 *src = Bset + (size_t)(v < 0 ? nkg : v >> 12) * rowst + 128 * t + nlo;
-    if (t < kPPG - 1 || lane < kLastLanes)
-        __builtin_amdgcn_global_load_lds((const void *)src,
-                                         (lds_void *)(buf + j * kGroupBytes + t * 1024), 16, 0, 0);
+    const int piece = min(wave + WAVES * i, kPieces - 1);
+    auto src = [&](int h) {
+        const int j = h / kSlotHalves, v = __builtin_amdgcn_readlane(ek, 16 * j);
+        return (size_t)(v < 0 ? nkg : v >> 12) * rowst + 64 * (h - kSlotHalves * j);
+    };
+    const size_t lo = src(2 * piece), hi = src(2 * piece + 1);
+    __builtin_amdgcn_global_load_lds((const void *)(Bset + (lane < 32 ? lo : hi) + nlo),
+                                     (lds_void *)(buf + piece * 1024), 16, 0, 0);
 }
 
 template <int WAVES>
-__device__ __forceinline__ void stage_block_k8(const __bf16 *Bset, size_t rowst, int nkg, int4 ek,
+__device__ __forceinline__ void stage_block_k8(const __bf16 *Bset, size_t rowst, int nkg, int ek,
                                                int nlo, unsigned char *buf, int wave, int lane) {
-    const int np = pieces_of(wave, WAVES);
 #pragma unroll
     for (int i = 0; i < pieces_max<WAVES>(); i++)
-        if (i < np) stage_piece_k8<WAVES>(Bset, rowst, nkg, ek, nlo, buf, wave, lane, i);
+        stage_piece_k8<WAVES>(Bset, rowst, nkg, ek, nlo, buf, wave, lane, i);
 }
 
 // One step of a transposing sum over the 16 lanes of a DPP row: lanes whose
@@ -169,19 +181,17 @@ __device__ __forceinline__ void row16_xsum(float (&v)[32], int c) {
     xsum_step<2, 0xB1>(v, (c & 1) != 0);
 }
 
-// the part products of split order <= 2, smallest first (three parts each:
-// lh, mm, hl, mh, hm, hh)
-__device__ __forceinline__ v4f mfma_split(const v8bf (&a)[kAParts], const v8bf (&b)[kBParts],
-                                          v4f acc) {
+// the part products (ia, ib) of split order <= 2, smallest first (three
+// parts each: lh, mm, hl, mh, hm, hh)
+template <typename F>
+__device__ __forceinline__ void for_split_products(F &&f) {
 #pragma unroll
     for (int ord = 2; ord >= 0; ord--)
 #pragma unroll
         for (int ia = kAParts - 1; ia >= 0; ia--) {
             const int ib = ord - ia;
-            if (ib >= 0 && ib < kBParts)
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ia], b[ib], acc, 0, 0, 0);
+            if (ib >= 0 && ib < kBParts) f(ia, ib);
         }
-    return acc;
 }
 
 }  // namespace
@@ -229,14 +239,16 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
     // -1 pads the last four (zero right operand)
     const int *K8 = a.klist + (size_t)rtile * a.nblk * 4;
     const int nq = (a.kcount[rtile] + 3) >> 2;
+    const int ranges = a.plain ? a.nsplit : filled_ranges(a.kcount[rtile], a.nsplit);
+    if (split >= ranges) return;
     // This tile's basis rows hold only its live groups, in list order
     // (EvalArgs): A and the gradients are addressed by list position
-    const size_t wcols = (size_t)8 * a.kcount[rtile];  // functions per row
-    const size_t arow = kAParts * wcols;                // BF16 per split row
+    // (a tile's rows are below 4 GiB: 32-bit offsets from uniform bases)
+    const unsigned wcols = 8u * a.kcount[rtile];  // functions per row
+    const unsigned arow = kAParts * wcols;        // BF16 per split row
     const __bf16 *Atile = a.as3 + row0 * lda * kAParts;
     const float *Gtile = a.g32 + row0 * lda * 3;
-    const size_t gpl = (size_t)kRows * wcols;           // gradient plane stride
-    const int np = pieces_of(wave, WAVES);  // pieces this wavefront copies per block
+    const unsigned gpl = kRows * wcols;           // gradient plane stride
     // this workgroup's partial sums, row-major [row][kNQ]
     double *pout = a.part + ((size_t)set * a.nsplit + split) * kNQ * rows;
     // the epilogue's point coordinates, once per workgroup (visible after
@@ -249,52 +261,69 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
     }
 
     // lane (g, c) of row block rb: row wave*32 + rb*16 + c, k-group entry g of the K-step
-    const __bf16 *Arow = Atile + (size_t)(wave * 16 * kRB + c) * arow;
-    auto a_off = [&](int4 v) -> size_t {  // this lane's group of a K-step, in BF16 of a row
-        const int x = g == 0 ? v.x : g == 1 ? v.y : g == 2 ? v.z : v.w;
-        return x < 0 ? 0 : (size_t)(x & 4095) * (8 * kAParts);
+    const unsigned lrow = (wave * 16 * kRB + c) * arow;
+    auto a_off = [&](int x) -> unsigned {  // this lane's group of a K-step, in BF16 of a row
+        return x < 0 ? 0u : (unsigned)(x & 4095) * (8 * kAParts);
     };
+    auto a_frag = [&](unsigned ao, int rb, int p) -> v8bf {
+        return *(const v8bf *)((const char *)(Atile + rb * 16 * arow) + 2 * (lrow + ao) + 16 * p);
+    };
+    // entry g of K-step ks (the last K-step beyond the end)
+    auto entry = [&](int ks) -> int { return K8[4 * min(ks, nq - 1) + g]; };
     // pair blocks of this density set: rows of K-groups (nkg: the zero row)
     // of ngn + 1 N-groups (ngn: the zero block)
     const int nkg = lda / 8, ngn = a.ncol_pad / 8;
     const size_t rowst = (size_t)(ngn + 1) * kMx2PairElems;
     const __bf16 *Bset = a.bs3 + (size_t)set * mx2_set_elems(lda, a.ncol_pad);
-    const int e0 = (int)((long long)split * nq / a.nsplit);
-    const int e1 = (int)((long long)(split + 1) * nq / a.nsplit);
+    const int e0 = (int)((long long)split * nq / ranges);
+    const int e1 = (int)((long long)(split + 1) * nq / ranges);
+    if (e0 == e1) {  // plain only: the range's sums are zero
+        for (int i = tid; i < kRows * kNQ; i += 64 * WAVES) pout[row0 * kNQ + i] = 0.0;
+        return;
+    }
+    const int q0 = entry(0), q1 = entry(1), q2 = entry(2);
+    // what an N-tile's first K-steps need: the first NBUF - 1 blocks, and the A
+    // fragments of step 0
+    v8bf an[kRB][kAParts];
+    auto start_tile = [&](int nlo) {
+        stage_block_k8<WAVES>(Bset, rowst, nkg, q0, nlo, bbuf, wave, lane);
+        if (NBUF == 3 && nq > 1)
+            stage_block_k8<WAVES>(Bset, rowst, nkg, q1, nlo, bbuf + kBufBytes, wave, lane);
+        const unsigned ao = a_off(q0);
+#pragma unroll
+        for (int rb = 0; rb < kRB; rb++)
+#pragma unroll
+            for (int p = 0; p < kAParts; p++)
+                an[rb][p] = a_frag(ao, rb, p);
+    };
+    // entry of this lane's N-slot, (lane / 8) % 4, of this and the next N-tile
+    const int nslot = (lane >> 3) & 3;
+    int xn = K8[4 * e0 + nslot], xnext = K8[4 * min(e0 + 1, nq - 1) + nslot];
+    int nlo = lane_offset(xn, ngn, lane);
+    start_tile(nlo);
 
     for (int e = e0; e < e1; e++) {
-        const int4 en = *(const int4 *)(K8 + 4 * e);  // this N-tile's four groups
-        const int nlo = lane_offset(en, ngn, lane);
         v4f acc[kRB][kCB];
 #pragma unroll
         for (int rb = 0; rb < kRB; rb++)
 #pragma unroll
             for (int cb = 0; cb < kCB; cb++) acc[rb][cb] = v4f{0.f, 0.f, 0.f, 0.f};
 
-        const int4 q0 = *(const int4 *)K8, q1 = *(const int4 *)(K8 + (nq > 1 ? 4 : 0));
-        stage_block_k8<WAVES>(Bset, rowst, nkg, q0, nlo, bbuf, wave, lane);
-        if (NBUF == 3 && nq > 1)
-            stage_block_k8<WAVES>(Bset, rowst, nkg, q1, nlo, bbuf + kBufBytes, wave, lane);
-        v8bf an[kRB][kAParts];
-        {
-            const size_t ao = a_off(q0);
-#pragma unroll
-            for (int rb = 0; rb < kRB; rb++)
-#pragma unroll
-                for (int p = 0; p < kAParts; p++)
-                    an[rb][p] = *(const v8bf *)(Arow + rb * 16 * arow + ao + p * 8);
-        }
         __builtin_amdgcn_s_waitcnt(kWaitAll);
         __syncthreads();
 
-        // groups of the next step's A fragments and of the next step's copy,
-        // read one K-step early (the end-of-step wait covers the scalar loads)
-        int4 ent_a = q1;
-        int4 ent_c = *(const int4 *)(K8 + 4 * min(NBUF - 1, nq - 1));
+        // groups of the next step's A fragments and of this step's copy: each
+        // lane reads its group's entry a K-step before the copy needs it (the
+        // first load of a step, so the end-of-step wait covers it), and the
+        // copy takes the four of its step from lanes 0, 16, 32 and 48
+        int ent_a = q1, ent_c = NBUF == 3 ? q2 : q1;
         for (int ks = 0; ks < nq; ks++) {
-            const int4 ea = ent_a, ec = ent_c;
-            ent_a = *(const int4 *)(K8 + 4 * min(ks + 2, nq - 1));
-            ent_c = *(const int4 *)(K8 + 4 * min(ks + NBUF, nq - 1));
+            // opaque: otherwise the scalar copies are taken right after the
+            // load, which stalls the step for the load's latency
+            asm volatile("" : "+v"(ent_c));
+            const int ea = ent_a, ec = ent_c;
+            ent_c = entry(ks + NBUF);
+            ent_a = NBUF == 3 ? ec : ent_c;
             v8bf as[kRB][kAParts];
 #pragma unroll
             for (int rb = 0; rb < kRB; rb++)
@@ -312,13 +341,12 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
             // works through them.  With NBUF = 3 the copy comes after all A
             // loads (column blocks 3 to 13), so that waiting for "all but the
             // last copy" covers the A loads.
-            const bool more = ks + 1 < nq;
             constexpr int kALoads = kAParts * kRB;
             constexpr int kCopyFrom = NBUF == 3 ? kCB - kPW : 0;
             static_assert(NBUF != 3 || (kALoads + 1) / 2 <= kCopyFrom, "A loads must precede the copy");
             const int ahead = ks + NBUF - 1;
             const bool copy = NBUF == 3 || ahead < nq;
-            const size_t aoff = a_off(ea);
+            const unsigned aoff = a_off(ea);
             unsigned char *cbuf = bbuf + (size_t)(ahead % NBUF) * kBufBytes;
             const __bf16 *cur = (const __bf16 *)(bbuf + (size_t)(ks % NBUF) * kBufBytes);
             v8bf bf[2][kBParts];
@@ -331,22 +359,31 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
 #pragma unroll
             for (int cb = 0; cb < kCB; cb++) {
                 const int sl = cb & 1;
-                if (cb + 1 < kCB) {
-                    const int off = g * kMx2GroupElems + ((cb + 1) * 16 + c) * 8;
+                bool first = true;
+                for_split_products([&](int ia, int ib) {
 #pragma unroll
-                    for (int p = 0; p < kBParts; p++)
-                        bf[sl ^ 1][p] = *(const v8bf *)(cur + p * kPartElems + off);
-                }
+                    for (int rb = 0; rb < kRB; rb++)
+                        acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            as[rb][ia], bf[sl][ib], acc[rb][cb], 0, 0, 0);
+                    if (!first) return;
+                    first = false;
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (cb + 1 < kCB) {
+                        const int off = g * kMx2GroupElems + ((cb + 1) * 16 + c) * 8;
 #pragma unroll
-                for (int j = 2 * cb; j < 2 * cb + 2; j++)
-                    if (more && j < kALoads)
-                        an[j / kAParts][j % kAParts] = *(const v8bf *)(
-                            Arow + (j / kAParts) * 16 * arow + aoff + (j % kAParts) * 8);
-                if (copy && cb >= kCopyFrom && cb - kCopyFrom < np)
-                    stage_piece_k8<WAVES>(Bset, rowst, nkg, ec, nlo, cbuf, wave, lane, cb - kCopyFrom);
-                __builtin_amdgcn_sched_barrier(0);
+                        for (int p = 0; p < kBParts; p++)
+                            bf[sl ^ 1][p] = *(const v8bf *)(cur + p * kPartElems + off);
+                    }
 #pragma unroll
-                for (int rb = 0; rb < kRB; rb++) acc[rb][cb] = mfma_split(as[rb], bf[sl], acc[rb][cb]);
+                    for (int j = 2 * cb; j < 2 * cb + 2; j++)
+                        if (j < kALoads)
+                            an[j / kAParts][j % kAParts] =
+                                a_frag(aoff, j / kAParts, j % kAParts);
+                    if (copy && cb >= kCopyFrom && cb - kCopyFrom < kPW)
+                        stage_piece_k8<WAVES>(Bset, rowst, nkg, ec, nlo, cbuf, wave, lane,
+                                              cb - kCopyFrom);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
                 __builtin_amdgcn_sched_barrier(0);
             }
             // this wavefront's A loads and the copy of block ks+1 have landed
@@ -355,15 +392,9 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
             // visible and nobody reads the buffer the next copy overwrites
             // (a bare s_barrier: __syncthreads would add a fence that waits
             // for every outstanding load, the early copy included)
-            if (NBUF == 3) {
-                // np is uniform per wavefront: kPW, or kPW - 1 when the
-                // pieces do not split evenly over the wavefronts
-                if (np == kPW) __builtin_amdgcn_s_waitcnt(wait_all_but(kPW));
-                else __builtin_amdgcn_s_waitcnt(wait_all_but(kPW > 1 ? kPW - 1 : 0));
-            } else {
-                __builtin_amdgcn_s_waitcnt(kWaitAll);
-            }
+            __builtin_amdgcn_s_waitcnt(NBUF == 3 ? wait_all_but(kPW) : kWaitAll);
             __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
         }
         // no copy may still be writing a buffer that the next N-tile's
         // first copies reuse
@@ -378,37 +409,49 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
         // The global loads (phi parts and gradients) of each row are issued
         // one row ahead, so their latency overlaps the previous row's work.
         float R[2][3];
-        int acol[2];  // column of the lane's function in this tile's basis rows
+        unsigned acol[2];  // column of the lane's function in this tile's basis rows
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            const int x = pick4(en, 2 * h + (c >> 3));
-            const int fn = x < 0 ? 0 : (x >> 12) * 8 + (c & 7);
+            const int x = __shfl(xn, 8 * (2 * h + (c >> 3)));
+            const unsigned fn = x < 0 ? 0 : (x >> 12) * 8 + (c & 7);
             acol[h] = x < 0 ? 0 : (x & 4095) * 8 + (c & 7);
 #pragma unroll
-            for (int d = 0; d < 3; d++) R[h][d] = a.rf32[(size_t)d * a.ncol_pad + fn];
+            for (int d = 0; d < 3; d++) R[h][d] = (a.rf32 + (size_t)d * a.ncol_pad)[fn];
         }
         constexpr int kIt = 4 * kRB;  // rows per lane: it = 4 rb + r
         auto row_of = [&](int it) { return wave * 16 * kRB + (it >> 2) * 16 + 4 * g + (it & 3); };
-        __bf16 pc[2][kAParts], pn[2][kAParts];
-        float Gc[2][3], Gn[2][3];
+        constexpr int kAhead = KRB == 4 ? 1 : 2;  // rows whose loads are in flight beside the one in work
+        __bf16 pv[kAhead + 1][2][kAParts];
+        float Gv[kAhead + 1][2][3];
         auto load_row = [&](int it, __bf16 (&pv)[2][kAParts], float (&Gv)[2][3]) {
-            const size_t rl = row_of(it);
+            if (it >= kIt) return;
+            const unsigned rl = row_of(it);
 #pragma unroll
             for (int h = 0; h < 2; h++) {
-                const __bf16 *pe = Atile + rl * arow + (acol[h] >> 3) * (8 * kAParts) + (acol[h] & 7);
+                const unsigned pe = rl * arow + (acol[h] >> 3) * (8 * kAParts) + (acol[h] & 7);
 #pragma unroll
-                for (int k = 0; k < kAParts; k++) pv[h][k] = pe[8 * k];
-                const size_t gi = rl * wcols + acol[h];
+                for (int k = 0; k < kAParts; k++)
+                    pv[h][k] = *(const __bf16 *)((const char *)Atile + 2 * pe + 16 * k);
+                const unsigned gi = rl * wcols + acol[h];
 #pragma unroll
-                for (int d = 0; d < 3; d++) Gv[h][d] = Gtile[d * gpl + gi];
+                for (int d = 0; d < 3; d++)
+                    Gv[h][d] = *(const float *)((const char *)(Gtile + d * (size_t)gpl) + 4 * gi);
             }
         };
-        load_row(0, pc, Gc);
+#pragma unroll
+        for (int it = 0; it < kAhead; it++) load_row(it, pv[it], Gv[it]);
+        if (e + 1 < e1) {
+            xn = xnext;
+            xnext = K8[4 * min(e + 2, nq - 1) + nslot];
+            nlo = lane_offset(xn, ngn, lane);
+            start_tile(nlo);
+        }
 #pragma unroll
         for (int it = 0; it < kIt; it++) {
             const int rb = it >> 2, r = it & 3;
             {
-                if (it + 1 < kIt) load_row(it + 1, pn, Gn);
+                const int cur = it % (kAhead + 1), far = (it + kAhead) % (kAhead + 1);
+                load_row(it + kAhead, pv[far], Gv[far]);
                 const int rl = row_of(it);
                 const float rp[3] = {rps[3 * rl], rps[3 * rl + 1], rps[3 * rl + 2]};
                 float q[kNQ];
@@ -417,10 +460,10 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     // the basis value from its parts (three: exactly the FP32 value)
-                    float ph = (float)pc[h][0];
+                    float ph = (float)pv[cur][h][0];
 #pragma unroll
-                    for (int k = 1; k < kAParts; k++) ph += (float)pc[h][k];
-                    const float *G = Gc[h];
+                    for (int k = 1; k < kAParts; k++) ph += (float)pv[cur][h][k];
+                    const float *G = Gv[cur][h];
                     const float t0 = acc[rb][h][r] * ph;
                     q[0] += t0;
 #pragma unroll
@@ -455,19 +498,9 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
                     if (c + 16 < kNQ) unsafeAtomicAdd(o + c + 16, (double)s1);
                 }
             }
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-#pragma unroll
-                for (int k = 0; k < kAParts; k++) pc[h][k] = pn[h][k];
-#pragma unroll
-                for (int k = 0; k < 3; k++) Gc[h][k] = Gn[h][k];
-            }
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    // a workgroup without N-tiles still owns its rows' sums for this split
-    if (e0 == e1)
-        for (int i = tid; i < kRows * kNQ; i += 64 * WAVES) pout[row0 * kNQ + i] = 0.0;
 }
 
 template <int NBUF, int KRB, int WAVES>

@@ -134,6 +134,7 @@ struct ContractArgs {
     // split s of a tile takes N-tiles [s * count / nsplit, (s+1) * count / nsplit)
     int nblk, tile_rows;  // tile_rows: FP64 kernel only
     int spread;           // workgroups of fewer than kSpreadTiles row tiles to all XCDs in turn
+    int plain;            // mixed: every range of a tile writes its sums, without N-tiles zeros
     const int *kcount, *klist;
     int compressed;      // FP64 kernel: rows as in EvalArgs
 };
@@ -204,11 +205,19 @@ struct OperandArgs {
 hipError_t launch_operand_f64(const OperandArgs &a, double *out, hipStream_t s);
 hipError_t launch_operand_split(const OperandArgs &a, __bf16 *out, hipStream_t s);
 
+// Of the nsplit N-ranges of a mixed row tile with `groups` listed 8-function
+// groups, those that hold N-tiles (of four groups); the others write no sums
+__device__ __forceinline__ int filled_ranges(int groups, int nsplit) {
+    return min(nsplit, (groups + 3) >> 2);
+}
+
 struct FinalizeArgs {
     const double *part;  // [nmatset][nsplit][kNQ][rows], or [nmatset][nsplit][rows][kNQ] if part_rows
     int part_rows;
     int nsplit, rows, npts, nmatset;
     int nsum;            // of the nsplit blocks of a set, the first nsum are added
+    const int *kcount;   // mixed: of these, only the filled ranges of a row's tile (or null)
+    int tile_rows;       // rows per entry of kcount
     const double *pts;   // chunk points in row order
     const int *perm;     // caller index (within the chunk) of each row, or null
     const long long *pidx;  // output index of each caller index (subset runs), or null
@@ -224,8 +233,10 @@ struct FinalizeArgs {
     double *contrib_acid; // ACID contribution w_p dT^2 or null
 };
 hipError_t launch_finalize(const FinalizeArgs &a, hipStream_t s);
-// per set, the sum of nsplit blocks of `count` partial sums, in order, into the first
-hipError_t launch_split_sum(double *part, int nmatset, int nsplit, long long count, hipStream_t s);
+// per set, the sum of the nsplit blocks of partial sums, in order, into the
+// first (kcount: as in FinalizeArgs, for row-major partials)
+hipError_t launch_split_sum(double *part, int nmatset, int nsplit, int rows, const int *kcount,
+                            int tile_rows, hipStream_t s);
 // Shielding (per nucleus) and magnetizability sums per point partition:
 // out[(k * npart + p) * 5 + q], k < nnuc shielding of nucleus k, k == nnuc
 // magnetizability; q = sum w s_x, s_y, s_z, positive part, negative part.

@@ -22,13 +22,14 @@ __device__ __forceinline__ double eps3(int i, int j, int k) {
     return (double)((i - j) * (j - k) * (k - i)) * 0.5;
 }
 
-__global__ __launch_bounds__(256) void finalize_kernel(FinalizeArgs a) {
-    // row-major partials: the workgroup's 256 rows are 256 kNQ contiguous
+__global__ __launch_bounds__(64) void finalize_kernel(FinalizeArgs a) {
+    // row-major partials: the workgroup's 64 rows are 64 kNQ contiguous
     // doubles per (set, split), staged through LDS with coalesced 16-byte
     // loads (a thread's own row is 176 bytes: read directly, every load of
-    // a wavefront would touch 64 separate pieces)
-    __shared__ double2 stage[256 * kNQ / 2];
-    const int p = blockIdx.x * 256 + threadIdx.x;
+    // a wavefront would touch 64 separate pieces).  One wavefront a workgroup,
+    // so that none waits for another's loads
+    __shared__ double2 stage[64 * kNQ / 2];
+    const int p = blockIdx.x * 64 + threadIdx.x;
     const bool valid = p < a.npts;
     double r[3] = {0.0, 0.0, 0.0};
     long long o = 0;
@@ -39,16 +40,21 @@ __global__ __launch_bounds__(256) void finalize_kernel(FinalizeArgs a) {
         o = a.perm ? a.perm[p] : p;  // caller index of row p
         if (a.pidx) o = a.pidx[o];   // its place in the output arrays
     }
+    // blocks of partial sums of these rows (one tile's)
+    const int nsum =
+        a.kcount ? filled_ranges(a.kcount[blockIdx.x * 64 / a.tile_rows], a.nsum) : a.nsum;
     for (int set = 0; set < a.nmatset; set++) {
         double q[kNQ];
 #pragma unroll
         for (int i = 0; i < kNQ; i++) q[i] = 0.0;
-        for (int s = 0; s < a.nsum; s++) {
+        for (int s = 0; s < nsum; s++) {
             const double *src = a.part + ((size_t)set * a.nsplit + s) * kNQ * (size_t)a.rows;
             if (a.part_rows) {
-                const double2 *blk = (const double2 *)(src + (size_t)blockIdx.x * 256 * kNQ);
+                const double2 *blk = (const double2 *)(src + (size_t)blockIdx.x * 64 * kNQ);
                 __syncthreads();  // the previous (set, split) has been read out
-                for (int i = threadIdx.x; i < 256 * kNQ / 2; i += 256) stage[i] = blk[i];
+#pragma unroll
+                for (int i = 0; i < kNQ / 2; i++)
+                    stage[i * 64 + threadIdx.x] = blk[i * 64 + threadIdx.x];
                 __syncthreads();
 #pragma unroll
                 for (int j = 0; j < kNQ / 2; j++) {
@@ -279,29 +285,34 @@ hipError_t launch_fill_zero(double *p, size_t n, hipStream_t s) {
 // few rows are split over many ranges the assembly's one thread per row would
 // read them one after another (1,331 points of the 60-atom cage, 57 ranges: the
 // assembly alone 110 us against 9 + 6).
-__global__ __launch_bounds__(256) void split_sum_kernel(double *part, int nsplit, long long count) {
+__global__ __launch_bounds__(256) void split_sum_kernel(double *part, int nsplit, long long count,
+                                                        const int *kcount, int tile_rows) {
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i >= count) return;
     double *p = part + (long long)blockIdx.y * nsplit * count + i;
+    const int n = kcount ? filled_ranges(kcount[i / kNQ / tile_rows], nsplit) : nsplit;
     double v = 0.0;
 #pragma unroll 8
-    for (int s = 0; s < nsplit; s++) v += p[s * count];
+    for (int s = 0; s < n; s++) v += p[s * count];
     *p = v;
 }
 
-hipError_t launch_split_sum(double *part, int nmatset, int nsplit, long long count, hipStream_t s) {
+hipError_t launch_split_sum(double *part, int nmatset, int nsplit, int rows, const int *kcount,
+                            int tile_rows, hipStream_t s) {
+    const long long count = (long long)kNQ * rows;
     const long long n = (count + 255) / 256;
     if (count <= 0 || n > 0x7fffffffLL || nmatset > 65535) return hipErrorInvalidValue;
     hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)n, nmatset), dim3(256), 0, s, part, nsplit,
-                       count);
+                       count, kcount, tile_rows);
     return hipGetLastError();
 }
 
 hipError_t launch_finalize(const FinalizeArgs &a, hipStream_t s) {
     if (a.npts <= 0) return hipSuccess;
-    // row-major partials are read in whole workgroups of 256 rows
-    if (a.part_rows && (a.rows % 256 || a.npts > a.rows)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(finalize_kernel, dim3((a.npts + 255) / 256), dim3(256), 0, s, a);
+    // row-major partials are read in whole workgroups of 64 rows, of one tile each
+    if (a.npts > a.rows || (a.part_rows && a.rows % 64)) return hipErrorInvalidValue;
+    if (a.kcount && (!a.part_rows || a.tile_rows % 64)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(finalize_kernel, dim3((a.npts + 63) / 64), dim3(64), 0, s, a);
     return hipGetLastError();
 }
 

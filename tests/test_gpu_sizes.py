@@ -118,3 +118,20 @@ def test_small_launches_split_over_k_and_all_xcds(cage, n):
     far = np.random.default_rng(9).uniform(-8.0, 8.0, (60000, 3))
     K = ctx.jtensor(np.concatenate([pts, far]), precision="fp64")[:n]
     assert rel_err(K, J).max() <= 1e-12
+
+
+@pytest.mark.parametrize("variant,split", [(3, 4), (4, 1), (5, 4), (8, 2), (9, 1), (9, 8)])
+@pytest.mark.parametrize("n", [1, 127, 129, 256, 257, 1000])
+def test_mixed_tiles_with_fewer_n_tiles_than_ranges(ring, n, variant, split):
+    """near and far points in one set: the row tiles list from none to all of
+    the ring's functions, so N-ranges stay empty in some; the mixed path's 1e-5,
+    of the largest tensor (the far ones vanish)"""
+    s, _ = ring
+    pts = _points(n)
+    pts[::2] *= 1.0 + 12.0 * np.arange(len(pts[::2]))[:, None] / n
+    print("case ring12 mixed", variant, split, n, flush=True)
+    with s.context(screening=1e-8) as ctx:
+        J = ctx.jtensor(pts, precision="fp64")
+        ctx.set_mixed_kernel(variant, split)
+        M = ctx.jtensor(pts, precision="mixed")
+    assert np.abs(M - J).max() <= 1e-5 * np.abs(J).max()
