@@ -933,6 +933,18 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
             plan_variant(variant, split);
             ca.spread = split < 0;
             ca.plain = plain;
+            // longest lists first, where a launch has more workgroups than fit
+            // the chip at once (4 to 6 us for the order)
+            const int tr = variant == 0 ? tr64 : mixed_tile_rows(variant), nt = rows / tr;
+            const long long wgs =
+                (long long)nt * ca.nsplit * nmatset * (variant == 0 ? tr / 64 : 1);
+            ca.order = nullptr;
+            if (!plain && nt >= kSpreadTiles && wgs > (variant == 0 ? 512 : 256)) {
+                int2 *order = (int2 *)W.sortscr.as<int>();  // the sort is done with it
+                hip_check(launch_tile_order(ca.kcount, nt, nblk * (variant == 0 ? 8 : 4), order, st),
+                          "tile_order");
+                ca.order = order;
+            }
             ca.compressed = !dense;
             ca.tile_rows = tr64;
             if (variant == 0) hip_check(launch_contract_f64(ca, st), "contract_f64");
@@ -1028,7 +1040,7 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
             // cage.  Candidates are timed at their own split and plain order
             // whatever the size of this chunk: the choice is for every later one.
             const int cand[][2] = {{3, 4}, {4, 4}, {9, 2}, {9, 4}, {9, 8},
-                                   {5, 4}, {8, 2}, {8, 4}, {8, 8}};
+                                   {5, 4}, {8, 2}, {8, 4}, {8, 8}, {9, 1}};
             const int ntile = 5;  // candidates that stand for their tile
             auto time = [&](int v, int sp, bool plain) {
                 hipEvent_t e0, e1;

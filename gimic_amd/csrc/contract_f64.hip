@@ -78,10 +78,12 @@ __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
     const int ntile = a.rows / a.tile_rows, tiles = a.spread ? ntile : (ntile + 7) / 8;
     const int set = slot / (tiles * a.nsplit), split = slot % a.nsplit;
     const int rt = slot % (tiles * a.nsplit) / a.nsplit;
-    const int rtile = a.spread ? rt : rt * 8 + (blockIdx.x & 7);
-    if (rtile >= ntile) return;
+    const int rank = a.spread ? rt : rt * 8 + (blockIdx.x & 7);
+    if (rank >= ntile) return;
+    const int2 tile = a.order ? a.order[rank] : make_int2(rank, a.kcount[rank]);
+    const int rtile = tile.x, count = tile.y;
     const int *K4 = a.klist + (size_t)rtile * a.nblk * 8;
-    const int nks = (a.kcount[rtile] + 3) >> 2;
+    const int nks = (count + 3) >> 2;
     // this workgroup's N-tiles e0 .. e1 and, of each, kn K-steps from k0 on
     const int nsn = a.nsplit / a.ksplit, sn = split / a.ksplit, sk = split % a.ksplit;
     const int e0 = (int)((long long)sn * nks / nsn), e1 = (int)((long long)(sn + 1) * nks / nsn);
@@ -96,7 +98,7 @@ __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
     const size_t row = (size_t)rtile * a.tile_rows + rin;
     // the point's values and gradients: dense, or compressed to the tile's granules
     const bool cmp = a.compressed;
-    const size_t w = cmp ? (size_t)a.kcount[rtile] * 4 : (size_t)a.lda;
+    const size_t w = cmp ? (size_t)count * 4 : (size_t)a.lda;
     const size_t base = (size_t)rtile * a.tile_rows * a.lda;
     const double *A = a.a64 + base + rin * w;
     const double *G = a.g64 + (cmp ? 3 * base : base) + rin * w;

@@ -228,9 +228,11 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
     const int set = slot / per_set;
     const int split = slot % a.nsplit;
     const int jt = (slot % per_set) / a.nsplit;
-    const int rtile =
+    const int rank =
         a.spread ? jt : (jt / kTileRun) * 8 * kTileRun + xcd * kTileRun + jt % kTileRun;
-    if (rtile >= a.rows / kRows) return;  // padding of the last run
+    if (rank >= a.rows / kRows) return;  // padding of the last run
+    const int2 tile = a.order ? a.order[rank] : make_int2(rank, a.kcount[rank]);
+    const int rtile = tile.x, count = tile.y;
     const size_t row0 = (size_t)rtile * kRows;
     const int lda = a.lda;
     const size_t rows = (size_t)a.rows;
@@ -238,13 +240,13 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
     // group << 12) | position of the group in this tile's compressed rows;
     // -1 pads the last four (zero right operand)
     const int *K8 = a.klist + (size_t)rtile * a.nblk * 4;
-    const int nq = (a.kcount[rtile] + 3) >> 2;
-    const int ranges = a.plain ? a.nsplit : filled_ranges(a.kcount[rtile], a.nsplit);
+    const int nq = (count + 3) >> 2;
+    const int ranges = a.plain ? a.nsplit : filled_ranges(count, a.nsplit);
     if (split >= ranges) return;
     // This tile's basis rows hold only its live groups, in list order
     // (EvalArgs): A and the gradients are addressed by list position
     // (a tile's rows are below 4 GiB: 32-bit offsets from uniform bases)
-    const unsigned wcols = 8u * a.kcount[rtile];  // functions per row
+    const unsigned wcols = 8u * count;  // functions per row
     const unsigned arow = kAParts * wcols;        // BF16 per split row
     const __bf16 *Atile = a.as3 + row0 * lda * kAParts;
     const float *Gtile = a.g32 + row0 * lda * 3;

@@ -136,6 +136,7 @@ struct ContractArgs {
     int spread;           // workgroups of fewer than kSpreadTiles row tiles to all XCDs in turn
     int plain;            // mixed: every range of a tile writes its sums, without N-tiles zeros
     const int *kcount, *klist;
+    const int2 *order;   // (row tile, its kcount), longest lists first, or null: tiles in turn
     int compressed;      // FP64 kernel: rows as in EvalArgs
 };
 // FP64 right operand in HBM: one pair block per (density set, 4-function
@@ -307,6 +308,9 @@ struct TileArgs {
 };
 
 hipError_t launch_block_lists(const TileArgs &a, hipStream_t s);
+// order[i] = (t, kcount[t]) for the ntile row tiles t, by kcount (at most
+// `most`) from the largest to the smallest, to 1/1024 of `most`
+hipError_t launch_tile_order(const int *kcount, int ntile, int most, int2 *order, hipStream_t s);
 
 hipError_t run_mfma_layout_probe(double *h_f64, float *h_bf16);
 hipError_t run_mfma32_layout_probe(float *h_out);  // 2048 floats

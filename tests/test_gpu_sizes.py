@@ -121,7 +121,7 @@ def test_small_launches_split_over_k_and_all_xcds(cage, n):
 
 
 @pytest.mark.parametrize("variant,split", [(3, 4), (4, 1), (5, 4), (8, 2), (9, 1), (9, 8)])
-@pytest.mark.parametrize("n", [1, 127, 129, 256, 257, 1000])
+@pytest.mark.parametrize("n", [1, 127, 129, 256, 257, 1000, 40000])
 def test_mixed_tiles_with_fewer_n_tiles_than_ranges(ring, n, variant, split):
     """near and far points in one set: the row tiles list from none to all of
     the ring's functions, so N-ranges stay empty in some; the mixed path's 1e-5,
