@@ -5,6 +5,8 @@
 
 #include <cmath>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <random>
 #include <stdexcept>
 #include <string>
@@ -61,7 +63,7 @@ struct Part {
 }  // namespace
 
 struct gimic_mlp {
-    hipStream_t stream = nullptr;     // own stream
+    hipStream_t stream = nullptr;     // shared_stream() of its device
     hipStream_t user = nullptr;       // caller's stream, when set
     long long np = 0;                 // parameter count
     long long woff[kD + 1], boff[kD + 1];
@@ -72,16 +74,30 @@ struct gimic_mlp {
     long long cap = 0;  // batch capacity of the work buffers
     long long step = 0;
     ~gimic_mlp() {
-        if (stream) {
-            (void)hipStreamSynchronize(stream);
-            (void)hipStreamDestroy(stream);
-        }
+        if (stream) (void)hipStreamSynchronize(stream);
     }
 };
 
 namespace {
 
 std::string &errstr() { return error_slot(); }
+
+// The stream of the networks on this device whose caller gives none.  One for
+// all of them, kept for the process: a caller's allocator hands the output
+// of one network's call to the next call while the first may still be
+// running, which is sound only where the two run one after the other (on
+// streams of their own, the late first launch of one network wrote over the
+// other's result).
+hipStream_t shared_stream() {
+    static std::mutex lock;
+    static std::map<int, hipStream_t> streams;
+    std::lock_guard<std::mutex> hold(lock);
+    int device = 0;
+    chk(hipGetDevice(&device), "hipGetDevice");
+    hipStream_t &s = streams[device];
+    if (!s) chk(hipStreamCreate(&s), "hipStreamCreate");
+    return s;
+}
 
 hipStream_t work_stream(const gimic_mlp *n) { return n->user ? n->user : n->stream; }
 
@@ -161,7 +177,7 @@ int gimic_mlp_create(gimic_mlp **out, double sigma, const double *center_scale,
         if (!out || !center_scale || !out_scale) throw MlpError(GIMIC_EINVAL, "null argument");
         auto *n = new gimic_mlp();
         try {
-            chk(hipStreamCreate(&n->stream), "hipStreamCreate");
+            n->stream = shared_stream();
             long long off = 0;
             for (int l = 0; l <= kD; l++) {
                 n->kin[l] = l == 0 ? kK0 : kH;

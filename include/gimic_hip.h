@@ -331,7 +331,8 @@ int gimic_mlp_create(gimic_mlp **net, double sigma, const double *center_scale,
                      const double *out_scale, uint64_t seed);
 int gimic_mlp_destroy(gimic_mlp *net);
 /* run the network's kernels on `stream` (e.g. the caller's current stream),
- * NULL: on the network's own stream; waits for the previous stream first */
+ * NULL: on the stream that the device's networks without one share; waits
+ * for the previous stream first */
 int gimic_mlp_set_stream(gimic_mlp *net, void *stream);
 /* parameter count and the 3 x 64 frequency matrix (either may be NULL) */
 int gimic_mlp_info(const gimic_mlp *net, long long *nparams, float *freqs);

@@ -38,3 +38,24 @@ def test_batch_sizes_match_oracle(n):
     live = np.abs(grad) > 1e-5
     assert np.allclose(d[live], -1e-3 * np.sign(grad[live]), rtol=1e-2)
     net.close()
+
+
+def test_networks_that_share_an_output_buffer():
+    """the output of one network's call, dropped by the caller, becomes the
+    output of another's while nothing waits in between"""
+    import torch
+    from gimic_amd.surrogate import Network
+    for seed in range(8):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        r = [12.0 * torch.rand((n, 3), generator=g, dtype=torch.float64, device="cuda") - 6.0
+             for n in (100, 100)]
+        nets = [Network(1.5, CS, np.linspace(0.5, 2.0, 9), seed=seed + k) for k in (0, 1)]
+        torch.cuda.synchronize()
+        print("case mlp shared output", seed, flush=True)
+        nets[0].predict(r[0])
+        nets[1].predict(r[1])
+        got = nets[0].predict(r[0])
+        torch.cuda.synchronize()
+        assert torch.equal(got, nets[0].predict(r[0], unfused=True))
+        for net in nets:
+            net.close()
