@@ -891,9 +891,12 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
         // more, 8 or 16 per CU, which even out the tiles' unequal lists (cage60,
         // 857,375 points: 87.1, 80.5, 79.3 and 79.1 ms at 1024, 2048, 4096 and
         // 8192).  The FP64 kernel's cost of starting a workgroup (about 4 us)
-        // wants some 32 K-steps in each, though, and a tile of a small basis has
+        // wants some 64 K-steps in each, though, and a tile of a small basis has
         // few: then half as many pairs (ring12, 64,000 points: 0.183 ms at
-        // 2048 against 0.227 at 4096 and 0.266 at 8192)
+        // 2048 against 0.227 at 4096 and 0.266 at 8192; shielding of the
+        // 30-atom sheet, 1218 tiles: 0.639 ms with three ranges each, 0.592 with
+        // two), not fewer: one bond plane of it, 460 tiles, takes as long as the
+        // heaviest, 0.163 ms with two ranges, 0.080 with five
         // A tuned mixed count is that of a full chip: launches of few tiles take
         // more ranges (1,331 points of the 60-atom cage, 6 tiles, dealt to all
         // XCDs besides: 1.93 to 0.43 ms; 29,791 points 2.92 to 2.34 ms).
@@ -903,7 +906,7 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
             auto pairs = [&](long long n) { return std::max<long long>(1, (n + per - 1) / per); };
             int nsplit = (int)std::min(nt, pairs(prec == GIMIC_PREC_FP64 ? 4096 : 8192));
             if (prec == GIMIC_PREC_FP64)
-                nsplit = (int)std::min<long long>(nsplit, std::max(pairs(2048), nt * nt / 128));
+                nsplit = (int)std::min<long long>(nsplit, std::max(pairs(2048), nt * nt / 256));
             if (want_split > 0)
                 nsplit = (int)std::min<long long>(
                     at_least ? std::max<long long>(want_split, pairs(1024)) : want_split, nt);
