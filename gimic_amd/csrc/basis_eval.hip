@@ -71,10 +71,10 @@ __device__ __forceinline__ void radial_parts(const EvalArgs &a, const DevShell &
 
 // Candidate lists (below) for bases of at least this many shells: with fewer,
 // nearly every shell reaches every tile and the list costs registers and a
-// pass over the shells.  Tetracene (144 shells): its mixed scan is 6% slower
-// with the list, its FP64 scan 6% faster (basis 1.66 to 1.35 ms: the pass holds
-// three rows instead of seven, so screened pairs cost more there).
-constexpr int kCandMinShells = 400, kCandMinShellsF64 = 64;
+// pass over the shells.  256 planes of tetracene (144 shells): mixed basis
+// 1.46 ms without the list, 1.19 with it, FP64 1.66 and 1.35; twelve atoms
+// (54 shells), 40,000 points: 0.094 without, 0.097 with it.
+constexpr int kCandMinShells = 64;
 // Workgroups a launch should have before they take 32 rows each
 constexpr int kMinBasisGroups = 512;
 // Shells whose candidacy the staged kernel settles per pass of its loop
@@ -508,8 +508,8 @@ hipError_t launch_basis_eval(const EvalArgs &a, int mode, hipStream_t s) {
     b.tile_points = tp;
     b.lds_image = std::max<size_t>(36 * 1024, row_bytes);
     // the image, the group positions (16-byte aligned) and, for bases of
-    // kCandMinShells (F64) shells or more, the candidate list
-    const bool cand = a.nshell >= (f64 ? kCandMinShellsF64 : kCandMinShells);
+    // kCandMinShells shells or more, the candidate list
+    const bool cand = a.nshell >= kCandMinShells;
     const size_t lds = b.lds_image + gpos_bytes(a.nblk, f64 ? 4 : 8) + (cand ? kCandBytes : 0);
     // (the candidate list's bounding sphere takes one row per lane of a wavefront)
     if (a.tile_rows % b.tile_points || a.rows % a.tile_rows || a.nblk * 32 != a.lda)
