@@ -1023,7 +1023,7 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
         timed(c, 0, st, [&] {
             hip_check(launch_sort_points(d_r + 3 * start, n_c, W.spts.as<double>(),
                                          W.perm.as<int>(), W.bpart.as<double>(),
-                                         W.sortscr.as<int>(), st),
+                                         W.sortscr.as<int>(), prec == GIMIC_PREC_FP64, st),
                       "sort_points");
         });
         if (tune) {

@@ -283,12 +283,12 @@ hipError_t launch_plane_reduce(const double *contrib, long long stride, const in
                                double *out, hipStream_t s);
 
 // Spatial tiles (tiles.hip).  launch_sort_points orders n points along a
-// Morton curve of 32^3 cells over their bounding box (stable, so the same on
-// every run): spts[j] = pts[perm[j]]; bpart holds 256 * 6 doubles, scratch
+// Hilbert or Morton curve of 32^3 cells over their bounding box (stable, so
+// the same on every run): spts[j] = pts[perm[j]]; bpart holds 256 * 6 doubles, scratch
 // sort_scratch_ints(n) ints.
 int sort_scratch_ints(int n);
 hipError_t launch_sort_points(const double *pts, int n, double *spts, int *perm, double *bpart,
-                              int *scratch, hipStream_t s);
+                              int *scratch, bool hilbert, hipStream_t s);
 struct TileArgs {
     const double *spts;  // sorted chunk points
     int npts, rows;      // valid and padded rows

@@ -9,8 +9,11 @@
 // produces the same numbers as the dense product.
 //
 // Two steps per chunk of points:
-//  1. Order the points along a Morton curve of 32^3 cubic cells over their
-//     bounding box (a stable LSD radix sort with two 8-bit digits of the
+//  1. Order the points along a curve through 32^3 cubic cells over their
+//     bounding box (the Hilbert curve for the FP64 kernel, whose tiles list 2 to
+//     12% fewer pairs than on the Morton curve, the 60-atom cage on 95^3 76.6
+//     to 74.2 ms; the mixed kernels keep the latter, as their last digits
+//     depend on the tiles; a stable LSD radix sort with two 8-bit digits of the
 //     15-bit cell key, so the order - and with it every result bit - is the
 //     same on every run); the basis, contraction and finalize kernels work on the
 //     sorted rows, and finalize writes each tensor back to its caller index.
@@ -74,19 +77,44 @@ __global__ __launch_bounds__(256) void bbox_partial_kernel(const double *pts, in
     if (t < 6) out[blockIdx.x * 6 + t] = s[t][0];
 }
 
-// Morton key of the cell of a point in the box [lo, hi]
+// Index of a cell along the Hilbert curve, three bits an octant (J. Skilling,
+// "Programming the Hilbert curve", AIP Conf. Proc. 707, 381 (2004))
+__device__ __forceinline__ unsigned hilbert3(unsigned x, unsigned y, unsigned z) {
+    unsigned v[3] = {x, y, z};
+#pragma unroll
+    for (unsigned q = 1u << (kCellBits - 1); q > 1; q >>= 1) {
+        const unsigned low = q - 1;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            // set: invert the low bits of x; clear: exchange them with x's
+            const unsigned t = (v[0] ^ v[i]) & low;
+            const bool set = v[i] & q;
+            v[0] ^= set ? low : t;
+            if (i > 0) v[i] ^= set ? 0u : t;
+        }
+    }
+    v[1] ^= v[0];
+    v[2] ^= v[1];
+    unsigned t = 0;
+#pragma unroll
+    for (unsigned q = 1u << (kCellBits - 1); q > 1; q >>= 1)
+        if (v[2] & q) t ^= q - 1;
+    return spread3(v[0] ^ t) << 2 | spread3(v[1] ^ t) << 1 | spread3(v[2] ^ t);
+}
+
+// Key of the cell of a point in the box [lo, hi]: its place on the Morton or
+// the Hilbert curve
 __device__ __forceinline__ unsigned cell_key(const double *pt, const double (&lo)[3],
-                                             const double (&hi)[3]) {
+                                             const double (&hi)[3], bool hilbert) {
     double h = fmax(fmax(hi[0] - lo[0], hi[1] - lo[1]), hi[2] - lo[2]) / (1 << kCellBits);
     if (!(h > 0.0) || !isfinite(h)) h = 1.0;
-    unsigned key = 0;
+    unsigned c[3];
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
+    for (int d = 0; d < 3; d++)
         // fmax/fmin map NaN to the first cell
-        const double c = fmin(fmax((pt[d] - lo[d]) / h, 0.0), (double)((1 << kCellBits) - 1));
-        key |= spread3((unsigned)c) << d;
-    }
-    return key;
+        c[d] = (unsigned)fmin(fmax((pt[d] - lo[d]) / h, 0.0), (double)((1 << kCellBits) - 1));
+    return hilbert ? hilbert3(c[0], c[1], c[2])
+                   : spread3(c[0]) | spread3(c[1]) << 1 | spread3(c[2]) << 2;
 }
 
 // box of the lanes' boxes, left in every lane of the wavefront
@@ -105,7 +133,7 @@ __device__ __forceinline__ void wave_box(double (&lo)[3], double (&hi)[3]) {
 // and the sorted points.  A single point took 14 launches of the general sort,
 // half of the time of its tensor.
 __global__ __launch_bounds__(1024) void small_sort_kernel(const double *pts, int n, double *spts,
-                                                          int *perm) {
+                                                          int *perm, bool hilbert) {
     __shared__ unsigned v[kSmallSort];
     __shared__ double box[16][6];
     const int t = threadIdx.x, nt = blockDim.x, lane = t & 63, wave = t >> 6;
@@ -133,7 +161,7 @@ __global__ __launch_bounds__(1024) void small_sort_kernel(const double *pts, int
     int m = 1;
     while (m < n) m <<= 1;
     for (int i = t; i < m; i += nt)
-        v[i] = i < n ? cell_key(pts + 3 * i, lo, hi) << kSmallBits | (unsigned)i : ~0u;
+        v[i] = i < n ? cell_key(pts + 3 * i, lo, hi, hilbert) << kSmallBits | (unsigned)i : ~0u;
     for (int k = 2; k <= m; k <<= 1)
         for (int j = k >> 1; j > 0; j >>= 1) {
             __syncthreads();
@@ -160,7 +188,7 @@ __global__ __launch_bounds__(1024) void small_sort_kernel(const double *pts, int
 template <bool FIRST>
 __global__ __launch_bounds__(256) void radix_hist_kernel(const double *pts, const double *bpart,
                                                          int nbpart, unsigned *keys, int n, int shift,
-                                                         int *hist) {
+                                                         int *hist, bool hilbert) {
     __shared__ int cnt[kBins];
     __shared__ double box[4][6];
     const int t = threadIdx.x, b = blockIdx.x, nb = gridDim.x;
@@ -192,7 +220,7 @@ __global__ __launch_bounds__(256) void radix_hist_kernel(const double *pts, cons
         const long long i = (long long)b * kSortBlock + r * 256 + t;
         if (i >= n) break;
         unsigned key;
-        if (FIRST) keys[i] = key = cell_key(pts + 3 * i, lo, hi);
+        if (FIRST) keys[i] = key = cell_key(pts + 3 * i, lo, hi, hilbert);
         else key = keys[i];
         atomicAdd(&cnt[(key >> shift) & (kBins - 1)], 1);
     }
@@ -419,11 +447,12 @@ int sort_scratch_ints(int n) {
 }
 
 hipError_t launch_sort_points(const double *pts, int n, double *spts, int *perm, double *bpart,
-                              int *scratch, hipStream_t s) {
+                              int *scratch, bool hilbert, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     if (n <= kSmallSort) {
         const int threads = n <= 128 ? 64 : n <= 512 ? 256 : 1024;
-        hipLaunchKernelGGL(small_sort_kernel, dim3(1), dim3(threads), 0, s, pts, n, spts, perm);
+        hipLaunchKernelGGL(small_sort_kernel, dim3(1), dim3(threads), 0, s, pts, n, spts, perm,
+                           hilbert);
         return hipGetLastError();
     }
     const int nb = (n + kSortBlock - 1) / kSortBlock;
@@ -432,13 +461,13 @@ hipError_t launch_sort_points(const double *pts, int n, double *spts, int *perm,
     const int npart = n < 256 * 256 ? (n + 255) / 256 : 256;
     hipLaunchKernelGGL(bbox_partial_kernel, dim3(npart), dim3(256), 0, s, pts, n, bpart);
     hipLaunchKernelGGL(radix_hist_kernel<true>, dim3(nb), dim3(256), 0, s, pts, (const double *)bpart,
-                       npart, k0, n, 0, hist);
+                       npart, k0, n, 0, hist, hilbert);
     hipLaunchKernelGGL(radix_scan_kernel, dim3(kBins), dim3(256), 0, s, hist, nb, digits);
     hipLaunchKernelGGL(radix_scatter_kernel<false>, dim3(nb), dim3(256), 0, s, (const unsigned *)k0,
                        (const int *)nullptr, n, 0, (const int *)hist, (const int *)digits, k1, i1,
                        (const double *)nullptr, (double *)nullptr);
     hipLaunchKernelGGL(radix_hist_kernel<false>, dim3(nb), dim3(256), 0, s, (const double *)nullptr,
-                       (const double *)nullptr, 0, k1, n, 8, hist);
+                       (const double *)nullptr, 0, k1, n, 8, hist, hilbert);
     hipLaunchKernelGGL(radix_scan_kernel, dim3(kBins), dim3(256), 0, s, hist, nb, digits);
     hipLaunchKernelGGL(radix_scatter_kernel<true>, dim3(nb), dim3(256), 0, s, (const unsigned *)k1,
                        (const int *)i1, n, 8, (const int *)hist, (const int *)digits,
