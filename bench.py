@@ -75,8 +75,9 @@ def time_steps(ctx, d_pts, out, precision, steps, warmup):
 def kernel_roofline(ctx, d_pts, out, precision, nbf):
     """Two extra passes: one that counts the screening lists of every row
     tile (a tile of R rows with k live 8-function groups multiplies
-    R x 8k by 8k x 7*8k: 14 R (8 k)^2 flops; both kernels walk the live
-    groups along N and K), and one with event timing around each kernel
+    R x 8k by 8k x 7*8k: 14 R (8 k)^2 flops; the mixed kernel walks these
+    groups along N and K, the FP64 kernel the live granules of four functions
+    in them, up to a fifth fewer pairs, so its figure is an upper bound), and one with event timing around each kernel
     launch.  achieved = listed flops per launch / average launch time; the
     dense product would need 14 nbf^2 per point."""
     import torch
@@ -99,7 +100,7 @@ def kernel_roofline(ctx, d_pts, out, precision, nbf):
     npts = d_pts.shape[0]
     dense = 14.0 * nbf * nbf * npts
     if ts["tiles"] > 0:
-        # both kernels walk the live 8-function groups along N and K
+        # live 8-function groups along N and K (FP64: an upper bound)
         pairs = ts["groups_sq"] * 64.0
         flop = 14.0 * ts["tile_rows"] * pairs
         block_pairs = pairs / (ts["tiles"] * (32.0 * ts["nblk"]) ** 2)
