@@ -618,14 +618,14 @@ constexpr int kDefaultVariant = 9, kDefaultSplit = 4;
 constexpr int kScratchMaxSplit = 32;
 
 // How much faster the mixed kernels of 256-row tiles have to be than those of
-// 128 rows to be taken: 1.095, or 1.12 for the few tiles of a small chunk.
+// 128 rows to be taken: 1.07, or 1.12 for the few tiles of a small chunk.
 // Screening follows the tile, so the results of the two differ by some 2e-8 of
-// their norm.  The lines lie where the two were equally fast (all but 8 of
-// 248 timed sizes are chosen as then, or were within 1% of each other) when
+// their norm.  The lines lie where the two were equally fast (all but 13 of
+// 302 timed sizes are chosen as then, or were within 1.2% of each other) when
 // wavefronts waited for each K-step's list entries, which cost the 8-wavefront
 // kernels twice as much: a faster kernel does not move a program's results
 // between the two
-float wide_tile_gain(int points) { return points <= 25000 ? 1.12f : 1.095f; }
+float wide_tile_gain(int points) { return points <= 30000 ? 1.12f : 1.07f; }
 
 // Row tile of the mixed kernels: 128 rows (4 wavefronts x 32), 256 (4 x 64
 // or 8 x 32)
