@@ -39,11 +39,14 @@
 // workgroup of 128 points per CU with the same pipeline took 82.0 ms where
 // this takes 77.5, two buffers and a barrier that drains the matrix pipe 86.9.
 //
-// Bound: the matrix pipe.  On the 60-atom cage (857,375 points, 4.5 TFLOP of
-// listed work) 77.5 ms, 58 TF/s, 81% of a large FP64 matrix product on the
+// Bound: the matrix pipe.  On the 60-atom cage (857,375 points, 4.1 TFLOP of
+// listed work) 68.2 ms, 60 TF/s, 84% of a large FP64 matrix product on the
 // same card (71.6 TF/s); the kernel it replaced (points first, 8-function
 // groups, operands from global memory into registers) took 136 ms.  With every
-// operand load redirected to one cached block it ran within 1% of that.
+// operand load redirected to one cached block it ran within 1% of that.  A
+// wavefront takes its columns of compressed rows from the step's number: with
+// the place read from the list entry it took 69.2 ms, and 256 planes of the
+// 30-atom sheet 2.51 ms against 2.46.
 //
 // Workgroup order: the ranges of a row tile run back to back on one XCD
 // (workgroup i goes to XCD i mod 8), so its basis rows come from that L2; with
@@ -65,6 +68,7 @@ constexpr int kWaitLds = 0xC07F;
 
 // one workgroup: 64 points of a row tile of a.tile_rows (64 or 128), a range
 // of its N-tiles; 4 wavefronts, two workgroups per CU
+template <bool CMP>
 __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
     constexpr int kRows = 64;
     // [step mod 3][matrix][k pair][lane][2 k], lanes swizzled (below)
@@ -97,17 +101,22 @@ __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
     const int rin = part * kRows + wave * 16 + c;
     const size_t row = (size_t)rtile * a.tile_rows + rin;
     // the point's values and gradients: dense, or compressed to the tile's granules
-    const bool cmp = a.compressed;
-    const size_t w = cmp ? (size_t)count * 4 : (size_t)a.lda;
+    const size_t w = CMP ? (size_t)count * 4 : (size_t)a.lda;
     const size_t base = (size_t)rtile * a.tile_rows * a.lda;
     const double *A = a.a64 + base + rin * w;
-    const double *G = a.g64 + (cmp ? 3 * base : base) + rin * w;
-    const size_t gplane = cmp ? (size_t)a.tile_rows * w : (size_t)a.gplane;
+    const double *G = a.g64 + (CMP ? 3 * base : base) + rin * w;
+    const size_t gplane = CMP ? (size_t)a.tile_rows * w : (size_t)a.gplane;
     const bool valid = row < (size_t)a.npts;
     const double r[3] = {valid ? a.pts[3 * row] : 0.0, valid ? a.pts[3 * row + 1] : 0.0,
                          valid ? a.pts[3 * row + 2] : 0.0};
-    // a padding entry (-1) reads the row's first granule against zero blocks
-    auto acol = [&](int v) { return v < 0 ? 0 : (cmp ? v & 8191 : v >> 13) * 4; };
+    // column of the lane's granule of four-granule step s: compressed rows hold
+    // the granules in list order, so no list entry is waited for (a padding
+    // entry reads some granule of the row against zero blocks)
+    auto acol = [&](int s) -> unsigned {
+        if (CMP) return 4u * min(4 * s + g, count - 1);
+        const int v = K4[4 * s + g];
+        return v < 0 ? 0u : (v >> 13) * 4u;
+    };
 
     // Element pair sp of matrix m for lane l is at (2 m + sp) * 64 +
     // (l ^ (l >> 3 & 1) ^ 2 sp): eight consecutive lanes of a read (c fixed in
@@ -173,8 +182,8 @@ __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
         load(source());
         put(buf + nx1);
         load(source());
-        v4d an = *(const v4d *)(A + acol(KK[g]));
-        int xa = KK[(kn > 1 ? 4 : 0) + g];  // the next K-step's granule
+        v4d an = *(const v4d *)(A + acol(k0));
+        unsigned xa = acol(k0 + (kn > 1 ? 1 : 0));  // the next K-step's column
         __syncthreads();
         v2d b0[kNMat];
 #pragma unroll
@@ -183,9 +192,10 @@ __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
         for (int e = e0; e < e1; e++) {
             // the epilogue's operands: the four functions of this lane's granule
             const int xn = K4[4 * e + g];
-            const v4d ph = *(const v4d *)(A + acol(xn));
-            const v4d g0 = *(const v4d *)(G + acol(xn)), g1 = *(const v4d *)(G + gplane + acol(xn)),
-                      g2 = *(const v4d *)(G + 2 * gplane + acol(xn));
+            const unsigned xc = acol(e);
+            const v4d ph = *(const v4d *)(A + xc);
+            const v4d g0 = *(const v4d *)(G + xc), g1 = *(const v4d *)(G + gplane + xc),
+                      g2 = *(const v4d *)(G + 2 * gplane + xc);
             v4d acc[kNMat];
 #pragma unroll
             for (int m = 0; m < kNMat; m++) acc[m] = v4d{0.0, 0.0, 0.0, 0.0};
@@ -194,8 +204,8 @@ __global__ __launch_bounds__(256, 2) void contract_f64_kernel(ContractArgs a) {
                 v2d b1[kNMat];
 #pragma unroll
                 for (int m = 0; m < kNMat; m++) b1[m] = buf[cur + rd1 + m * 128];
-                an = *(const v4d *)(A + acol(xa));
-                xa = KK[4 * (ks + 2 < kn ? ks + 2 : ks + 2 - kn < kn ? ks + 2 - kn : 0) + g];
+                an = *(const v4d *)(A + xa);
+                xa = acol(k0 + (ks + 2 < kn ? ks + 2 : ks + 2 - kn < kn ? ks + 2 - kn : 0));
 #pragma unroll
                 for (int m = 0; m < kNMat; m++)
                     acc[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(b0[m].x, av[0], acc[m], 0, 0, 0);
@@ -274,7 +284,10 @@ hipError_t launch_contract_f64(const ContractArgs &a, hipStream_t s) {
     const long long nwg = (b.spread ? ntile : 8LL * ((ntile + 7) / 8)) * a.nsplit * a.nmatset *
                           (a.tile_rows / 64);
     if (nwg > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(contract_f64_kernel, dim3((unsigned)nwg), dim3(256), 0, s, b);
+    if (a.compressed)
+        hipLaunchKernelGGL(contract_f64_kernel<true>, dim3((unsigned)nwg), dim3(256), 0, s, b);
+    else
+        hipLaunchKernelGGL(contract_f64_kernel<false>, dim3((unsigned)nwg), dim3(256), 0, s, b);
     return hipGetLastError();
 }
 
