@@ -264,8 +264,10 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
 
     // lane (g, c) of row block rb: row wave*32 + rb*16 + c, k-group entry g of the K-step
     const unsigned lrow = (wave * 16 * kRB + c) * arow;
-    auto a_off = [&](int x) -> unsigned {  // this lane's group of a K-step, in BF16 of a row
-        return x < 0 ? 0u : (unsigned)(x & 4095) * (8 * kAParts);
+    // this lane's group of K-step ks in BF16 of a row, whose groups are in list
+    // order (beyond the list: some group of it against zero blocks)
+    auto a_off = [&](int ks) -> unsigned {
+        return (unsigned)min(4 * ks + g, count - 1) * (8 * kAParts);
     };
     auto a_frag = [&](unsigned ao, int rb, int p) -> v8bf {
         return *(const v8bf *)((const char *)(Atile + rb * 16 * arow) + 2 * (lrow + ao) + 16 * p);
@@ -291,7 +293,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
         stage_block_k8<WAVES>(Bset, rowst, nkg, q0, nlo, bbuf, wave, lane);
         if (NBUF == 3 && nq > 1)
             stage_block_k8<WAVES>(Bset, rowst, nkg, q1, nlo, bbuf + kBufBytes, wave, lane);
-        const unsigned ao = a_off(q0);
+        const unsigned ao = a_off(0);
 #pragma unroll
         for (int rb = 0; rb < kRB; rb++)
 #pragma unroll
@@ -314,18 +316,17 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
         __builtin_amdgcn_s_waitcnt(kWaitAll);
         __syncthreads();
 
-        // groups of the next step's A fragments and of this step's copy: each
-        // lane reads its group's entry a K-step before the copy needs it (the
-        // first load of a step, so the end-of-step wait covers it), and the
-        // copy takes the four of its step from lanes 0, 16, 32 and 48
-        int ent_a = q1, ent_c = NBUF == 3 ? q2 : q1;
+        // groups of this step's copy: each lane reads its group's entry a K-step
+        // before the copy needs it (the first load of a step, so the
+        // end-of-step wait covers it), and the copy takes the four of its step
+        // from lanes 0, 16, 32 and 48
+        int ent_c = NBUF == 3 ? q2 : q1;
         for (int ks = 0; ks < nq; ks++) {
             // opaque: otherwise the scalar copies are taken right after the
             // load, which stalls the step for the load's latency
             asm volatile("" : "+v"(ent_c));
-            const int ea = ent_a, ec = ent_c;
+            const int ec = ent_c;
             ent_c = entry(ks + NBUF);
-            ent_a = NBUF == 3 ? ec : ent_c;
             v8bf as[kRB][kAParts];
 #pragma unroll
             for (int rb = 0; rb < kRB; rb++)
@@ -348,7 +349,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
             static_assert(NBUF != 3 || (kALoads + 1) / 2 <= kCopyFrom, "A loads must precede the copy");
             const int ahead = ks + NBUF - 1;
             const bool copy = NBUF == 3 || ahead < nq;
-            const unsigned aoff = a_off(ea);
+            const unsigned aoff = a_off(ks + 1);
             unsigned char *cbuf = bbuf + (size_t)(ahead % NBUF) * kBufBytes;
             const __bf16 *cur = (const __bf16 *)(bbuf + (size_t)(ks % NBUF) * kBufBytes);
             v8bf bf[2][kBParts];
@@ -416,7 +417,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
         for (int h = 0; h < 2; h++) {
             const int x = __shfl(xn, 8 * (2 * h + (c >> 3)));
             const unsigned fn = x < 0 ? 0 : (x >> 12) * 8 + (c & 7);
-            acol[h] = x < 0 ? 0 : (x & 4095) * 8 + (c & 7);
+            acol[h] = min(4 * e + 2 * h + (c >> 3), count - 1) * 8 + (c & 7);
 #pragma unroll
             for (int d = 0; d < 3; d++) R[h][d] = (a.rf32 + (size_t)d * a.ncol_pad)[fn];
         }
