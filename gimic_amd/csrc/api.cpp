@@ -861,6 +861,7 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
             ta.gran = gran;
             ta.shells = c->shells.as<DevShell>();
             ta.nshell = (int)c->basis.shells.size();
+            ta.natoms = (int)(c->basis.coords.size() / 3);
             ta.coords = c->coords.as<double>();
             ta.bcount = W.bcount.as<int>();
             ta.k8count = W.k8count.as<int>();

@@ -296,7 +296,7 @@ struct TileArgs {
     int nblk;            // 32-function blocks (lda / 32), at most 1024
     int gran;            // functions per list entry: 8 (mixed) or 4 (FP64)
     const DevShell *shells;
-    int nshell;
+    int nshell, natoms;
     const double *coords;
     // per row tile: 32-function blocks and 8-function groups that screening
     // can leave non-zero (statistics), and the list the contraction walks, the

@@ -24,7 +24,8 @@
 //     not is never left out) and, for the FP64 kernel, of one of its points:
 //     4 to 33% fewer (N-tile, K-step) pairs (shielding of the 30-atom sheet
 //     1.17 to 1.06 ms, 256 planes of it 4.90 to 4.71, the 60-atom cage on 95^3
-//     80.1 to 76.6, lists included: 28 to 56 us a launch of 5735 tiles).  The
+//     80.1 to 76.6).  The points are tested once per atom, 43 us for 5735 tiles
+//     (28 with the box alone; 53 when every shell tested them).  The
 //     mixed kernels keep the box alone: which groups share a K-step decides
 //     the last digits of their FP32 sums.
 #include "device_common.h"
@@ -35,6 +36,9 @@ namespace {
 
 constexpr int kSortBlock = 1024;  // elements per radix block (4 rounds of 256)
 constexpr int kBins = 256;        // 8-bit digits
+// atoms whose distances an FP64 list takes into account (4 KiB of LDS); the
+// lists of a larger molecule go by the box alone
+constexpr int kListAtoms = 512;
 constexpr int kCellBits = 5;      // 32 cells per axis: a 15-bit key, two digits
 constexpr int kSmallSort = 2048;  // points that one workgroup sorts by itself
 constexpr int kSmallBits = 11;    // of their index
@@ -326,7 +330,7 @@ __global__ __launch_bounds__(256) void block_list_kernel(TileArgs a) {
     __shared__ double box[4][6];
     __shared__ int wsum[4][3];
     __shared__ unsigned live[kMaxBlk];  // live granules of each block, 8 bits
-    __shared__ double pts[3 * kWgRows];
+    __shared__ double pts[3 * kWgRows], near2[kListAtoms];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const long long r0 = (long long)blockIdx.x * a.tile_rows;
     double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
@@ -357,13 +361,29 @@ __global__ __launch_bounds__(256) void block_list_kernel(TileArgs a) {
             lo[d] = fmin(lo[d], box[w][d]);
             hi[d] = fmax(hi[d], box[w][3 + d]);
         }
-    // FP64 lists: the points after the box, four at a time (their LDS reads
-    // overlap), `share` threads a shell
-    const int np = a.gran == 4 ? (int)min((long long)a.tile_rows, max(0LL, a.npts - r0)) : 0;
-    const int share = a.nshell <= 64 ? 4 : a.nshell <= 128 ? 2 : 1;
+    // FP64 lists: the points after the box, by the squared distance of every
+    // atom from the nearest one (`share` lanes an atom)
+    const bool points = a.gran == 4 && a.natoms <= kListAtoms;
+    if (points) {
+        const int np = (int)min((long long)a.tile_rows, max(0LL, a.npts - r0));
+        const int share = a.natoms <= 32 ? 8 : a.natoms <= 64 ? 4 : a.natoms <= 128 ? 2 : 1;
+        for (int i0 = 0; i0 < a.natoms * share; i0 += 256) {
+            const int atom = (i0 + t) / share, q = t % share;
+            const double *R = a.coords + 3 * min(atom, a.natoms - 1);
+            const double R0 = R[0], R1 = R[1], R2 = R[2];
+            double m = INFINITY;
+#pragma unroll 4
+            for (int p = q; p < np; p += share) {
+                const double x = pts[3 * p] - R0, y = pts[3 * p + 1] - R1, z = pts[3 * p + 2] - R2;
+                m = fmin(m, x * x + y * y + z * z);
+            }
+            for (int d = 1; d < share; d <<= 1) m = fmin(m, __shfl_xor(m, d));
+            if (q == 0 && atom < a.natoms) near2[atom] = m;
+        }
+        __syncthreads();
+    }
     if (r0 < a.npts)
-        for (int i = t; i < a.nshell * share; i += 256) {
-            const int k = i / share;
+        for (int k = t; k < a.nshell; k += 256) {
             const DevShell sh = a.shells[k];
             const double *R = a.coords + 3 * sh.atom;
             double d2 = 0.0;
@@ -374,20 +394,7 @@ __global__ __launch_bounds__(256) void block_list_kernel(TileArgs a) {
             }
             // relative slack for rounding in the basis kernel's own distance
             const double reach = sh.radius * (1.0 + 1e-12) + 1e-12;
-            bool hit = sqrt(d2) <= reach;
-            if (hit && a.gran == 4) {
-                hit = false;
-                for (int p0 = i % share; p0 < np && !hit; p0 += 4 * share) {
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const int p = min(p0 + j * share, np - 1);
-                        const double x = pts[3 * p] - R[0], y = pts[3 * p + 1] - R[1],
-                                     z = pts[3 * p + 2] - R[2];
-                        hit |= x * x + y * y + z * z <= reach * reach;
-                    }
-                }
-            }
-            if (hit)
+            if (sqrt(d2) <= reach && (!points || near2[sh.atom] <= reach * reach))
                 for (int q = sh.fout >> 2; q <= (sh.fout + sh.ncomp_out - 1) >> 2; q++)
                     atomicOr(&live[q >> 3], 1u << (q & 7));
         }
