@@ -135,3 +135,23 @@ def test_mixed_tiles_with_fewer_n_tiles_than_ranges(ring, n, variant, split):
         ctx.set_mixed_kernel(variant, split)
         M = ctx.jtensor(pts, precision="mixed")
     assert np.abs(M - J).max() <= 1e-5 * np.abs(J).max()
+
+
+@pytest.mark.parametrize("natoms", [1, 33, 65, 129, 513])
+def test_fp64_lists_by_atoms(natoms):
+    """FP64 lists test a tile's points with 8, 4, 2 or 1 lanes an atom, and go by
+    the box alone beyond 512 atoms; a chain of hydrogen atoms, points all along it"""
+    from gimic_amd import synth
+    xyz = np.c_[1.7 * np.arange(natoms), np.zeros((natoms, 2))]
+    s, rng = synth.build_system("chain", ["H"] * natoms, xyz, {"H": "2s1p"}, natoms)
+    s.dens = synth.density_family(rng, s.nbf, max(1, s.nbf // 4))[None]
+    pts = np.random.default_rng(natoms).uniform(-4.0, 4.0, (700, 3))
+    pts[:, 0] = np.random.default_rng(1).uniform(-4.0, 1.7 * natoms + 4.0, 700)
+    print("case chain of", natoms, flush=True)
+    with s.context(screening=1e-8) as ctx:
+        J = ctx.jtensor(pts, precision="fp64")
+    sub = np.arange(0, 700, 35)
+    ref = oracle.jtensor(s.arrays(), sph.to_cartesian(s.dens, s.shell_l), pts[sub], screening=1e-8)
+    scale = np.linalg.norm(J, axis=1).max()
+    e = np.linalg.norm(J[sub] - ref, axis=1) / np.maximum(np.linalg.norm(ref, axis=1), 1e-3 * scale)
+    assert e.max() <= 1e-10, e.max()
