@@ -362,14 +362,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
 #pragma unroll
             for (int cb = 0; cb < kCB; cb++) {
                 const int sl = cb & 1;
-                bool first = true;
-                for_split_products([&](int ia, int ib) {
-#pragma unroll
-                    for (int rb = 0; rb < kRB; rb++)
-                        acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            as[rb][ia], bf[sl][ib], acc[rb][cb], 0, 0, 0);
-                    if (!first) return;
-                    first = false;
+                auto loads = [&] {
                     __builtin_amdgcn_sched_barrier(0);
                     if (cb + 1 < kCB) {
                         const int off = g * kMx2GroupElems + ((cb + 1) * 16 + c) * 8;
@@ -386,6 +379,19 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
                         stage_piece_k8<WAVES>(Bset, rowst, nkg, ec, nlo, cbuf, wave, lane,
                                               cb - kCopyFrom);
                     __builtin_amdgcn_sched_barrier(0);
+                };
+                // after the first products: a wait for the operands of these is
+                // then no wait for the reads just issued (with four row blocks
+                // it costs moves between register files instead)
+                bool first = true;
+                if (kRB == 4) loads();
+                for_split_products([&](int ia, int ib) {
+#pragma unroll
+                    for (int rb = 0; rb < kRB; rb++)
+                        acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            as[rb][ia], bf[sl][ib], acc[rb][cb], 0, 0, 0);
+                    if (first && kRB != 4) loads();
+                    first = false;
                 });
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -443,12 +449,14 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
         };
 #pragma unroll
         for (int it = 0; it < kAhead; it++) load_row(it, pv[it], Gv[it]);
-        if (e + 1 < e1) {
+        auto next_tile = [&] {
+            if (e + 1 >= e1) return;
             xn = xnext;
             xnext = K8[4 * min(e + 2, nq - 1) + nslot];
             nlo = lane_offset(xn, ngn, lane);
             start_tile(nlo);
-        }
+        };
+        if (kRB != 4) next_tile();  // (four row blocks leave no registers for it)
 #pragma unroll
         for (int it = 0; it < kIt; it++) {
             const int rb = it >> 2, r = it & 3;
@@ -503,6 +511,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void contract_mx2_kernel(ContractArg
             }
             __builtin_amdgcn_sched_barrier(0);
         }
+        if (kRB == 4) next_tile();
     }
 }
 
