@@ -432,14 +432,21 @@ void basis_eval_staged_kernel(EvalArgs a) {
             const size_t row = row0 + r0 + lp;
             if (row >= (size_t)a.npts) return;  // padding rows stay zero
             DevShell sh = a.shells[si];
-            const int cg = gpos[sh.fout / kGran];
+            const int fout = sh.fout, cg = gpos[fout / kGran];
             if (cg < 0) return;  // zero over the whole tile
-            sh.fout = cg * kGran + sh.fout % kGran;
+            sh.fout = cg * kGran + fout % kGran;
             const double *r = a.pts + 3 * row;
             const double *R = a.coords + 3 * sh.atom;
             double rr[3] = {r[0] - R[0], r[1] - R[1], r[2] - R[2]};
             const double s = rr[0] * rr[0] + rr[1] * rr[1] + rr[2] * rr[2];
             if (sqrt(s) > sh.radius) return;  // screened: zeros already in place
+            if (isnan(s)) {
+                // a point that is not a number screens nothing out, so this shell
+                // may be one that is beyond reach of the tile and only shares its
+                // first group: its functions have no columns of their own then
+                const int last = (fout + sh.ncomp_out - 1) / kGran;
+                if (gpos[last] != cg + last - fout / kGran) return;
+            }
             double g, h;
             radial_parts<!F64>(a, sh, s, g, h);
             constexpr int M = F64 ? 4 : 3;

@@ -155,3 +155,27 @@ def test_fp64_lists_by_atoms(natoms):
     scale = np.linalg.norm(J, axis=1).max()
     e = np.linalg.norm(J[sub] - ref, axis=1) / np.maximum(np.linalg.norm(ref, axis=1), 1e-3 * scale)
     assert e.max() <= 1e-10, e.max()
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("mixed", 1e-5)])
+def test_many_points_not_a_number(precision, tol):
+    """no shell is screened out at such a point, those that only share a group
+    with a shell in reach of its tile included: these have no columns in the
+    tile's compressed rows and must not be written.  A chain of 20 hydrogen
+    atoms, so that every tile lists a part of the functions only"""
+    from gimic_amd import synth
+    xyz = np.c_[1.7 * np.arange(20), np.zeros((20, 2))]
+    s, rng = synth.build_system("chain", ["H"] * 20, xyz, {"H": "2s1p"}, 20)
+    s.dens = synth.density_family(rng, s.nbf, s.nbf // 4)[None]
+    n = 3000
+    pts = rng.uniform(-2.0, 2.0, (n, 3))
+    pts[:, 0] = rng.uniform(-2.0, 34.3, n)
+    odd = pts.copy()
+    odd[::7, 1] = np.nan
+    keep = ~np.isnan(odd[:, 1])
+    with s.context(screening=1e-8) as ctx:
+        J = ctx.jtensor(pts, precision="fp64")
+        print("case chain of 20, every seventh point nan", precision, flush=True)
+        K = ctx.jtensor(odd, precision=precision)
+    assert rel_err(K[keep], J[keep]).max() <= tol
+    assert np.isnan(K[~keep]).all()
