@@ -80,8 +80,8 @@ constexpr int kMinBasisGroups = 512;
 // Shells whose candidacy the staged kernel settles per pass of its loop
 constexpr int kCandChunk = 1024;
 // LDS beyond the image and the block positions: candidate list, bounding
-// sphere, per-wavefront counts
-constexpr size_t kCandBytes = kCandChunk * 2 + 4 * 8 + 4 * 4;
+// box, per-wavefront counts
+constexpr size_t kCandBytes = kCandChunk * 2 + 6 * 8 + 4 * 4;
 
 // LDS for the place of each group of `gran` functions (nblk * 32 / gran shorts)
 __host__ __device__ constexpr size_t gpos_bytes(int nblk, int gran) {
@@ -337,43 +337,31 @@ void basis_eval_staged_kernel(EvalArgs a) {
     // Candidate shells (CAND): the shells that can reach a row of this workgroup,
     // listed in shell order, kCandChunk at a time.  A shell is dropped only
     // if its group is not live (compressed output) or if it is beyond its
-    // screening radius from the rows' bounding sphere, hence from every row;
+    // screening radius from the box of the rows, hence from every row;
     // the per-row radius test below still decides each (row, shell) pair,
     // so the output is the same, but the lanes of a wavefront no longer
     // idle beside pairs that every row screens out.
     short *cand = (short *)(basis_tile + a.lds_image + gpos_bytes(a.nblk, kGran));
-    double *sphere = (double *)(cand + kCandChunk);  // centre x, y, z and radius
-    int *wcnt = (int *)(sphere + 4);                 // kept shells per wavefront
+    double *box = (double *)(cand + kCandChunk);  // lower and upper corner
+    int *wcnt = (int *)(box + 6);                 // kept shells per wavefront
     if (CAND) {
-        // the rows' bounding sphere: centre = mean of the valid rows, radius
-        // = the largest distance from it (wavefront 0, one row per lane)
+        // the rows' bounding box (wavefront 0, one row per lane; a coordinate
+        // that is not a number makes it unbounded, so that its row becomes NaN)
         if (tid < 64) {
             const bool v = tid < tp && row0 + tid < (size_t)a.npts;
-            double p[3], c[3], n = v ? 1.0 : 0.0;
+            double lo[3], hi[3];
 #pragma unroll
-            for (int d = 0; d < 3; d++) c[d] = p[d] = v ? a.pts[3 * (row0 + tid) + d] : 0.0;
-#pragma unroll
-            for (int off = 32; off; off >>= 1) {
-#pragma unroll
-                for (int d = 0; d < 3; d++) c[d] += __shfl_xor(c[d], off);
-                n += __shfl_xor(n, off);
+            for (int d = 0; d < 3; d++) {
+                const double x = v ? a.pts[3 * (row0 + tid) + d] : 0.0;
+                lo[d] = !v ? INFINITY : isnan(x) ? -INFINITY : x;
+                hi[d] = !v ? -INFINITY : isnan(x) ? INFINITY : x;
             }
-            double r = 0.0;
-            if (v) {
-                double q = 0.0;
-#pragma unroll
+            wave_box(lo, hi);
+            if (tid == 0)
                 for (int d = 0; d < 3; d++) {
-                    const double t = p[d] - c[d] / n;
-                    q += t * t;
+                    box[d] = lo[d];
+                    box[3 + d] = hi[d];
                 }
-                r = sqrt(q);
-            }
-#pragma unroll
-            for (int off = 32; off; off >>= 1) r = fmax(r, __shfl_xor(r, off));
-            if (tid == 0) {
-                for (int d = 0; d < 3; d++) sphere[d] = n > 0.0 ? c[d] / n : 0.0;
-                sphere[3] = n > 0.0 ? r : -1.0;  // negative: no valid row
-            }
         }
         __syncthreads();
     }
@@ -384,16 +372,10 @@ void basis_eval_staged_kernel(EvalArgs a) {
         for (int i0 = 0; i0 < kCandChunk && s0 + i0 < a.nshell; i0 += 256) {
             const int si = s0 + i0 + tid;
             bool keep = false;
-            if (i0 + tid < kCandChunk && si < a.nshell && sphere[3] >= 0.0) {
+            if (i0 + tid < kCandChunk && si < a.nshell) {
                 const DevShell sh = a.shells[si];
-                keep = gpos[sh.fout / kGran] >= 0;
-                if (keep) {
-                    const double *R = a.coords + 3 * sh.atom;
-                    const double dx = sphere[0] - R[0], dy = sphere[1] - R[1], dz = sphere[2] - R[2];
-                    const double dist = sqrt(dx * dx + dy * dy + dz * dz);
-                    // margin: beyond the radius by more than rounding can explain
-                    keep = dist - sphere[3] <= sh.radius * (1.0 + 1e-12) + 1e-12;
-                }
+                keep = gpos[sh.fout / kGran] >= 0 &&
+                       box_distance(box, box + 3, a.coords + 3 * sh.atom) <= shell_reach(sh);
             }
             const unsigned long long m = __ballot(keep);
             if (lane == 0) wcnt[wave] = __popcll(m);
@@ -518,7 +500,7 @@ hipError_t launch_basis_eval(const EvalArgs &a, int mode, hipStream_t s) {
     // kCandMinShells shells or more, the candidate list
     const bool cand = a.nshell >= kCandMinShells;
     const size_t lds = b.lds_image + gpos_bytes(a.nblk, f64 ? 4 : 8) + (cand ? kCandBytes : 0);
-    // (the candidate list's bounding sphere takes one row per lane of a wavefront)
+    // (the candidate list's bounding box takes one row per lane of a wavefront)
     if (a.tile_rows % b.tile_points || a.rows % a.tile_rows || a.nblk * 32 != a.lda)
         return hipErrorInvalidValue;
     auto launch = [&](auto kernel) -> hipError_t {

@@ -80,6 +80,34 @@ __device__ __forceinline__ double row16_sum(double x) {
     return x;
 }
 
+// box of the lanes' boxes, left in every lane of the wavefront
+__device__ __forceinline__ void wave_box(double (&lo)[3], double (&hi)[3]) {
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            lo[d] = fmin(lo[d], __shfl_xor(lo[d], w));
+            hi[d] = fmax(hi[d], __shfl_xor(hi[d], w));
+        }
+}
+
+// Distance of R from the box [lo, hi].  No two sides are subtracted from one
+// another, so an infinite or huge one only widens the box.
+__device__ __forceinline__ double box_distance(const double *lo, const double *hi, const double *R) {
+    double d2 = 0.0;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const double e = fmax(0.0, fmax(lo[d] - R[d], R[d] - hi[d]));
+        d2 += e * e;
+    }
+    return sqrt(d2);
+}
+
+// screening radius with slack for rounding in the basis kernel's own distance
+__device__ __forceinline__ double shell_reach(const DevShell &sh) {
+    return sh.radius * (1.0 + 1e-12) + 1e-12;
+}
+
 // launchers (defined in the .hip files)
 struct EvalArgs {
     const double *pts;   // 3*npts of this chunk

@@ -121,17 +121,6 @@ __device__ __forceinline__ unsigned cell_key(const double *pt, const double (&lo
                    : spread3(c[0]) | spread3(c[1]) << 1 | spread3(c[2]) << 2;
 }
 
-// box of the lanes' boxes, left in every lane of the wavefront
-__device__ __forceinline__ void wave_box(double (&lo)[3], double (&hi)[3]) {
-#pragma unroll
-    for (int w = 32; w > 0; w >>= 1)
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            lo[d] = fmin(lo[d], __shfl_xor(lo[d], w));
-            hi[d] = fmax(hi[d], __shfl_xor(hi[d], w));
-        }
-}
-
 // Up to kSmallSort points in one workgroup and launch: box, keys, a bitonic
 // sort of (key, index) in LDS (unique keys, so the order is the stable one),
 // and the sorted points.  A single point took 14 launches of the general sort,
@@ -385,16 +374,9 @@ __global__ __launch_bounds__(256) void block_list_kernel(TileArgs a) {
     if (r0 < a.npts)
         for (int k = t; k < a.nshell; k += 256) {
             const DevShell sh = a.shells[k];
-            const double *R = a.coords + 3 * sh.atom;
-            double d2 = 0.0;
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                const double e = fmax(0.0, fmax(lo[d] - R[d], R[d] - hi[d]));
-                d2 += e * e;
-            }
-            // relative slack for rounding in the basis kernel's own distance
-            const double reach = sh.radius * (1.0 + 1e-12) + 1e-12;
-            if (sqrt(d2) <= reach && (!points || near2[sh.atom] <= reach * reach))
+            const double reach = shell_reach(sh);
+            if (box_distance(lo, hi, a.coords + 3 * sh.atom) <= reach &&
+                (!points || near2[sh.atom] <= reach * reach))
                 for (int q = sh.fout >> 2; q <= (sh.fout + sh.ncomp_out - 1) >> 2; q++)
                     atomicOr(&live[q >> 3], 1u << (q & 7));
         }

@@ -179,3 +179,36 @@ def test_many_points_not_a_number(precision, tol):
         K = ctx.jtensor(odd, precision=precision)
     assert rel_err(K[keep], J[keep]).max() <= tol
     assert np.isnan(K[~keep]).all()
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf, 1e200], ids=str)
+@pytest.mark.parametrize("n", [100, 3000, 20000])
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("mixed", 1e-5)])
+def test_point_that_is_not_finite_beside_others(sheet, n, precision, tol, bad):
+    """a basis of 64 shells or more, whose basis kernel lists the shells that
+    reach its rows: a coordinate that is not a number, infinite or too large to
+    square costs only its own tensor (1, 4 or 32 rows a workgroup)"""
+    s, ctx = sheet
+    rng = np.random.default_rng(n)
+    R = np.asarray(s.coords)
+    pts = R[rng.integers(0, len(R), n)] + rng.uniform(-2.0, 2.0, (n, 3))
+    J = ctx.jtensor(pts, precision="fp64")
+    odd = pts.copy()
+    for k in range(3):
+        odd[(2 * k + 1) * n // 7, k] = bad
+    keep = np.isfinite(odd).all(axis=1) & (np.abs(odd) < 1e100).all(axis=1)
+    assert keep.sum() == n - 3
+    print("case sheet30", n, "points, three", bad, precision, flush=True)
+    K = ctx.jtensor(odd, precision=precision)
+    assert rel_err(K[keep], J[keep]).max() <= tol
+    if np.isnan(bad):
+        assert np.isnan(K[~keep]).all()
+
+
+@pytest.fixture(scope="module")
+def sheet():
+    from gimic_amd import synth
+    s = synth.sheet30()
+    ctx = s.context(screening=1e-8)
+    yield s, ctx
+    ctx.close()
