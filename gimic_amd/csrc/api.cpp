@@ -1695,9 +1695,9 @@ void flux_run(gimic_ctx *c, int64_t npts, int nplanes, const int64_t *offs, cons
             (uintptr_t)npts, (uintptr_t)nplanes, (uintptr_t)precision, (uintptr_t)spin,
             (uintptr_t)(out_mod != nullptr), (uintptr_t)(out_acid != nullptr),
             (uintptr_t)c->giao, (uintptr_t)c->diamag, (uintptr_t)c->paramag,
-            (uintptr_t)c->mixed_variant, (uintptr_t)st, (uintptr_t)c->pts_tmp.p,
-            (uintptr_t)c->jt_tmp.p, (uintptr_t)c->contrib.p, (uintptr_t)c->planes.p,
-            (uintptr_t)c->pparams.p, (uintptr_t)c->outs.p,
+            (uintptr_t)c->mixed_variant, (uintptr_t)c->split_fixed, (uintptr_t)st,
+            (uintptr_t)c->pts_tmp.p, (uintptr_t)c->jt_tmp.p, (uintptr_t)c->contrib.p,
+            (uintptr_t)c->planes.p, (uintptr_t)c->pparams.p, (uintptr_t)c->outs.p,
             (uintptr_t)c->ws.phi64.p, (uintptr_t)c->ws.grad64.p, (uintptr_t)c->ws.grad32.p,
             (uintptr_t)c->ws.part.p, (uintptr_t)M.b64.p, (uintptr_t)c->ws.phis.p,
             (uintptr_t)M.bs3.p, (uintptr_t)c->mixed_split, (uintptr_t)c->ws.spts.p,

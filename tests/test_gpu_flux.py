@@ -248,3 +248,28 @@ def test_plane_grid_descriptors_are_checked():
     assert np.isclose(out[0], expect, rtol=1e-13, atol=1e-300)
     assert out[1] + out[2] == out[0]
     ctx.close()
+
+
+def test_fixed_kernel_of_the_tuned_numbers_builds_its_own_graph():
+    """a kernel and split that the caller fixes are kept for launches of few
+    tiles too, where the same numbers from the tuner give more ranges: the
+    graph of one is not the other's"""
+    from gimic_amd import synth
+    s = synth.sheet30()
+    with s.context() as ctx:
+        planes = _uneven_planes(np.asarray(s.coords))[:1]
+        print("case graph of a fixed kernel", flush=True)
+        ctx.set_graph(True)
+        tuned = ctx.flux_planes(planes, precision="mixed", modulus=True, acid=True)
+        variant, split = ctx.tuning()[:2]
+        ctx.set_mixed_kernel(variant, split)
+        fixed = ctx.flux_planes(planes, precision="mixed", modulus=True, acid=True)
+        assert ctx.graph_stats() == (2, 2)
+        again = ctx.flux_planes(planes, precision="mixed", modulus=True, acid=True)
+        assert ctx.graph_stats() == (2, 3)
+        ctx.set_graph(False)
+        eager = ctx.flux_planes(planes, precision="mixed", modulus=True, acid=True)
+        for f, g, e in zip(fixed, again, eager):
+            assert np.array_equal(f, e) and np.array_equal(g, e)
+        # and the same physics as before
+        assert np.allclose(tuned[0], fixed[0], rtol=1e-6, atol=1e-6 * np.abs(tuned[0]).max())
