@@ -46,7 +46,13 @@ struct Buf {
         if (bytes <= n && p) return;
         if (p) (void)hipFree(p);
         p = nullptr;
-        chk(hipMalloc(&p, bytes ? bytes : 256), "hipMalloc");
+        n = 0;
+        const hipError_t e = hipMalloc(&p, bytes ? bytes : 256);
+        if (e != hipSuccess) {
+            p = nullptr;
+            (void)hipGetLastError();  // else the next launch reports it
+        }
+        chk(e, "hipMalloc");
         n = bytes;
     }
     template <class T>
@@ -118,6 +124,7 @@ int guard(F &&f) {
 
 void reserve(gimic_mlp *n, long long P) {
     if (P <= n->cap) return;
+    n->cap = 0;  // until every buffer is there: one that cannot grow is gone
     const size_t rows = (size_t)(P + 63) / 64 * 64;  // whole tiles
     for (int l = 0; l <= kD; l++) n->X[l].need(rows * n->kin[l] * 2);
     for (int l = 0; l < kD; l++) n->dZ[l].need(rows * kH * 2);

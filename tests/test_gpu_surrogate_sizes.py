@@ -59,3 +59,27 @@ def test_networks_that_share_an_output_buffer():
         assert torch.equal(got, nets[0].predict(r[0], unfused=True))
         for net in nets:
             net.close()
+
+
+def test_batch_after_one_too_large_for_the_device():
+    """a batch whose work buffers exceed the device's memory (22 TB; refused
+    before any launch) is an error, and a batch within the earlier capacity
+    then gets buffers again"""
+    import ctypes
+    import torch
+    from gimic_amd import lib
+    from gimic_amd.surrogate import Network
+    g = torch.Generator(device="cuda").manual_seed(3)
+    r = 12.0 * torch.rand((300, 3), generator=g, dtype=torch.float64, device="cuda") - 6.0
+    t = torch.randn((300, 9), generator=g, dtype=torch.float64, device="cuda")
+    net = Network(1.5, CS, np.linspace(0.5, 2.0, 9), seed=5)
+    before = net.loss_grad(r, t, 0.05)
+    print("case mlp batch of 2^36", flush=True)
+    loss = ctypes.c_double()
+    with pytest.raises(lib.GimicError, match="out of memory"):
+        lib.check(net._lib.gimic_mlp_loss_grad(net._h, 1 << 36, ctypes.c_void_p(r.data_ptr()),
+                                               ctypes.c_void_p(t.data_ptr()), 0.05,
+                                               ctypes.byref(loss), None))
+    after = net.loss_grad(r, t, 0.05)
+    assert after[0] == before[0] and np.array_equal(after[1], before[1])
+    net.close()
