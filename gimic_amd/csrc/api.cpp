@@ -30,6 +30,24 @@ std::string &error_slot() {
     static thread_local std::string s;
     return s;
 }
+
+// One stream of each device, kept for the process, for the work of callers who
+// are themselves on the null stream.  Their allocator hands the output of one
+// call, once dropped, to the next call of any context or network while the
+// first may still be running, which is sound only where the two run one after
+// the other: on streams of their own, the first wrote over the other's result.
+hipError_t shared_stream(hipStream_t *stream) {
+    static std::mutex lock;
+    static std::map<int, hipStream_t> streams;
+    std::lock_guard<std::mutex> hold(lock);
+    int device = 0;
+    hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess) return e;
+    hipStream_t &s = streams[device];
+    if (!s) e = hipStreamCreate(&s);
+    *stream = s;
+    return e;
+}
 }  // namespace gimic
 
 namespace {
@@ -309,6 +327,9 @@ struct gimic_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     hipStream_t copy_stream = nullptr;  // host copies of pipelined batches
+    hipStream_t shared = nullptr;       // the device's shared stream, once asked for
+    hipStream_t last = nullptr;         // which of `stream` and `shared` was used last
+    hipEvent_t handover = nullptr;      // from one of these to the other
     size_t chunk_bytes = 0;  // basis buffers of one chunk of points
     size_t chunk_bytes_large = 0;  // the large setting: a third of the device memory
     Basis basis;
@@ -378,6 +399,8 @@ struct gimic_ctx {
                 (void)hipEventDestroy(e.first);
                 (void)hipEventDestroy(e.second);
             }
+        if (shared) (void)hipStreamSynchronize(shared);
+        if (handover) (void)hipEventDestroy(handover);
         if (stream) {
             (void)hipStreamSynchronize(stream);
             (void)hipStreamDestroy(stream);
@@ -566,6 +589,20 @@ gimic_ctx::Mats &get_mats(gimic_ctx *c, const std::vector<int> &spins, int prec)
     auto &ref = *m;
     c->mats[key] = std::move(m);
     return ref;
+}
+
+// A call on `st` uses the buffers of the context's earlier calls: it starts
+// after these also where they ran on the other one of the library's streams
+// (the caller orders streams of its own).
+void follow(gimic_ctx *c, hipStream_t st) {
+    if (st != c->stream && st != c->shared) return;
+    if (c->last && c->last != st) {
+        if (!c->handover)
+            hip_check(hipEventCreateWithFlags(&c->handover, hipEventDisableTiming), "hipEventCreate");
+        hip_check(hipEventRecord(c->handover, c->last), "hipEventRecord");
+        hip_check(hipStreamWaitEvent(st, c->handover, 0), "hipStreamWaitEvent");
+    }
+    c->last = st;
 }
 
 // Run `launch` between two events on stream st when timing is on.
@@ -1519,12 +1556,22 @@ int gimic_ctx_destroy(gimic_ctx *c) {
     return guarded([&] { delete c; });
 }
 
+int gimic_ctx_shared_stream(gimic_ctx *c, void **stream) {
+    return guarded([&] {
+        if (!c || !stream) throw Error(GIMIC_EINVAL, "null argument");
+        DeviceGuard device(c->device);
+        hip_check(shared_stream(&c->shared), "shared_stream");
+        *stream = c->shared;
+    });
+}
+
 int gimic_jtensor_multi_device(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
                                int nspin, const int *spins, int precision, void *stream) {
     return guarded([&] {
         if (!c || npts < 0 || (npts > 0 && (!d_r || !d_jt)) || nspin < 1 || !spins)
             throw Error(GIMIC_EINVAL, "bad argument");
         hipStream_t st = stream ? (hipStream_t)stream : c->stream;
+        follow(c, st);
         evaluate(c, npts, d_r, d_jt, std::vector<int>(spins, spins + nspin), precision, st,
                  nullptr);
     });
@@ -1592,6 +1639,7 @@ int gimic_jtensor_batch(gimic_ctx *c, int64_t npts, const double *r, double *jt,
         if (!c || npts < 0 || (npts > 0 && (!r || !jt))) throw Error(GIMIC_EINVAL, "bad argument");
         if (npts == 0) return;
         hipStream_t st = c->stream;
+        follow(c, st);
         c->pts_tmp.alloc((size_t)npts * 3 * 8, st, false);
         c->jt_tmp.alloc((size_t)npts * 9 * 8, st, false);
         if (npts > kPipeMin) {
@@ -1770,6 +1818,7 @@ int gimic_flux_planes(gimic_ctx *c, int nplanes, const int64_t *offs, const doub
             if (offs[k + 1] < offs[k]) throw Error(GIMIC_EINVAL, "plane_offs must be non-decreasing");
         const int64_t npts = offs[nplanes];
         hipStream_t st = c->stream;
+        follow(c, st);
         flux_buffers(c, npts, nplanes);
         const size_t np = (size_t)std::max<int64_t>(npts, 1);
         double *d_r = c->pts_tmp.as<double>(), *d_w = d_r + 3 * np;
@@ -1809,6 +1858,7 @@ int gimic_flux_plane_grids(gimic_ctx *c, int nplanes, const int *n1, const int *
         }
         const int64_t npts = poff[nplanes];
         hipStream_t st = c->stream;
+        follow(c, st);
         flux_buffers(c, npts, nplanes);
         // one spec buffer: n1 | off1 off2 poff | origin axes p3w3 nodes1 wts1 nodes2 wts2
         const size_t ni = (size_t)nplanes, nl = 3 * ni + 1,
@@ -1973,6 +2023,7 @@ int gimic_ctx_properties(gimic_ctx *c, int64_t npts, const double *r, const doub
             if (part_offs[k + 1] < part_offs[k])
                 throw Error(GIMIC_EINVAL, "part_offs must be non-decreasing");
         hipStream_t st = c->stream;
+        follow(c, st);
         const size_t np = (size_t)std::max<int64_t>(npts, 1);
         c->prop_in.alloc(np * 32, st, false);  // points then weights
         c->prop_jt.alloc(np * 72, st, false);

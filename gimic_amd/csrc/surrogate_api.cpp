@@ -5,8 +5,6 @@
 
 #include <cmath>
 #include <cstring>
-#include <map>
-#include <mutex>
 #include <random>
 #include <stdexcept>
 #include <string>
@@ -17,6 +15,7 @@
 
 namespace gimic {
 std::string &error_slot();
+hipError_t shared_stream(hipStream_t *stream);
 }
 
 using namespace gimic;
@@ -87,23 +86,6 @@ struct gimic_mlp {
 namespace {
 
 std::string &errstr() { return error_slot(); }
-
-// The stream of the networks on this device whose caller gives none.  One for
-// all of them, kept for the process: a caller's allocator hands the output
-// of one network's call to the next call while the first may still be
-// running, which is sound only where the two run one after the other (on
-// streams of their own, the late first launch of one network wrote over the
-// other's result).
-hipStream_t shared_stream() {
-    static std::mutex lock;
-    static std::map<int, hipStream_t> streams;
-    std::lock_guard<std::mutex> hold(lock);
-    int device = 0;
-    chk(hipGetDevice(&device), "hipGetDevice");
-    hipStream_t &s = streams[device];
-    if (!s) chk(hipStreamCreate(&s), "hipStreamCreate");
-    return s;
-}
 
 hipStream_t work_stream(const gimic_mlp *n) { return n->user ? n->user : n->stream; }
 
@@ -184,7 +166,7 @@ int gimic_mlp_create(gimic_mlp **out, double sigma, const double *center_scale,
         if (!out || !center_scale || !out_scale) throw MlpError(GIMIC_EINVAL, "null argument");
         auto *n = new gimic_mlp();
         try {
-            n->stream = shared_stream();
+            chk(shared_stream(&n->stream), "shared_stream");
             long long off = 0;
             for (int l = 0; l <= kD; l++) {
                 n->kin[l] = l == 0 ? kK0 : kH;

@@ -20,7 +20,7 @@ EXPORTS = [
     "gimic_get_gauss_points", "mkgausspoints", "gimic_last_error", "gimic_ctx_create_files",
     "gimic_ctx_create", "gimic_ctx_set_density", "gimic_ctx_set_density_rows", "gimic_ctx_set_flags", "gimic_ctx_info",
     "gimic_ctx_destroy", "gimic_ctx_atoms", "gimic_ctx_atom_symbols", "gimic_ctx_set_timing", "gimic_ctx_get_timing", "gimic_ctx_tuning", "gimic_ctx_tuning_log", "gimic_ctx_set_mixed_kernel", "gimic_ctx_set_tile_stats", "gimic_ctx_tile_stats", "gimic_ctx_set_fp64_radius", "gimic_ctx_fp64_refined", "gimic_ctx_set_chunk_bytes", "gimic_ctx_chunk_bytes", "gimic_ctx_set_graph", "gimic_ctx_graph_stats", "gimic_jtensor_batch", "gimic_jtensor_batch_device", "gimic_jtensor_batch_device_noalloc",
-    "gimic_jtensor_multi_device", "gimic_flux_planes", "gimic_flux_plane_grids", "gimic_ctx_properties", "gimic_sph_transform", "gimic_quadrature",
+    "gimic_ctx_shared_stream", "gimic_jtensor_multi_device", "gimic_flux_planes", "gimic_flux_plane_grids", "gimic_ctx_properties", "gimic_sph_transform", "gimic_quadrature",
     "gimic_selftest_mfma_layout", "gimic_selftest_mfma32_layout", "gimic_mlp_create", "gimic_mlp_destroy", "gimic_mlp_set_stream", "gimic_mlp_info",
     "gimic_mlp_params", "gimic_mlp_loss_grad", "gimic_mlp_train_step", "gimic_mlp_predict",
     "gimic_mlp_predict_unfused",
@@ -90,6 +90,7 @@ def load():
         "gimic_jtensor_batch": [P, I64, P, P, I, I],
         "gimic_jtensor_batch_device": [P, I64, P, P, I, I, P],
         "gimic_jtensor_batch_device_noalloc": [P, I64, P, P, I, I, P],
+        "gimic_ctx_shared_stream": [P, P],
         "gimic_jtensor_multi_device": [P, I64, P, P, I, P, I, P],
         "gimic_flux_planes": [P, I, P, P, P, P, P, P, P, I, I, P, P, P, P],
         "gimic_flux_plane_grids": [P, I, P, P, P, P, P, P, P, P, P, P, P, P, P, I, I, P, P, P],
@@ -208,6 +209,7 @@ class Context:
     def __init__(self, handle):
         self._h = handle
         self._lib = load()
+        self._shared = None
 
     # -- construction ----------------------------------------------------
     @classmethod
@@ -374,6 +376,19 @@ class Context:
         check(self._lib.gimic_ctx_set_flags(self._h, int(giao), int(diamag), int(paramag)))
 
     # -- evaluation --------------------------------------------------------
+    def _stream(self, device, stream):
+        """the handle to run on: `stream`, by default torch's current stream.
+        For the null stream, torch's default, it is the one that all contexts
+        share: torch hands a tensor that was dropped to the next call at once"""
+        import torch
+        if stream is None:
+            stream = torch.cuda.current_stream(device).cuda_stream
+        if not stream and self._shared is None:
+            s = ctypes.c_void_p()
+            check(self._lib.gimic_ctx_shared_stream(self._h, ctypes.byref(s)))
+            self._shared = s.value
+        return ctypes.c_void_p(stream or self._shared)
+
     def jtensor(self, points, spin="total", precision="fp64"):
         """(N,3) host points -> (N,9) tensors, element m + 3b = J(m,b)."""
         pts = _f64(points, (-1, 3))
@@ -390,8 +405,7 @@ class Context:
         n = pts.shape[0]
         if out is None:
             out = torch.empty((n, 9), dtype=torch.float64, device=pts.device)
-        s = ctypes.c_void_p(stream) if stream is not None else \
-            ctypes.c_void_p(torch.cuda.current_stream(pts.device).cuda_stream)
+        s = self._stream(pts.device, stream)
         check(self._lib.gimic_jtensor_batch_device(self._h, n, ctypes.c_void_p(pts.data_ptr()),
                                                    ctypes.c_void_p(out.data_ptr()), SPIN[spin],
                                                    PREC[precision], s))
@@ -408,8 +422,7 @@ class Context:
         n = pts.shape[0]
         if out is None:
             out = torch.empty((n, 9), dtype=torch.float64, device=pts.device)
-        s = ctypes.c_void_p(stream) if stream is not None else \
-            ctypes.c_void_p(torch.cuda.current_stream(pts.device).cuda_stream)
+        s = self._stream(pts.device, stream)
         check(self._lib.gimic_jtensor_batch_device_noalloc(
             self._h, n, ctypes.c_void_p(pts.data_ptr()), ctypes.c_void_p(out.data_ptr()),
             SPIN[spin], PREC[precision], s))
@@ -422,8 +435,7 @@ class Context:
         sp = _i32([SPIN[s] for s in spins])
         if out is None:
             out = torch.empty((len(spins), n, 9), dtype=torch.float64, device=pts.device)
-        s = ctypes.c_void_p(stream) if stream is not None else \
-            ctypes.c_void_p(torch.cuda.current_stream(pts.device).cuda_stream)
+        s = self._stream(pts.device, stream)
         check(self._lib.gimic_jtensor_multi_device(self._h, n, ctypes.c_void_p(pts.data_ptr()),
                                                    ctypes.c_void_p(out.data_ptr()), len(spins),
                                                    ptr(sp), PREC[precision], s))

@@ -221,8 +221,17 @@ int gimic_ctx_destroy(gimic_ctx *ctx);
 int gimic_jtensor_batch(gimic_ctx *ctx, int64_t npts, const double *r, double *jt, int spin,
                         int precision);
 
+/* The stream that the contexts of one device, and its networks without a
+ * stream, share: for callers whose own work is on the null stream and whose
+ * allocator may hand the output of one context's call to another's while
+ * nothing has waited for the first.  It waits for the null stream and the null
+ * stream for it; a context's calls on it and on the context's own stream run in
+ * the order of the calls.  Kept until the process ends. */
+int gimic_ctx_shared_stream(gimic_ctx *ctx, void **stream);
+
 /* Same with device pointers (HBM) on the given HIP stream (NULL: the
- * context's stream); asynchronous with respect to the host. */
+ * context's own, which nothing orders against other contexts' streams);
+ * asynchronous with respect to the host. */
 int gimic_jtensor_batch_device(gimic_ctx *ctx, int64_t npts, const double *d_r, double *d_jt,
                                int spin, int precision, void *stream);
 
@@ -333,8 +342,8 @@ int gimic_mlp_create(gimic_mlp **net, double sigma, const double *center_scale,
                      const double *out_scale, uint64_t seed);
 int gimic_mlp_destroy(gimic_mlp *net);
 /* run the network's kernels on `stream` (e.g. the caller's current stream),
- * NULL: on the stream that the device's networks without one share; waits
- * for the previous stream first */
+ * NULL: on the stream that the device's contexts and networks share
+ * (gimic_ctx_shared_stream); waits for the previous stream first */
 int gimic_mlp_set_stream(gimic_mlp *net, void *stream);
 /* parameter count and the 3 x 64 frequency matrix (either may be NULL) */
 int gimic_mlp_info(const gimic_mlp *net, long long *nparams, float *freqs);
