@@ -52,8 +52,6 @@ hipError_t shared_stream(hipStream_t *stream) {
 
 namespace {
 
-std::string &g_error = gimic::error_slot();
-
 struct Error : std::runtime_error {
     int code;
     Error(int c, const std::string &m) : std::runtime_error(m), code(c) {}
@@ -69,16 +67,16 @@ template <class F>
 int guarded(F &&f) {
     try {
         f();
-        g_error.clear();
+        error_slot().clear();
         return GIMIC_OK;
     } catch (const Error &e) {
-        g_error = e.what();
+        error_slot() = e.what();
         return e.code;
     } catch (const std::bad_alloc &) {
-        g_error = "host allocation failed";
+        error_slot() = "host allocation failed";
         return GIMIC_ENOMEM;
     } catch (const std::exception &e) {
-        g_error = e.what();
+        error_slot() = e.what();
         return GIMIC_EIO;
     }
 }
@@ -1406,14 +1404,14 @@ int g_uhf_next = 0;
 double g_thrs_next = 1e-6;  // SCREEN_THRS, globals.f90:58
 
 void report(const char *where) {
-    if (!g_error.empty()) std::fprintf(stderr, "gimic: %s: %s\n", where, g_error.c_str());
+    if (!error_slot().empty()) std::fprintf(stderr, "gimic: %s: %s\n", where, error_slot().c_str());
 }
 
 }  // namespace
 
 extern "C" {
 
-const char *gimic_last_error(void) { return g_error.c_str(); }
+const char *gimic_last_error(void) { return error_slot().c_str(); }
 
 int gimic_ctx_create_files(gimic_ctx **out, const char *molfile, const char *densfile, int uhf,
                            double screen_thrs) {
@@ -2129,7 +2127,7 @@ void gimic_set_spin(const char *s) {
     else if (v == "total") g_spin = GIMIC_SPIN_TOTAL;
     else if (v == "spindens") g_spin = GIMIC_SPIN_SPINDENS;
     else {
-        g_error = "Invalid spin case.";
+        error_slot() = "Invalid spin case.";
         report("gimic_set_spin");
     }
 }
@@ -2141,7 +2139,7 @@ void gimic_set_screening(const double *thrs) {
 void gimic_calc_jtensor(const double *r, double *jt) {
     if (!jt) return;
     if (!g_ctx) {
-        g_error = "gimic_init has not been called";
+        error_slot() = "gimic_init has not been called";
         report("gimic_calc_jtensor");
         for (int i = 0; i < 9; i++) jt[i] = 0.0;
         return;

@@ -110,3 +110,26 @@ def test_spherical_transform_zeros_follow_parity():
             assert any(T[mi, k] != 0.0 for k in range(len(comps)) if mask[k]), (l, m)
             kept += sum(mask)
         assert kept < 0.4 * T.size, (l, kept, T.size)
+
+
+def test_error_message_belongs_to_its_thread():
+    """a failing call of another thread leaves this thread's message alone,
+    and that thread reads its own"""
+    import threading
+    from gimic_amd import lib
+    L = lib.load()
+    seen = {}
+    assert L.gimic_quadrature(0.0, 1.0, 5, 7, 0, lib.ptr(np.zeros(7)), lib.ptr(np.zeros(7))) != 0
+    mine = L.gimic_last_error()
+    assert b"multiple of the quadrature order" in mine
+
+    def other():
+        seen["before"] = L.gimic_last_error()
+        seen["rc"] = L.gimic_sph_transform(-1, lib.ptr(np.zeros(4)))
+        seen["after"] = L.gimic_last_error()
+
+    t = threading.Thread(target=other)
+    t.start()
+    t.join()
+    assert seen["rc"] != 0 and seen["before"] == b"" and seen["after"] == b"bad argument"
+    assert L.gimic_last_error() == mine
