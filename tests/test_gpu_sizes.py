@@ -212,3 +212,41 @@ def sheet():
     ctx = s.context(screening=1e-8)
     yield s, ctx
     ctx.close()
+
+
+def test_fp64_rows_too_wide_to_compress():
+    """4,825 functions: FP64 rows wider than the basis kernel's LDS image stay
+    dense (4,832 columns, 7 of them padding that must read as zero).  Two chunks
+    of 256 and 44 points, then fewer points in the same buffers (other plane
+    strides), and the allocation-free call, whose scratch held other data"""
+    import torch
+    from gimic_amd import synth
+    at = np.arange(965)
+    xyz = 3.0 * np.c_[at % 10, at // 10 % 10, at // 100] - 13.5
+    s, rng = synth.build_system("block", ["H"] * 965, xyz, {"H": "2s1p"}, 7)
+    s.dens = rng.standard_normal((1, 4, s.nbf, s.nbf))
+    pts = rng.uniform(-15.0, 15.0, (300, 3))
+    sub = np.r_[0:300:43, 299]
+    ref = oracle.jtensor(s.arrays(), sph.to_cartesian(s.dens, s.shell_l), pts[sub], screening=1e-8)
+    with s.context(screening=1e-8) as ctx:
+        assert ctx.nbf == 4825
+        ctx.set_chunk_bytes(256 * 4832 * 32)
+        print("case block of 4825 functions, 300 points in two chunks", flush=True)
+        J = ctx.jtensor(pts, precision="fp64")
+        assert rel_err(J[sub], ref).max() <= 1e-10
+        ctx.set_chunk_bytes(0)
+        for n in (70, 300, 129):
+            print("case block of 4825 functions", n, flush=True)
+            K = ctx.jtensor(pts[:n], precision="fp64")
+            assert rel_err(K, J[:n]).max() <= 1e-10
+        print("case block of 4825 functions, mixed", flush=True)
+        M = ctx.jtensor(pts, precision="mixed")
+        assert rel_err(M, J).max() <= 1e-5
+        d = torch.tensor(pts, device="cuda")
+        ctx.jtensor_device(d[:1])
+        for prec, n, tol in (("mixed", 300, 1e-5), ("fp64", 300, 1e-10), ("fp64", 70, 1e-10)):
+            print("case block of 4825 functions, allocation-free", prec, n, flush=True)
+            ctx.jtensor_device(d[:1], precision=prec)
+            K = ctx.jtensor_device_noalloc(d[:n], precision=prec)
+            torch.cuda.synchronize()
+            assert rel_err(K.cpu().numpy(), J[:n]).max() <= tol
