@@ -109,7 +109,12 @@ struct DevBuf {
             return;
         }
         release();
-        hip_check(hipMalloc(&p, std::max<size_t>(n, 256)), "hipMalloc");
+        const hipError_t e = hipMalloc(&p, std::max<size_t>(n, 256));
+        if (e != hipSuccess) {
+            p = nullptr;
+            (void)hipGetLastError();  // else the next launch reports it
+        }
+        hip_check(e, "hipMalloc");
         bytes = n;
         if (zero) hip_check(hipMemsetAsync(p, 0, n, s), "hipMemsetAsync");
     }
@@ -807,7 +812,6 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
             break;
         } catch (const Error &e) {
             if (e.code != GIMIC_ENOMEM || mode != EvalMode::Eager) throw;
-            (void)hipGetLastError();  // the failed hipMalloc is not a launch error
             if (prec == GIMIC_PREC_FP64 && (W.phis.p || W.grad32.p)) {
                 W.phis.release();
                 W.grad32.release();

@@ -250,3 +250,25 @@ def test_fp64_rows_too_wide_to_compress():
             K = ctx.jtensor_device_noalloc(d[:n], precision=prec)
             torch.cuda.synchronize()
             assert rel_err(K.cpu().numpy(), J[:n]).max() <= tol
+
+
+def test_call_after_one_too_large_for_the_device(ring):
+    """a host batch of 2^40 points (26 TB of them alone; refused before any copy
+    or launch) is an error, and none of the call that follows it"""
+    from gimic_amd import lib
+    s, ctx = ring
+    pts = _points(100)
+    J = ctx.jtensor(pts)
+    out = np.zeros((1, 9))
+    for call in ("points", "planes"):
+        print("case 2^40", call, flush=True)
+        with pytest.raises(lib.GimicError, match="out of memory"):
+            if call == "points":
+                lib.check(ctx._lib.gimic_jtensor_batch(ctx._h, 1 << 40, lib.ptr(pts), lib.ptr(out),
+                                                       0, 0))
+            else:
+                offs = np.array([0, 1 << 40], dtype=np.int64)
+                lib.check(ctx._lib.gimic_flux_planes(
+                    ctx._h, 1, lib.ptr(offs), lib.ptr(pts), lib.ptr(pts), lib.ptr(pts),
+                    lib.ptr(pts), lib.ptr(pts), lib.ptr(pts), 0, 0, lib.ptr(out), None, None, None))
+        assert np.array_equal(ctx.jtensor(pts), J)
