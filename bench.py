@@ -77,8 +77,8 @@ def kernel_roofline(ctx, d_pts, out, precision, nbf):
     tile (a tile of R rows with k live 8-function groups multiplies
     R x 8k by 8k x 7*8k: 14 R (8 k)^2 flops; the mixed kernel walks these
     groups along N and K, the FP64 kernel the live granules of four functions
-    in them, up to a fifth fewer pairs, so its figure is an upper bound), and one with event timing around each kernel
-    launch.  achieved = listed flops per launch / average launch time; the
+    in them, up to a fifth fewer pairs, so its figure is an upper bound), and
+    one with event timing around each kernel launch.  achieved = listed flops per launch / average launch time; the
     dense product would need 14 nbf^2 per point."""
     import torch
     # these passes measure the mixed contraction kernel alone: the FP64 pass
@@ -491,6 +491,8 @@ def main():
     ms_f64, wall_f64 = time_steps(ctx, d_pts, out, "fp64", args.steps, args.warmup)
     J_f64_sample = out[:: max(1, npts // 65536)].cpu().numpy()
     roof64, _ = kernel_roofline(ctx, d_pts, out, "fp64", nbf)
+    roof64["flop_count"] = ("upper bound: live 8-function groups; the kernel walks the live "
+                            "granules of four functions in them")
 
     nb = np.linalg.norm(J_f64_sample, axis=1)
     e = np.linalg.norm(J_mixed_sample - J_f64_sample, axis=1) / np.maximum(nb, 1e-3 * nb.max())

@@ -1061,7 +1061,8 @@ void evaluate(gimic_ctx *c, int64_t npts, const double *d_r, double *d_jt,
             plan_variant(prec == GIMIC_PREC_FP64 ? 0 : mv);
             continue;
         }
-        // rows in Morton order of their cells (spts, perm)
+        // rows along the curve of their cells (spts, perm): Hilbert for FP64,
+        // Morton for the mixed kernels
         timed(c, 0, st, [&] {
             hip_check(launch_sort_points(d_r + 3 * start, n_c, W.spts.as<double>(),
                                          W.perm.as<int>(), W.bpart.as<double>(),

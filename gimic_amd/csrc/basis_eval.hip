@@ -71,9 +71,10 @@ __device__ __forceinline__ void radial_parts(const EvalArgs &a, const DevShell &
 
 // Candidate lists (below) for bases of at least this many shells: with fewer,
 // nearly every shell reaches every tile and the list costs registers and a
-// pass over the shells.  256 planes of tetracene (144 shells): mixed basis
-// 1.46 ms without the list, 1.19 with it, FP64 1.66 and 1.35; twelve atoms
-// (54 shells), 40,000 points: 0.094 without, 0.097 with it.
+// pass over the shells.  256 planes of tetracene (144 shells), lists included:
+// mixed basis 1.27 ms without the list, 1.04 with it, FP64 1.44 and 1.19; twelve
+// atoms (54 shells), 40,000 points: mixed 0.085 without, 0.087 with it, FP64
+// 0.097 and 0.099.
 constexpr int kCandMinShells = 64;
 // Workgroups a launch should have before they take 32 rows each
 constexpr int kMinBasisGroups = 512;

@@ -8,8 +8,8 @@
 // sums are kept across N-tiles.  Both operands arrive split:
 //   * the basis kernel writes the left operand as [row][k/8][kAParts][8]
 //     (16 kAParts contiguous bytes per lane and K-step), and
-//   * the right operand (constant per density) is split once on the host into
-//     pair blocks of kBParts x 896 bytes per (density set, 8-function
+//   * the right operand (constant per density) is split once on the device
+//     (operands.hip) into pair blocks of kBParts x 896 bytes per (density set, 8-function
 //     K-group, 8-function N-group), [part][matrix][n][8 k]; a K-step's LDS
 //     buffer gathers the 16 pair blocks of its four K-groups and the N-tile's
 //     four N-groups.

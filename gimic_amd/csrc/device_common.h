@@ -69,16 +69,6 @@ __device__ __forceinline__ float row16_sum(float x) {
     x += GIMIC_DPP(x, 0x140);  // row_mirror
     return x;
 }
-#define GIMIC_DPP_D(x, ctrl)                                                                    \
-    __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), (ctrl), 0xF, 0xF, false), \
-                     __builtin_amdgcn_update_dpp(0, __double2loint(x), (ctrl), 0xF, 0xF, false))
-__device__ __forceinline__ double row16_sum(double x) {
-    x += GIMIC_DPP_D(x, 0xB1);
-    x += GIMIC_DPP_D(x, 0x4E);
-    x += GIMIC_DPP_D(x, 0x141);
-    x += GIMIC_DPP_D(x, 0x140);
-    return x;
-}
 
 // box of the lanes' boxes, left in every lane of the wavefront
 __device__ __forceinline__ void wave_box(double (&lo)[3], double (&hi)[3]) {
@@ -158,8 +148,10 @@ struct ContractArgs {
     const float *rf32;
     double *part;        // [nmatset][nsplit][kNQ][rows]; pre-split kernels: [nmatset][nsplit][rows][kNQ]
     // screening lists per row tile (TileArgs): its live groups of 8 functions
-    // (pre-split kernels) or 4 (FP64 kernel), four per N-tile and K-step;
-    // split s of a tile takes N-tiles [s * count / nsplit, (s+1) * count / nsplit)
+    // (pre-split kernels) or 4 (FP64 kernel), four per N-tile and K-step.  The
+    // N-tiles of a row tile are dealt evenly to its N-ranges: all nsplit / ksplit
+    // of them (FP64 kernel, mixed in the plain form), else as many of the nsplit
+    // as filled_ranges() says
     int nblk, tile_rows;  // tile_rows: FP64 kernel only
     int spread;           // workgroups of fewer than kSpreadTiles row tiles to all XCDs in turn
     int plain;            // mixed: every range of a tile writes its sums, without N-tiles zeros
@@ -186,7 +178,9 @@ hipError_t launch_contract_f64(const ContractArgs &a, hipStream_t s);
 // contract_mx2.hip); nbuf 2 or 3 LDS buffers, krb 2 or 4 row blocks per
 // wavefront, 4 or 8 wavefronts (16 * krb * waves rows per workgroup: 4 waves
 // with krb 2, nbuf 2 or 3, or krb 4, nbuf 2; 8 waves with krb 2, nbuf 2 or
-// 3).  Writes every partial sum of a.part, row-major (no clearing needed).
+// 3).  Writes the partial sums of the filled ranges (filled_ranges(); in the
+// plain form of all nsplit) whole, row-major, and leaves the others as they
+// are: the assembly must be given kcount then.
 hipError_t launch_contract_mx2(const ContractArgs &a, int nbuf, int krb, int waves, hipStream_t s);
 // Mixed arithmetic: an FP32 operand value x is the sum of BF16 parts
 // x = h + m + l (three parts: exact); the basis values (left operand) keep

@@ -327,9 +327,9 @@ class Context:
         """dict(tiles, blocks, blocks_sq, tile_rows, nblk, blocks_kn,
         groups_sq): row tiles seen, sum of listed blocks and of their
         squares, rows per tile, blocks of a dense row, the sum of listed
-        blocks x live 8-function groups / 4 (the FP64 kernel's block
-        products) and of squared live groups (the pre-split mixed kernels'
-        group products)"""
+        blocks x live 8-function groups / 4 and of squared live groups (the
+        pre-split mixed kernels' group products, and an upper bound of those
+        of the FP64 kernel, which walks granules of four functions)"""
         out = np.zeros(7)
         check(self._lib.gimic_ctx_tile_stats(self._h, ptr(out)))
         return dict(tiles=int(out[0]), blocks=float(out[1]), blocks_sq=float(out[2]),
